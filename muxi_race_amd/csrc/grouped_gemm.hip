@@ -7,8 +7,9 @@
 // :1391-1635) and Stage2 family (:655-795, :1132-1378); base form
 // xpuoj_data/submission.py:31-129 and :253-331.  The tiling here is this
 // build's own.  One workgroup per item:
-//   - 32- and 64-row tiles (4 waves) for decode-sized batches; fp16 Stage 1 of
-//     32-row tiles runs the narrow kernel (32 gate + 32 up features per item);
+//   - 32- and 64-row tiles (4 waves) for decode-sized batches; fp16 and int8
+//     Stage 1 of 32-row tiles run the narrow kernel (32 gate + 32 up features
+//     per item);
 //   - 128-row tiles (8 waves): BM rows x 256 weight rows (Stage 1: 128 gate +
 //     128 up, sharing the token tile; Stage 2: 256 features), or a paired item
 //     of 2*BM rows x 128 weight rows for two blocks of one expert, which
@@ -46,7 +47,7 @@
 #define MOE_S1_SPLIT 1
 #endif
 // 8-bit 256-row items: weight tiles that no other item of the launch reads
-// are loaded non-temporal -- int8 Stage 1's weight slots of the split ring and
+// are loaded non-temporal (32-row tiles of every format always do so) -- int8 Stage 1's weight slots of the split ring and
 // both formats' Stage 2 weight rows (1, the default); 0: the default policy
 // everywhere.  A/B at the w8a8 shape, 3 runs each, interleaved: int8 step
 // 0.853 -> 0.822 ms (Stage 1 0.489 -> 0.479, Stage 2 0.284 -> 0.274); fp8
@@ -248,7 +249,10 @@ __device__ __forceinline__ void stage1_triple(const Stage1Params& p, const Work&
 // 0.474 -> 0.453 ms.  fp16 (mixtral) measured slower on it, 1.158 -> 1.197 ms:
 // its token rows, 4 MiB per expert, often come from beyond L2, and one step of
 // lead is not enough for them; it keeps the two-stage ring.
-template <int BM, int WAVES_M, int S, int NW, int QT, bool GATHER, bool PAIR>
+//
+// STREAM (whole-stage rings): weight tiles no other item reads are loaded
+// non-temporal.
+template <int BM, int WAVES_M, int S, int NW, int QT, bool GATHER, bool PAIR, bool STREAM>
 __global__ __launch_bounds__(64 * NW) void stage1_kernel(Stage1Params p) {
   constexpr bool I8 = QT != kQF16;  // 8-bit operands (int8 or fp8) with row scales
   constexpr bool F8 = QT == kQF8;
@@ -416,6 +420,11 @@ __global__ __launch_bounds__(64 * NW) void stage1_kernel(Stage1Params p) {
   const int aj = L::NBN == 2 ? (wm & 1) : 0;   // block among the wave's gate / up blocks
   const int awr0 = (agate ? gr0 : ur0) + 32 * aj;
   const int q_wave = LD::NI + (adma ? 1 : 0);  // loads per stage of this wave
+  auto issue = [&](char* stage, int k) {
+    if constexpr (STREAM) ld.issue(stage, k, w.shared ? kNoStream : rx);
+    else ld.issue(stage, k);
+    issue_abs(stage, k);
+  };
 
   // S-stage ring: stages ks+1 .. ks+S-2 stay in flight while stage ks is used.
   constexpr int Q = LD::NI;  // loads per wave per stage
@@ -436,10 +445,7 @@ __global__ __launch_bounds__(64 * NW) void stage1_kernel(Stage1Params p) {
     } else {
 #pragma unroll
       for (int s = 0; s < S - 1; ++s)
-        if (s < nk) {
-          ld.issue(smem + s * STAGE, s);
-          issue_abs(smem + s * STAGE, s);
-        }
+        if (s < nk) issue(smem + s * STAGE, s);
     }
     int cur = 0;
     for (int ks = 0; ks < nk; ++ks) {
@@ -468,11 +474,8 @@ __global__ __launch_bounds__(64 * NW) void stage1_kernel(Stage1Params p) {
       char* pbuf = smem + (cur == 0 ? S - 1 : cur - 1) * STAGE;
       const int pk = ks + S - 1;
       if constexpr (!SPLIT) cur = cur + 1 == S ? 0 : cur + 1;
-      constexpr bool kSpread = MOE_SPREAD_ISSUE != 0 && NB > 0 && S >= 3;
-      if (!kSpread && pend) {
-        ld.issue(pbuf, pk);
-        issue_abs(pbuf, pk);
-      }
+      constexpr bool kSpread = MOE_SPREAD_ISSUE != 0 && NB > 0 && !STREAM && S >= 3;
+      if (!kSpread && pend) issue(pbuf, pk);
       if constexpr (NB > 0 || A) {
         // Fragments double-buffered across the 4 K sub-steps: the LDS reads of
         // sub-step s+1 are in flight while the MFMAs of sub-step s run.
@@ -673,7 +676,7 @@ __global__ __launch_bounds__(64 * NW) void stage1_kernel(Stage1Params p) {
   }
 }
 
-// Stage 1 (fp16) for 32-row tiles with narrow gate / up tiles (BN = 64 or
+// Stage 1 (fp16, int8) for 32-row tiles with narrow gate / up tiles (BN = 64 or
 // 32 features each): two or four times the items of the 128-wide tiles, for
 // shapes with few items per CU (decode), where the last round of workgroups
 // would otherwise stream on a fraction of the CUs.  Each of the 4 waves owns
@@ -681,10 +684,21 @@ __global__ __launch_bounds__(64 * NW) void stage1_kernel(Stage1Params p) {
 //   BN = 64: features 32 * (w & 1) of the tile, all 4 K sub-steps of a step;
 //   BN = 32: all 32 features, K sub-steps 2 * (w & 1) and 2 * (w & 1) + 1,
 //            the two halves summed in the epilogue.
-// The other accumulators reach the wave writing h through LDS.
-template <int BN, int S>
+// The other accumulators reach the wave writing h through LDS (int8: as exact
+// int32 sums, so h has the bits that the 128-wide tiles give).
+// int8 ran the 128-wide tiles here until this kernel took it: one workgroup
+// per CU, weights under the default cache policy, and at one token (6 experts,
+// I 2048) 96 items on 256 CUs.  64 experts, H 7168, I 2048, top-6: 24 tokens
+// 291 -> 254 us (5.8 -> 6.6 TB/s of weights), 129 tokens 321 -> 294, 1 token
+// 54 -> 41.  fp8 keeps 128-wide items (it scales h per 128 columns) and gains
+// from the non-temporal weights alone: 24 tokens 290 -> 268 us.
+template <int BN, int S, int QT>
 __global__ __launch_bounds__(256) void stage1_narrow_kernel(Stage1Params p) {
   constexpr int BM = 32, NW = 4;
+  constexpr bool I8 = QT == kQI8;
+  static_assert(QT != kQF8, "fp8 quantises h per 128-column tile: items must span 128 columns");
+  using Acc = typename std::conditional<I8, i32x16, f32x16>::type;
+  using Elem = typename std::conditional<I8, int, float>::type;
   static_assert(BN == 64 || BN == 32, "narrow tiles are 64 or 32 features wide");
   constexpr bool KSPLIT = BN == 32;
   constexpr int ROWS = BM + 2 * BN;  // stage rows: tokens, gate rows, up rows
@@ -704,7 +718,7 @@ __global__ __launch_bounds__(256) void stage1_narrow_kernel(Stage1Params p) {
   actual = actual < 0 ? 0 : (actual > BM ? BM : actual);
   if (actual == 0) return;
 
-  const int64_t kbytes = p.H * 2;
+  const int64_t kbytes = p.H * (I8 ? 1 : 2);
   const int nk = (int)(kbytes / kRowBytes);
   const bool sh = p.e_shared >= 0 && e == p.e_shared;  // see stage1_kernel
   const char* gexp = sh ? p.wg_shared : p.wg + (int64_t)e * p.w_es;
@@ -731,7 +745,23 @@ __global__ __launch_bounds__(256) void stage1_narrow_kernel(Stage1Params p) {
   const int wr0 = BM + mat * BN + (KSPLIT ? 0 : 32 * half);
   constexpr int SUB = KSPLIT ? 2 : 4;    // K sub-steps per wave per step
   const int s0 = KSPLIT ? 2 * half : 0;  // first of them
-  f32x16 acc = f32x16{};
+  Acc acc = Acc{};
+  // int8: the dequantisation scales of this lane's token row and features,
+  // loaded before the K loop so that their latency hides behind it
+  const int l = lane_id();
+  const int fbase = KSPLIT ? 0 : 32 * half;  // the wave's first feature in the tile
+  float sx = 0.0f;
+  f32x4 sgv[4], suv[4];
+  if constexpr (I8) {
+    const int pid = p.sorted_ids[row0 + (l & 31)];
+    sx = p.x_scale[(l & 31) < actual ? pid / p.topk : 0];
+#pragma unroll
+    for (int rg = 0; rg < 4; ++rg) {
+      const int64_t n = (int64_t)e * p.I + n0 + fbase + 8 * rg + 4 * (l >> 5);
+      sgv[rg] = *reinterpret_cast<const f32x4*>(p.sg + n);
+      suv[rg] = *reinterpret_cast<const f32x4*>(p.su + n);
+    }
+  }
   const int stream_from = w.shared ? kNoStream : BM;  // weight rows no other item reads: streamed
   constexpr int Q = LD::NI;
 #pragma unroll
@@ -763,9 +793,8 @@ __global__ __launch_bounds__(256) void stage1_narrow_kernel(Stage1Params p) {
   // Accumulator register r of lane l holds the same (token, feature) in every
   // wave that covers the same features, so the hand-over is by (r, l):
   // slot(w, r) for the waves other than the one writing h.
-  float* xs = reinterpret_cast<float*>(smem);
-  const int l = lane_id();
-  auto slot = [&](int wv, int r) -> float& { return xs[(wv * 16 + r) * 64 + l]; };
+  Elem* xs = reinterpret_cast<Elem*>(smem);
+  auto slot = [&](int wv, int r) -> Elem& { return xs[(wv * 16 + r) * 64 + l]; };
   const bool writer = KSPLIT ? wave == 0 : mat == 0;
   if (!writer) {
 #pragma unroll
@@ -776,7 +805,6 @@ __global__ __launch_bounds__(256) void stage1_narrow_kernel(Stage1Params p) {
     const int m = l & 31;
     if (m < actual) {
       _Float16* hrow = reinterpret_cast<_Float16*>(p.h) + (int64_t)(row0 + m) * p.h_ld;
-      const int fbase = KSPLIT ? 0 : 32 * half;
 #pragma unroll
       for (int rg = 0; rg < 4; ++rg) {
         const int n = n0 + fbase + 8 * rg + 4 * (l >> 5);
@@ -784,7 +812,7 @@ __global__ __launch_bounds__(256) void stage1_narrow_kernel(Stage1Params p) {
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
           const int r = 4 * rg + q;
-          float g, u;
+          Elem g, u;
           if constexpr (KSPLIT) {  // waves: 0 gate k0, 1 gate k1, 2 up k0, 3 up k1
             g = acc[r] + slot(1, r);
             u = slot(2, r) + slot(3, r);
@@ -792,7 +820,8 @@ __global__ __launch_bounds__(256) void stage1_narrow_kernel(Stage1Params p) {
             g = acc[r];
             u = slot(2 + half, r);
           }
-          v[q] = (_Float16)silu_mul(g, u);
+          if constexpr (I8) v[q] = (_Float16)silu_mul(((float)g * sx) * sgv[rg][q], ((float)u * sx) * suv[rg][q]);
+          else v[q] = (_Float16)silu_mul(g, u);
         }
         *reinterpret_cast<f16x4*>(hrow + n) = v;
       }
@@ -800,7 +829,7 @@ __global__ __launch_bounds__(256) void stage1_narrow_kernel(Stage1Params p) {
   }
 }
 
-// STREAM: weight tiles no other item reads are loaded non-temporal.
+// STREAM: as Stage 1's.
 template <int BM, int WAVES_M, int BN, int S, int NW, int QT, bool FUSED, bool PAIR, bool STREAM>
 __global__ __launch_bounds__(64 * NW) void stage2_kernel(Stage2Params p) {
   constexpr bool I8 = QT != kQF16;  // 8-bit operands (int8 or fp8) with row / block scales
@@ -1188,7 +1217,15 @@ __global__ __launch_bounds__(64 * NW) void stage2_kernel(Stage2Params p) {
 constexpr int s1_stages(int bm) {
   return bm == 256 ? 2 : bm == 128 ? MOE_S1_STAGES_128 : (bm == 64 ? MOE_S1_STAGES_64 : MOE_S1_STAGES_32);
 }
-constexpr int s2_stages(int bm) {
+// fp8 Stage 2 of 32-row tiles: a stage also holds the step's row scales (21 KiB
+// in all), so four of them leave one workgroup per CU and three leave two.
+// 64 experts, H 7168, I 2048, top-6: 129 tokens 171 -> 154 us, 24 tokens
+// 148 -> 137 us.
+#ifndef MOE_S2_STAGES_32_F8
+#define MOE_S2_STAGES_32_F8 3
+#endif
+constexpr int s2_stages(int bm, int qt) {
+  if (bm == 32 && qt == kQF8) return MOE_S2_STAGES_32_F8;
   return bm == 256 ? 2 : bm == 128 ? MOE_S2_STAGES_128 : (bm == 64 ? MOE_S2_STAGES_64 : MOE_S2_STAGES_32);
 }
 
@@ -1206,8 +1243,8 @@ constexpr int s2_stages(int bm) {
 #ifndef MOE_PAIR
 #define MOE_PAIR 1
 #endif
-// fp16 Stage 1 of 32-row tiles: gate / up tile width of the narrow kernel
-// (64 or 32; 0 = the 128-wide tiles) and its ring depth.
+// fp16 and int8 Stage 1 of 32-row tiles: gate / up tile width of the narrow
+// kernel (64 or 32) and its ring depth.
 #ifndef MOE_S1_NARROW32
 #define MOE_S1_NARROW32 32
 #endif
@@ -1218,8 +1255,16 @@ constexpr int s2_stages(int bm) {
 template <int BM, int WM, int NW, int QT, bool GATHER, bool PAIR>
 static hipError_t go1(const Stage1Params& p, int64_t grid, hipStream_t s) {
   constexpr int kS = s1_stages(BM);
-  hipLaunchKernelGGL((stage1_kernel<BM, WM, kS, NW, QT, GATHER, PAIR>), dim3((unsigned)grid),
+  hipLaunchKernelGGL((stage1_kernel<BM, WM, kS, NW, QT, GATHER, PAIR, BM == 32>), dim3((unsigned)grid),
                      dim3(64 * NW), 0, s, p);
+  return hipGetLastError();
+}
+
+template <int QT>
+static hipError_t go1_narrow(const Stage1Params& p, int64_t max_blocks, hipStream_t s) {
+  constexpr int kW = MOE_S1_NARROW32;
+  const int64_t grid = schedule_grid(max_blocks, p.I / kW);
+  hipLaunchKernelGGL((stage1_narrow_kernel<kW, MOE_S1N_STAGES, QT>), dim3((unsigned)grid), dim3(256), 0, s, p);
   return hipGetLastError();
 }
 
@@ -1229,7 +1274,7 @@ static hipError_t go1(const Stage1Params& p, int64_t grid, hipStream_t s) {
 // epilogue.  Paired items are then 256 x 128.
 template <int BM, int WM, int BN, int NW, int QT, bool FUSED, bool PAIR>
 static hipError_t go2(const Stage2Params& p, int64_t max_blocks, hipStream_t s) {
-  constexpr int kS = s2_stages(BM);
+  constexpr int kS = s2_stages(BM, QT);
   const int64_t grid = schedule_grid(max_blocks, p.H / BN);
   if (grid <= 0) return hipSuccess;
   constexpr bool kStream = BM == 32 || (MOE_W8_STREAM != 0 && QT != kQF16 && BM == 256);
@@ -1261,15 +1306,8 @@ hipError_t launch_stage1(const Stage1Params& params, int block_m, int qt, bool g
   }
   switch (block_m) {
     case 32:
-      if (qt == kQI8) return go1<32, 1, 4, kQI8, true, false>(p, grid, s);
       if (qt == kQF8) return go1<32, 1, 4, kQF8, true, false>(p, grid, s);
-      if constexpr (MOE_S1_NARROW32 != 0) {
-        constexpr int kW = MOE_S1_NARROW32;
-        const int64_t gn = schedule_grid(max_blocks, p.I / kW);
-        hipLaunchKernelGGL((stage1_narrow_kernel<kW, MOE_S1N_STAGES>), dim3((unsigned)gn), dim3(256), 0, s, p);
-        return hipGetLastError();
-      }
-      return go1<32, 1, 4, kQF16, true, false>(p, grid, s);
+      return qt == kQI8 ? go1_narrow<kQI8>(p, max_blocks, s) : go1_narrow<kQF16>(p, max_blocks, s);
     case 64:
       if (qt == kQI8) return go1<64, 1, 4, kQI8, true, false>(p, grid, s);
       if (qt == kQF8) return go1<64, 1, 4, kQF8, true, false>(p, grid, s);

@@ -85,6 +85,21 @@ def test_w8a8_skewed_ragged(bm):
     _run(skewed_8bit_case(22), block_m=bm)
 
 
+@pytest.mark.parametrize("T,H,I", [(1, 128, 128), (33, 384, 256), (70, 1024, 384)])
+def test_int8_narrow_tiles_match_wide(T, H, I):
+    """32-row blocks (Stage 1 on 32-wide K-split tiles; K loops shorter than
+    the ring, one row, a second block of a few rows) against 128-row blocks:
+    exact int32 sums, so the same bits."""
+    from muxi_race_amd import fused_moe, quantize_w8a8_weights
+    g = torch.Generator(device="cuda").manual_seed(T)
+    mk = lambda *sh: torch.randn(sh, generator=g, device="cuda").half()
+    x, lg = mk(T, H), torch.randn(T, 5, generator=g, device="cuda")
+    qw = quantize_w8a8_weights(mk(5, I, H) * 0.05, mk(5, I, H) * 0.05, mk(5, H, I) * 0.05)
+    a, b = (fused_moe(x, lg, None, None, None, 2, w8a8=qw, block_m=bm) for bm in (32, 128))
+    torch.cuda.synchronize()
+    assert bool(torch.isfinite(a).all()) and torch.equal(a, b)
+
+
 def test_w8a8_config_full():
     _run(moe_inputs("w8a8", 22))
 
