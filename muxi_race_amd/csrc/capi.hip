@@ -10,12 +10,6 @@
 
 #include <mutex>
 
-// fp16 Stage 2 over the 256-row padding: 256-row items (1) or 128-row paired
-// items (0).
-#ifndef MOE_S2_F16_256
-#define MOE_S2_F16_256 1
-#endif
-
 namespace {
 
 thread_local char g_err[512] = "";
@@ -43,12 +37,13 @@ int64_t cap_rows(int64_t T, int64_t k, int64_t E, int64_t bm) {
 }
 
 struct FusedLayout {
-  int64_t ids, w, sorted, bexp, gs, go, gpo, whist, h, hq, hs, xq, sx, ypair, pos, total;
+  int64_t ids, w, sorted, bexp, gs, go, gpo, istart, whist, h, hq, hs, xq, sx, ypair, pos, total;
 };
 
 // qt: moe::kQF16, kQI8 or kQF8.  The intermediate h is fp16 for fp16 and int8
 // operands (int8 quantises it per row afterwards, into hq + hs), fp8 codes
-// for fp8 (with per-(row, 128-column) scales in hs).
+// for fp8 (with per-(row, 128-column) scale bytes in hs).
+int64_t hs_pitch(int64_t I) { return (I / moe::kBN + 15) / 16 * 16; }  // fp8: scale bytes of a row, 16 K steps a load
 FusedLayout fused_layout(int64_t T, int64_t H, int64_t I, int64_t E, int64_t k, int64_t bm,
                          int qt) {
   FusedLayout L{};
@@ -62,10 +57,11 @@ FusedLayout fused_layout(int64_t T, int64_t H, int64_t I, int64_t E, int64_t k, 
   L.gs = o; o += up(E * 4);
   L.go = o; o += up((E + 1) * 4);
   L.gpo = o; o += up((E + 1) * 4);
+  L.istart = o; o += up((E + 19) * 4);                   // wide items per N tile below each expert, XCD bounds
   L.whist = o; o += up((int64_t)moe::align_groups((int)P) * E * 4);  // align workgroup histograms
   L.h = o; o += up(rows * I * (qt == moe::kQF8 ? 1 : 2));
   L.hq = o; o += i8 ? up(rows * I) : 0;                   // int8: per-row codes of h
-  L.hs = o; o += w8 ? up(rows * (i8 ? 1 : I / moe::kBN) * 4) : 0;  // int8 [rows]; fp8 [I/128][rows], block-major
+  L.hs = o; o += w8 ? up(rows * (i8 ? 4 : hs_pitch(I))) : 0;  // int8: fp32 per row; fp8: E8M0 bytes
   L.xq = o; o += w8 ? up(T * H) : 0;
   L.sx = o; o += w8 ? up(T * 4) : 0;
   L.ypair = o; o += up(P * H * 2);                        // per-pair outputs, expert-sorted rows
@@ -81,20 +77,53 @@ int64_t pick_bm(int64_t T, int64_t E, int64_t k) {
   return 128;
 }
 
-// Rows per block of the align padding.  block_m != 0 is the caller's choice,
-// used by both stages.  0: pick_bm's size, except that 128 becomes 256 when
-// experts hold >= 192 routed rows on average and H is a multiple of 256: then
-// both stages run 256-row items for every format, measured faster on each.
-// (Built with MOE_S2_F16_256=0, fp16 Stage 2 keeps 128-row paired items over
-// the 256-row padding; those that fall in a block's empty second half end at
-// once.)  At fewer rows per expert half-empty 256-row blocks cost more than
-// they save.
-int64_t align_bm(int64_t T, int64_t E, int64_t k, int64_t H, int64_t block_m) {
+// Rows per block of the align padding, and with it the items: 32-row blocks
+// run narrow items, others wide ones, which do not depend on the padding
+// (moe_common.h Item).  block_m != 0 is the caller's choice.  0:
+//   - narrow up to kNarrowRows routed rows per expert on average.  Both stages
+//     together, narrow against wide, H 7168 and I 2048: 256 experts top-8, 640
+//     tokens (20 rows) 3.35 / 3.37 ms, 768 (24) 3.42 / 3.37, 900 (28) 3.57 /
+//     3.57, 1024 (32) 4.24 / 3.56; 64 experts top-6, 256 tokens (24) 0.88 /
+//     0.86, 300 (28) 0.97 / 0.89; int8 256 tokens 0.469 / 0.475, 300 0.484 /
+//     0.456.  Above it more and more experts need a second 32-row block.
+//   - narrow up to kLowRows rows where one wide item per expert and tile would
+//     leave half of the CUs idle: 8 experts, H 1024, I 512, top-2, 400 tokens
+//     22 / 34 us, but 1000 tokens (250 rows) 41 / 34.
+//   - otherwise pick_bm's padding, at least 64, and 256 from 192 rows on if H is
+//     a multiple of 256.
+constexpr int64_t kNarrowRows = 24;
+// too many rows for the kernels' 32-bit indices
+bool too_large(int64_t T, int64_t k, int64_t E, int64_t I, int64_t bm) { return cap_rows(T, k, E, bm) * I >= ((int64_t)1 << 32); }
+int64_t align_bm(int64_t T, int64_t E, int64_t k, int64_t H, int64_t I, int64_t block_m) {
   if (block_m) return block_m;
   const int64_t bm = pick_bm(T, E, k);
-  if (bm != 128 || H % 256) return bm;
-  const int64_t avg = (T * k + E - 1) / E;
-  return avg >= 192 ? 256 : 128;
+  const int64_t avg = E > 0 ? (T * k + E - 1) / E : 0;
+  if (avg <= kNarrowRows || (avg <= moe::kLowRows && E * (I / moe::kBN) < 128)) return 32;
+  if (bm == 32) return too_large(T, k, E, I, 64) ? 32 : 64;
+  return bm == 128 && H % 256 == 0 && avg >= 192 ? 256 : bm;
+}
+
+// How the wide items split `rows` routed rows over at most `experts` experts:
+// the most rows of an item, whether Stage 2 takes 256 features, and an upper
+// bound on the items per N tile.  An expert is assumed to hold the average.
+// Launches that would not give every CU an item take shorter and narrower ones.
+struct WidePlan {
+  int hmax;
+  bool bn256;
+  int64_t nt2;        // Stage 2's N tiles
+  int64_t max_items;
+};
+WidePlan wide_plan(int64_t rows, int64_t experts, int64_t H, int64_t I, int qt) {
+  constexpr int64_t kCus = 256;
+  const int64_t used = rows < experts ? rows : experts;
+  const int64_t avg = used > 0 ? (rows + used - 1) / used : 0;
+  WidePlan w;
+  w.hmax = qt == moe::kQF16 ? moe::kTallRows : moe::kWideRows;
+  if (used * moe::items_of((int)avg, w.hmax) * (I / moe::kBN) < kCus) w.hmax = moe::kLowRows;
+  w.bn256 = H % 256 == 0 && used * moe::items_of((int)avg, w.hmax) * (H / 256) >= kCus;
+  w.nt2 = H / (w.bn256 ? 256 : 128);
+  w.max_items = rows / w.hmax + used;  // sum of ceil(n / hmax) over `used` experts
+  return w;
 }
 
 bool aligned16(const void* p) { return ((uintptr_t)p & 15) == 0; }
@@ -105,7 +134,7 @@ int check_dims(int64_t T, int64_t H, int64_t I, int64_t E, int64_t k, int64_t bm
   if (E > 1024) return fail(MOE_ERR_UNSUPPORTED, "E=%lld > 1024", (long long)E);
   if (H <= 0 || I <= 0 || H % 128 || I % 128) return fail(MOE_ERR_UNSUPPORTED, "H=%lld and I=%lld must be positive multiples of 128", (long long)H, (long long)I);
   if (bm != 32 && bm != 64 && bm != 128 && bm != 256) return fail(MOE_ERR_UNSUPPORTED, "block_m=%lld not in {32,64,128}", (long long)bm);
-  if (cap_rows(T, k, E, bm) * I >= ((int64_t)1 << 31) * 2 || T * k >= ((int64_t)1 << 31)) return fail(MOE_ERR_UNSUPPORTED, "problem too large for 32-bit row indices");
+  if (too_large(T, k, E, I, bm) || T * k >= ((int64_t)1 << 31)) return fail(MOE_ERR_UNSUPPORTED, "problem too large for 32-bit row indices");
   return MOE_OK;
 }
 
@@ -161,11 +190,13 @@ int moe_run_prerouted_events(const void* x, const void* w_gate, const void* w_up
   p1.E = (int)E;
   p1.H = H;
   p1.I = I;
-  p1.absorb = 2;  // absorbed rows, pairs kept: few items here (moe_common.h kAbsorbRows)
+  const int64_t experts = E < blocks ? E : blocks;
+  const WidePlan wide = wide_plan(V > experts ? V : experts, experts, H, I, moe::kQF16);
+  p1.hmax = wide.hmax;
   // optional stage markers: ev[0] start, [1] stage 1, [2] stage 2
   auto mark = [&](int i) { if (stage_events && stage_events[i]) (void)hipEventRecord((hipEvent_t)stage_events[i], s); };
   mark(0);
-  int rc = check_launch(moe::launch_stage1(p1, 128, moe::kQF16, false, blocks, s), "stage1");
+  int rc = check_launch(moe::launch_stage1(p1, false, moe::kQF16, false, blocks, 0, s), "stage1");
   if (rc) return rc;
   mark(1);
 
@@ -183,8 +214,8 @@ int moe_run_prerouted_events(const void* x, const void* w_gate, const void* w_up
   p2.H = H;
   p2.I = I;
   p2.V = V;
-  p2.absorb = 2;  // as in Stage 1
-  rc = check_launch(moe::launch_stage2(p2, 128, moe::kQF16, false, blocks, s), "stage2");
+  p2.hmax = wide.hmax;
+  rc = check_launch(moe::launch_stage2(p2, false, moe::kQF16, false, wide.bn256, blocks, 0, s), "stage2");
   mark(2);
   return rc;
 }
@@ -270,7 +301,7 @@ int64_t moe_fused_workspace_bytes(int64_t T, int64_t H, int64_t I, int64_t E, in
   if (T < 0 || H <= 0 || I <= 0 || E <= 0 || k <= 0) return 0;
   // w8a8: 0 fp16, 1 int8, 2 fp8 (one padding rule for all)
   if (w8a8 < 0 || w8a8 > 2) return 0;
-  block_m = align_bm(T, E, k, H, block_m);
+  block_m = align_bm(T, E, k, H, I, block_m);
   return fused_layout(T, H, I, E, k, block_m, w8a8 == 2 ? moe::kQF8 : (w8a8 ? moe::kQI8 : moe::kQF16)).total;
 }
 
@@ -305,7 +336,8 @@ static int fused_common(int qt, const void* x, const float* logits, const void* 
   const int64_t Ee = E + (shared ? 1 : 0), ke = k + (shared ? 1 : 0);  // experts / choices incl. the shared one
   if (block_m != 0 && block_m != 32 && block_m != 64 && block_m != 128)
     return fail(MOE_ERR_UNSUPPORTED, "block_m=%lld not in {0,32,64,128}", (long long)block_m);
-  block_m = align_bm(T, shard ? E_route : Ee, ke, H, block_m);
+  const int64_t asked_bm = block_m;
+  block_m = align_bm(T, shard ? E_route : Ee, ke, H, I, block_m);
   int rc = check_dims(T, H, I, shard ? E_route : Ee, ke, block_m);
   if (rc) return rc;
   if (T == 0) return MOE_OK;
@@ -327,16 +359,14 @@ static int fused_common(int qt, const void* x, const float* logits, const void* 
       (shared && (!aligned16(wg_s) || !aligned16(wu_s) || !aligned16(wd_s))))
     return fail(MOE_ERR_INVALID_ARG, "x, weights, scales, out and workspace must be 16-byte aligned");
   const int64_t router_ws = w_router ? moe_router_workspace_bytes(T, H, E) : 0;
-  // a workspace sized for the 128-row padding (block_m = 128) keeps it
-  if (block_m == 256 && workspace_bytes < fused_layout(T, H, I, Ee, ke, 256, qt).total + router_ws) block_m = 128;
+  // a workspace sized for pick_bm's padding (128 or 32) keeps it
+  if (!asked_bm && workspace_bytes < fused_layout(T, H, I, Ee, ke, block_m, qt).total + router_ws)
+    block_m = pick_bm(T, shard ? E_route : Ee, ke);
   const FusedLayout L = fused_layout(T, H, I, Ee, ke, block_m, qt);
   const int64_t need = L.total + router_ws;
   if (workspace_bytes < need) return fail(MOE_ERR_WORKSPACE, "workspace %lld < %lld bytes", (long long)workspace_bytes, (long long)need);
-  // rows per item of each stage: block_m for both stages and every format
-  // (over the 256-row padding, 256-row items), unless built with
-  // MOE_S2_F16_256=0, where fp16 Stage 2 keeps 128-row paired items there
-  const int64_t bm1 = block_m;
-  const int64_t bm2 = block_m == 256 && qt == moe::kQF16 && MOE_S2_F16_256 == 0 ? 128 : block_m;
+  // 32-row blocks run narrow items, others wide ones
+  const bool narrow = block_m == 32;
   hipStream_t s = (hipStream_t)stream;
   char* ws = (char*)workspace;
   // routing written by route / router (ids, wts), read by align, Stage 2 and the combine (rids, rwts)
@@ -348,7 +378,13 @@ static int fused_common(int qt, const void* x, const float* logits, const void* 
   int32_t* gs = (int32_t*)(ws + L.gs);
   int32_t* go = (int32_t*)(ws + L.go);
   int32_t* gpo = (int32_t*)(ws + L.gpo);
+  int32_t* istart = (int32_t*)(ws + L.istart);
   const int64_t rows = cap_rows(T, ke, Ee, block_m);
+  // (a shard's share of the pairs decides how its items are shaped; the bound
+  // on their number holds for any routing)
+  WidePlan wide = wide_plan(shard ? (T * ke * E + E_route - 1) / E_route : T * ke, Ee, H, I, qt);
+  wide.max_items = T * ke / wide.hmax + (T * ke < Ee ? T * ke : Ee);
+  const int64_t max_blocks = narrow ? rows / 32 : wide.max_items;
   const int e_shared = shared ? (int)E : -1;
 
   // optional stage markers: ev[0] start, [1] routed, [2] aligned, [3] x quantised,
@@ -370,7 +406,7 @@ static int fused_common(int qt, const void* x, const float* logits, const void* 
     return rc;
   }
   mark(1);
-  if ((rc = check_launch(moe::launch_align(rids, (int)(T * ke), (int)Ee, (int)block_m, sorted, (int32_t*)(ws + L.bexp), gs, go, gpo, (int32_t*)(ws + L.whist), s, (int)e_begin), "align"))) return rc;
+  if ((rc = check_launch(moe::launch_align(rids, (int)(T * ke), (int)Ee, (int)block_m, sorted, (int32_t*)(ws + L.bexp), gs, go, gpo, (int32_t*)(ws + L.whist), s, (int)e_begin, narrow ? nullptr : istart, wide.hmax, (int)(I / moe::kBN), (int)wide.nt2), "align"))) return rc;
   mark(2);
   if (w8 && !route_quant && (rc = check_launch(moe::launch_quant_rows(x, T, H, ws + L.xq, (float*)(ws + L.sx), qt, s), "quantize_x"))) return rc;
   mark(3);
@@ -380,8 +416,8 @@ static int fused_common(int qt, const void* x, const float* logits, const void* 
   p1.wg = (const char*)wg;
   p1.wu = (const char*)wu;
   p1.h = ws + L.h;
-  p1.h_scale = qt == moe::kQF8 ? (float*)(ws + L.hs) : nullptr;
-  p1.hs_stride = rows;
+  p1.h_scale = qt == moe::kQF8 ? (uint8_t*)(ws + L.hs) : nullptr;
+  p1.hs_pitch = hs_pitch(I);
   p1.x_scale = w8 ? (const float*)(ws + L.sx) : nullptr;
   p1.sg = sg;
   p1.su = su;
@@ -397,8 +433,11 @@ static int fused_common(int qt, const void* x, const float* logits, const void* 
   p1.E = (int)Ee;
   p1.H = H;
   p1.I = I;
-  p1.absorb = 1;  // absorbed rows, pairs may become single items (moe_common.h kAbsorbRows)
-  if ((rc = check_launch(moe::launch_stage1(p1, (int)bm1, qt, true, rows / bm1, s), "stage1"))) return rc;
+  p1.istart = istart;
+  p1.xb = istart + Ee + 1;
+  p1.rows_cap = (int)rows;
+  p1.hmax = wide.hmax;
+  if ((rc = check_launch(moe::launch_stage1(p1, narrow, qt, true, max_blocks, T * ke, s), "stage1"))) return rc;
   // int8: h (fp16) -> per-row int8 codes + scales, for the routed rows only
   // (sorted id below the sentinel T * ke, row below gpo[E])
   if (qt == moe::kQI8 &&
@@ -409,14 +448,18 @@ static int fused_common(int qt, const void* x, const float* logits, const void* 
 
   moe::Stage2Params p2{};
   p2.a = qt == moe::kQI8 ? ws + L.hq : ws + L.h;
-  p2.a_scale = w8 ? (const float*)(ws + L.hs) : nullptr;
-  p2.as_stride = rows;
+  p2.a_scale = qt == moe::kQI8 ? (const float*)(ws + L.hs) : nullptr;
+  p2.a_scale8 = qt == moe::kQF8 ? (const uint8_t*)(ws + L.hs) : nullptr;
+  p2.as_pitch = hs_pitch(I);
   p2.wd = (const char*)wd;
   p2.sd = sd;
   p2.out = MOE_S2_SCATTER ? (char*)out : ws + L.ypair;
   p2.topk = (int)ke;
   p2.pos = (int32_t*)(ws + L.pos);
-  p2.absorb = 1;  // as in Stage 1
+  p2.istart = istart;
+  p2.xb = istart + Ee + 10;
+  p2.rows_cap = (int)rows;
+  p2.hmax = wide.hmax;
   p2.routed = rwts;
   p2.routed_f16 = 0;
   p2.gs = gs;
@@ -431,7 +474,7 @@ static int fused_common(int qt, const void* x, const float* logits, const void* 
   p2.H = H;
   p2.I = I;
   if (MOE_S2_SCATTER && (rc = check_launch(moe::launch_zero(out, T * H * 2, s), "zero_out"))) return rc;
-  if ((rc = check_launch(moe::launch_stage2(p2, (int)bm2, qt, true, rows / bm2, s), "stage2"))) return rc;
+  if ((rc = check_launch(moe::launch_stage2(p2, narrow, qt, true, wide.bn256, max_blocks, T * ke, s), "stage2"))) return rc;
   mark(5);
   if (MOE_S2_SCATTER) {  // Stage 2 added every pair row into `out`
     mark(6);
@@ -474,7 +517,7 @@ int moe_fused_forward_hidden(const void* x, const void* w_router, const float* b
 int64_t moe_fused_shared_workspace_bytes(int64_t T, int64_t H, int64_t I, int64_t E, int64_t k,
                                          int64_t block_m) {
   if (T < 0 || H <= 0 || I <= 0 || E <= 0 || k <= 0) return 0;
-  block_m = align_bm(T, E + 1, k + 1, H, block_m);
+  block_m = align_bm(T, E + 1, k + 1, H, I, block_m);
   return fused_layout(T, H, I, E + 1, k + 1, block_m, moe::kQF16).total + moe_router_workspace_bytes(T, H, E);
 }
 
@@ -495,7 +538,7 @@ int64_t moe_fused_ex_workspace_bytes(int64_t T, int64_t H, int64_t I, int64_t E,
                                      int shared, int with_router) {
   if (T < 0 || H <= 0 || I <= 0 || E <= 0 || k <= 0) return 0;
   const int64_t s = shared ? 1 : 0;
-  block_m = align_bm(T, E + s, k + s, H, block_m);
+  block_m = align_bm(T, E + s, k + s, H, I, block_m);
   return fused_layout(T, H, I, E + s, k + s, block_m, moe::kQF16).total + (with_router ? moe_router_workspace_bytes(T, H, E) : 0);
 }
 
@@ -516,7 +559,7 @@ int moe_fused_forward_ex(const void* x, const float* logits, const void* w_route
 int64_t moe_fused_shard_workspace_bytes(int64_t T, int64_t H, int64_t I, int64_t E_total, int64_t k,
                                         int64_t E_local, int64_t block_m) {
   if (T < 0 || H <= 0 || I <= 0 || E_total <= 0 || E_local <= 0 || k <= 0) return 0;
-  block_m = align_bm(T, E_total, k, H, block_m);
+  block_m = align_bm(T, E_total, k, H, I, block_m);
   return fused_layout(T, H, I, E_local, k, block_m, moe::kQF16).total;
 }
 
@@ -595,14 +638,15 @@ int moe_fused_forward_noalloc(const void* x, const float* logits, const float* b
                               float* topk_weights_out, void* stream) {
   if (block_m != 0 && block_m != 32 && block_m != 64 && block_m != 128)
     return fail(MOE_ERR_UNSUPPORTED, "block_m=%lld not in {0,32,64,128}", (long long)block_m);
-  int64_t bm = align_bm(T, E, k, H, block_m);
+  int64_t bm = align_bm(T, E, k, H, I, block_m);
   int rc = check_dims(T, H, I, E, k, bm);
   if (rc) return rc;
   if (T == 0) return MOE_OK;
-  // the padding the call will use: 256-row blocks only where they fit (as
-  // for any workspace sized for 128-row blocks)
+  // the padding the call will use: pick_bm's where a larger one does not fit
+  // (as for any workspace sized for that)
   int64_t need = fused_layout(T, H, I, E, k, bm, moe::kQF16).total;
-  if (bm == 256 && need > kNoAllocScratchBytes) need = fused_layout(T, H, I, E, k, 128, moe::kQF16).total;
+  if (!block_m && need > kNoAllocScratchBytes)
+    need = fused_layout(T, H, I, E, k, pick_bm(T, E, k), moe::kQF16).total;
   if (need > kNoAllocScratchBytes)
     return fail(MOE_ERR_WORKSPACE,
                 "moe_fused_forward_noalloc: T=%lld H=%lld I=%lld E=%lld k=%lld needs %lld bytes of scratch, the "

@@ -30,8 +30,8 @@ struct Stage1Params {
   const char* wg;           // [E, I, H]
   const char* wu;           // [E, I, H]
   char* h;                  // fp16 [padded rows, I] (fp16 and int8 operands) | fp8 [padded rows, I]
-  float* h_scale;           // fp8 only: [I/128][hs_stride] (block-major)
-  int64_t hs_stride;        // fp8 only: rows of each h_scale block (>= padded rows)
+  uint8_t* h_scale;         // fp8 only: E8M0 bytes [padded rows][hs_pitch], one per 128 columns
+  int64_t hs_pitch;         // fp8 only: bytes between rows of h_scale, a multiple of 16
   const float* x_scale;     // 8-bit only: [T]
   const float* sg;          // 8-bit only: [E, I]
   const float* su;          // 8-bit only: [E, I]
@@ -49,17 +49,20 @@ struct Stage1Params {
   int E;
   int64_t H;
   int64_t I;
-  int host_blocks;          // BM-row blocks the row buffers hold (set by the launcher);
-                            // direct: blocks of the launch (gidx entries, clamped)
-  int absorb = 0;           // fp16, 256-row or 128-row paired items, E <= 256: absorbed
-                            // rows; the blocks a pair must keep (moe_common.h), 0: off
+  int host_blocks;          // narrow: 32-row blocks the row buffers hold; direct: blocks of
+                            // the launch (gidx entries, clamped); set by the launcher
+  const int32_t* istart = nullptr;  // wide, gather: [E+1] items per N tile below each expert
+  const int32_t* xb = nullptr;      // wide, gather: [9] first item of each XCD
+  int rows_cap = 0;         // wide, gather: rows the buffers hold
+  int hmax = 0;             // wide: most rows of an item (moe_common.h Item)
 };
 
 // Stage 2: y = h Wd^T, scaled by the routing weight of each row.
 struct Stage2Params {
   const char* a;            // fp16|int8|fp8 [padded rows, I]
-  const float* a_scale;     // int8: [padded rows] (per row); fp8: [I/128][as_stride] (block-major)
-  int64_t as_stride;        // fp8 only: rows of each a_scale block (>= padded rows)
+  const float* a_scale;     // int8: [padded rows] (per row)
+  const uint8_t* a_scale8;  // fp8: E8M0 bytes [padded rows][as_pitch], one per 128 columns
+  int64_t as_pitch;         // fp8: bytes between rows of a_scale8, a multiple of 16
   const char* wd;           // [E, H, I]
   const float* sd;          // 8-bit only: [E, H]
   char* out;                // pre-routed: fp16 [P, H]; fused: fp16 [T*topk, H], row = the pair's
@@ -81,9 +84,11 @@ struct Stage2Params {
   int64_t H;
   int64_t I;
   int64_t V;                // pre-routed: entries of `routed` (raw index is clamped to V-1)
-  int host_blocks;          // BM-row blocks the row buffers hold (set by the launcher);
-                            // pre-routed: blocks of the launch (gidx entries, clamped)
-  int absorb = 0;           // fp16, 128-row paired items, E <= 256: absorbed rows; as in Stage 1
+  int host_blocks;          // as Stage 1's
+  const int32_t* istart = nullptr;
+  const int32_t* xb = nullptr;
+  int rows_cap = 0;
+  int hmax = 0;
   int topk = 0;             // fused, built with MOE_S2_SCATTER: choices per token; `out` is then
                             // fp16 [T, H] (zeroed first) and each pair row is added to its token's
                             // row with packed fp16 atomics
@@ -93,11 +98,15 @@ struct Stage2Params {
 // a kernel, not hipMemsetAsync, so that it can be captured in a graph.
 hipError_t launch_zero(void* p, int64_t n, hipStream_t stream);
 
-// qt: a QuantType
-hipError_t launch_stage1(const Stage1Params& p, int block_m, int qt, bool gather,
-                         int64_t max_blocks, hipStream_t stream);
-hipError_t launch_stage2(const Stage2Params& p, int block_m, int qt, bool fused,
-                         int64_t max_blocks, hipStream_t stream);
+// qt: a QuantType.  narrow: 32-row items over rows padded to 32 (gather / fused
+// only); otherwise wide items.  max_blocks: an upper bound on the items per N
+// tile (narrow: 32-row blocks; wide: row pieces; direct: 128-row blocks);
+// max_rows: of the routed rows (wide, gather / fused).
+// bn256: Stage 2's wide items take 256 features where H allows.
+hipError_t launch_stage1(const Stage1Params& p, bool narrow, int qt, bool gather,
+                         int64_t max_blocks, int64_t max_rows, hipStream_t stream);
+hipError_t launch_stage2(const Stage2Params& p, bool narrow, int qt, bool fused, bool bn256,
+                         int64_t max_blocks, int64_t max_rows, hipStream_t stream);
 
 // With e_shared >= 0 every token also gets the shared expert as choice k
 // (id e_shared, weight 1): ids / w rows hold k + 1 entries.
@@ -118,10 +127,14 @@ inline int align_pairs_per_group(int P, int groups, int nw) {
   return (per + 64 * nw - 1) / (64 * nw) * (64 * nw);
 }
 // e_off: pairs are bucketed by id - e_off; ids outside [e_off, e_off + E)
-// are dropped (an expert shard of a wider routing).
+// are dropped (an expert shard of a wider routing).  With `istart` (int32
+// [E + 1], may be null) the items of hmax rows per N tile below each expert
+// are written there (moe_common.h Item), and behind it, at istart + E + 1, the 9
+// XCD bounds of Stage 1's items (nt1 N tiles) and the 9 of Stage 2's (nt2).
 hipError_t launch_align(const int32_t* ids, int P, int E, int BM, int32_t* sorted_ids,
                         int32_t* block_expert, int32_t* gs, int32_t* go, int32_t* gpo,
-                        int32_t* whist, hipStream_t stream, int e_off = 0);
+                        int32_t* whist, hipStream_t stream, int e_off = 0, int32_t* istart = nullptr,
+                        int hmax = 1, int nt1 = 0, int nt2 = 0);
 // Router GEMM (x . w_router^T, K split in router_splits parts) + routing of
 // the summed partials; `part` holds router_partial_floats fp32, `logits`
 // (fp32 [T, E]) may be null.

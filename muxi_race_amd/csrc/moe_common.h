@@ -74,31 +74,6 @@ __device__ __forceinline__ void wait_stages(int ahead) {
   }
 }
 
-// s_waitcnt vmcnt(n) for a wave-uniform n known only at run time: the
-// immediate is picked by scalar branches; n above MAX waits for MAX instead
-// (a stricter wait).
-template <int MAX>
-__device__ __forceinline__ void wait_vmcnt_rt(int n) {
-  if constexpr (MAX <= 0) {
-    wait_vmcnt<0>();
-  } else {
-    if (n >= MAX) wait_vmcnt<MAX>();
-    else wait_vmcnt_rt<MAX - 1>(n);
-  }
-}
-
-// wait_stages for waves that issue q <= Q loads per stage (q wave-uniform,
-// the same for every stage of the wave).
-template <int Q, int N>
-__device__ __forceinline__ void wait_stages_q(int q, int ahead) {
-  if constexpr (N <= 0) {
-    wait_vmcnt<0>();
-  } else {
-    if (ahead >= N) wait_vmcnt_rt<Q * N>(q * N);
-    else wait_stages_q<Q, N - 1>(q, ahead);
-  }
-}
-
 // Workgroup barrier without a memory fence.  __syncthreads() would first wait
 // for every outstanding vector-memory operation (vmcnt(0)), which includes the
 // direct-to-LDS loads of the stages still in flight; the pipelines below wait
@@ -158,42 +133,23 @@ __device__ __forceinline__ void dma_to_lds(const void* g, void* lds) {
 // logical chunk (l%8) ^ swz(r), so lane l loads that chunk of its row; the 8
 // lanes of a row still cover its 128 contiguous bytes.  Wave w issues the
 // instructions for row groups NW*i + w.
-template <int ROWS, int NW, bool WEIGHTS_FIRST = false>
+template <int ROWS, int NW>
 struct DmaTile {
   static constexpr int NI = ROWS / (8 * NW);  // instructions per wave per K step
   static_assert(NI >= 1 && ROWS == 8 * NW * NI, "tile rows must be a multiple of 8 * waves");
   const char* src[NI];
 
   __device__ __forceinline__ static int row_of(int i) { return 8 * (NW * i + wave_id()) + (lane_id() >> 3); }
-  // rowp: address of K-step 0 of tile row row_of(i).
-  __device__ __forceinline__ void set(int i, const char* rowp) {
-    const int l = lane_id();
-    src[i] = rowp + (((l & 7) ^ swz(row_of(i))) << 4);
+  // This lane's 16 bytes of a tile row r at rowp (K step 0).
+  __device__ __forceinline__ static const char* at(int r, const char* rowp) {
+    return rowp + ((((lane_id() & 7) ^ swz(r)) & 7) << 4);
   }
-  // WEIGHTS_FIRST: instructions go out last row group first.  A stage holds
-  // token rows, then weight rows; the weight rows (HBM misses) are its long
-  // pole and the token rows (L2 hits) its short one.  Measured per kernel:
-  // the fp16 two-stage rings (mixtral's Stage 1 1.000 -> 0.982 ms, Stage 2
-  // 0.495 -> 0.482 ms) take it; the 8-bit 256-row Stage 2 (+2.5%) and the
-  // three-stage rings with their spread issue (dsv3 Stage 2 +1%) do not.
-  __device__ __forceinline__ static constexpr int order(int j) { return WEIGHTS_FIRST ? NI - 1 - j : j; }
+  // rowp: address of K-step 0 of tile row row_of(i).
+  __device__ __forceinline__ void set(int i, const char* rowp) { src[i] = at(row_of(i), rowp); }
   __device__ __forceinline__ void issue(char* lds, int ks) const {
     const int w = wave_id();
 #pragma unroll
-    for (int j = 0; j < NI; ++j) {
-      const int i = order(j);
-      dma_to_lds<16>(src[i] + (size_t)ks * kRowBytes, lds + 1024 * (NW * i + w));
-    }
-  }
-  // The instructions i with i % PARTS == part of issue(lds, ks).
-  template <int PARTS>
-  __device__ __forceinline__ void issue_part(char* lds, int ks, int part) const {
-    const int w = wave_id();
-#pragma unroll
-    for (int j = 0; j < NI; ++j) {
-      const int i = order(j);
-      if (j % PARTS == part) dma_to_lds<16>(src[i] + (size_t)ks * kRowBytes, lds + 1024 * (NW * i + w));
-    }
+    for (int i = 0; i < NI; ++i) dma_to_lds<16>(src[i] + (size_t)ks * kRowBytes, lds + 1024 * (NW * i + w));
   }
   // As issue(), with tile rows from `weights_from` on loaded under the
   // streaming weight policy (kNoStream: none); an instruction's 8 rows never
@@ -339,104 +295,54 @@ __device__ __forceinline__ uint32_t quant_code4(float x0, float x1, float x2, fl
   }
 }
 
+// Inclusive prefix sum over the wave's 64 lanes: Hillis-Steele inside each
+// 16-lane row with DPP row shifts (lanes shifted in from outside the row read
+// 0), then each row adds the totals of the rows before it (read from lanes 15,
+// 31, 47).  Integer adds, so the order of the terms does not matter.
+__device__ __forceinline__ int wave_inclusive_scan(int v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xF, 0xF, false);  // row_shr:1
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xF, 0xF, false);  // row_shr:2
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xF, 0xF, false);  // row_shr:4
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xF, 0xF, false);  // row_shr:8
+  const int r0 = __builtin_amdgcn_readlane(v, 15), r1 = __builtin_amdgcn_readlane(v, 31),
+            r2 = __builtin_amdgcn_readlane(v, 47);
+  const int row = lane_id() >> 4;
+  return v + (row > 0 ? r0 : 0) + (row > 1 ? r1 : 0) + (row > 2 ? r2 : 0);
+}
+
 // ---------------------------------------------------------------------------
-// Work schedule.  A launch covers the BM-row blocks of all experts times the
-// nt output-feature tiles of width BN.  M blocks of expert e are
-// [gpo[e]/BM, gpo[e+1]/BM); `host_blocks` is the number of BM-row blocks the
-// caller's buffers hold: expert blocks beyond it are never scheduled (so
-// inconsistent metadata cannot move an access out of the buffers), and with
-// `tail` set, blocks between the experts' last block and host_blocks are
-// scheduled as tail items (e = -1) covering padded rows that no expert owns.
-//
-// Pairing.  With `pair` set, two consecutive blocks of one expert form one
-// item of 2*BM rows x BN/2 features instead of two items of BM x BN: the same
-// LDS stage (2*BM + 2*(BN/2) = BM + 2*BN rows when BN = BM) and the same MFMA
-// work, but the expert's weight tile is streamed once for both blocks instead
-// of once per block.  An expert of nb blocks then has P = nb/2 paired blocks
-// and nb%2 single blocks; either way it yields nb * nt items.  Its items are
-// ordered by N tile t: the 2P paired items of the two half tiles of t, then
-// the single block's item of t, so all items reading one weight tile are
-// adjacent.
-//
-// Items are numbered expert-major and the item range is cut into 8
-// contiguous chunks, one per XCD (workgroup g runs on XCD g % 8 and is that
-// XCD's (g / 8)-th workgroup), so the items sharing a weight tile or a token
-// tile run close together on one XCD and re-read it from that XCD's L2.
+// Work schedules.  Items are numbered expert-major and the item range is cut
+// into 8 contiguous chunks, one per XCD (workgroup g runs on XCD g % 8 and is
+// that XCD's (g / 8)-th workgroup), so the items sharing a weight tile or a
+// token tile run close together on one XCD and re-read it from that XCD's L2.
 // ---------------------------------------------------------------------------
-struct Work {
-  int e;        // expert, or -1 for a tail block owned by no expert
-  int row0;     // first row of the tile (in the expert-sorted row space)
-  int rows;     // BM, 2*BM for a paired item, 3*BM for a triple item
-  int n0;       // first output feature of the tile
-  int bn;       // BN, or BN/2 for a paired or triple item
-  bool shared;  // other items of this launch read the same weight rows
-  int ar0 = 0;  // absorbed rows (see below): first sorted row ...
-  int nar = 0;  // ... and count (0: none)
-};
 
-// Absorbed rows.  An expert's rows rarely fill its last block: at mixtral's
-// ~512 rows per expert, 256-row blocks leave 5 of 8 experts a third block of
-// 2-30 rows, and its items (a quarter of Stage 1's) each stream a whole weight
-// tile for those few rows.  With absorption on, an expert whose last block
-// holding routed rows holds at most kAbsorbRows of them, after at least one
-// other block, gets no items for that block (nor for an empty block after it,
-// which the 256-row padding leaves to 128-row launches): its first item group
-// -- block 0's item, or both halves of pair 0 when paired -- takes those rows
-// as w.nar extra token rows from sorted row w.ar0, against the weight tile it
-// streams anyway.  The item count drops by those blocks' items, and the
-// launch's items are renumbered so that the 8 XCD chunks stay even.  The
-// expert scan keeps 4 values per chunk of 64 experts in registers, so
-// absorption needs E <= kAbsorbMaxE.  `absorb` is 0 (off) or the blocks of
-// items a paired launch must keep: 1 lets a two-block expert's pair become
-// one full-width item with the rows (fewer, longer items: measured faster in
-// saturated launches, dsv3's Stage 2 1.88 -> 1.82 ms), 2 keeps such pairs
-// (launches of few items, such as the reference's run_kernel cases 1-2,
-// measured slower with fewer items: 0.41 -> 0.43 and 0.73 -> 0.80 ms).
-constexpr int kAbsorbRows = 32;
-constexpr int kAbsorbMaxE = 256;
-
-// Triple items.  With pairing, an expert with an odd number nm >= 3 of blocks
-// holding items runs, per N tile, its (nm - 1) / 2 pairs on each half tile
-// and one single block over the whole tile; the single streams the tile
-// again at its own pace, and a 4 MiB L2 does not keep it across the lag.
-// With `triple` set (schedule_absorbed only), the expert's last three blocks
-// instead form one item per half tile, 3*BM rows x BN/2 features, so every
-// weight row of the expert's tile is streamed by exactly one item per pair
-// group: (nm - 1) * nt items instead of nm * nt.  An expert whose absorbed
-// rows would have to ride with the triple (nm == 3) keeps its pair and
-// single.
-
-
-__device__ __forceinline__ bool schedule_absorbed(int g, const int32_t* __restrict__ gpo,
-                                                  const int32_t* __restrict__ gs, int E, int BM, int BN,
-                                                  int nt, int host_blocks, bool pair, int absorb, bool triple,
-                                                  Work& w);
-
-__device__ __forceinline__ bool schedule(int g, const int32_t* __restrict__ gpo, int E, int BM, int BN,
-                                         int nt, int host_blocks, bool tail, bool pair, Work& w,
-                                         const int32_t* __restrict__ gs = nullptr, int absorb = 0,
-                                         bool triple = false) {
-  if (absorb > 0 && !tail && E <= kAbsorbMaxE)
-    return schedule_absorbed(g, gpo, gs, E, BM, BN, nt, host_blocks, pair, absorb, triple, w);
-  int expert_blocks = gpo[E] / BM;
-  expert_blocks = expert_blocks < host_blocks ? expert_blocks : host_blocks;
-  const int total_blocks = tail ? host_blocks : expert_blocks;
-  const int total = total_blocks * nt;
+// The number of workgroup g's item among `total`, or -1 (surplus workgroup).
+__device__ __forceinline__ int xcd_item(int g, int total) {
   const int per = (total + kNumXcd - 1) / kNumXcd;
   const int slot = g / kNumXcd;
   const int v = (g % kNumXcd) * per + slot;
-  if (slot >= per || v >= total) return false;
-  const int expert_items = expert_blocks * nt;
-  if (v >= expert_items) {
-    const int t = v - expert_items;
-    w.e = -1;
-    w.row0 = (expert_blocks + t / nt) * BM;
-    w.rows = BM;
-    w.n0 = (t % nt) * BN;
-    w.bn = BN;
-    w.shared = false;
-    return true;
-  }
+  return slot < per && v < total ? v : -1;
+}
+
+// 32-row items: one per BM-row block of an expert and output-feature tile of
+// width BN, an expert's items ordered by tile.  M blocks of expert e are
+// [gpo[e]/BM, gpo[e+1]/BM); `host_blocks` is the number of BM-row blocks the
+// caller's buffers hold: expert blocks beyond it are never scheduled, so
+// inconsistent metadata cannot move an access out of the buffers.
+struct Work {
+  int e;        // expert
+  int row0;     // first row of the block (in the expert-sorted row space)
+  int n0;       // first output feature of the tile
+  bool shared;  // other items of this launch read the same weight rows
+};
+
+__device__ __forceinline__ bool schedule(int g, const int32_t* __restrict__ gpo, int E, int BM, int BN,
+                                         int nt, int host_blocks, Work& w) {
+  int blocks = gpo[E] / BM;
+  blocks = blocks < host_blocks ? blocks : host_blocks;
+  const int v = xcd_item(g, blocks * nt);
+  if (v < 0) return false;
   // e = (number of experts whose first item is <= v) - 1, found with ballots.
   const int l = lane_id();
   int cnt = 0;
@@ -453,202 +359,260 @@ __device__ __forceinline__ bool schedule(int g, const int32_t* __restrict__ gpo,
   if (nb <= 0) return false;
   const int local = v - b0 * nt;
   const int t = local / nb;  // N tile
-  const int r = local % nb;  // item within tile t
-  const int P = pair ? nb / 2 : 0;
   w.e = e;
-  w.shared = pair ? nb > 2 : nb > 1;
-  if (r < 2 * P) {
-    w.rows = 2 * BM;
-    w.row0 = (b0 + 2 * (r % P)) * BM;
-    w.bn = BN / 2;
-    w.n0 = (2 * t + r / P) * (BN / 2);
-  } else {
-    w.rows = BM;
-    w.row0 = (b0 + r) * BM;
-    w.bn = BN;
-    w.n0 = t * BN;
-  }
-  return (w.row0 + w.rows) / BM <= host_blocks && t < nt;
+  w.shared = nb > 1;
+  w.row0 = (b0 + local % nb) * BM;
+  w.n0 = t * BN;
+  return w.row0 / BM < host_blocks && t < nt;
 }
 
-// schedule() with absorbed rows (E <= kAbsorbMaxE, no ownerless tail items).
-// Lane l scans expert 64c + l of chunk c: nb blocks, of which d (the last
-// block with routed rows, if absorbed, and any empty block after it) get no
-// items, and one more block's worth of items goes when the expert takes a
-// triple item.  Expert e's items start at (gpo[e]/BM - sum of those below e)
-// * nt, counted with three ballots per chunk; the selected expert is the last
-// whose first item is <= the workgroup's item.
-__device__ __forceinline__ bool schedule_absorbed(int g, const int32_t* __restrict__ gpo,
-                                                  const int32_t* __restrict__ gs, int E, int BM, int BN,
-                                                  int nt, int host_blocks, bool pair, int absorb, bool triple,
-                                                  Work& w) {
-  constexpr int C = kAbsorbMaxE / 64;
+// Wide items (more than 32 rows per expert).  An expert of n routed rows runs
+// c = ceil(n / hmax) items per N tile, of rows_of(n, c) rows each (the last one
+// of what is left): its rows split evenly in multiples of 32, so an item
+// streams a weight tile for as many rows as the tallest tile holds and no item
+// is left with a few.  All items span the whole N tile; item v of expert e is
+// N tile (v - first) / c, row piece (v - first) % c, so the c items reading one
+// weight tile are adjacent.  hmax is kTallRows where the tiles take absorbed
+// rows (moe_common.h kAbsorbRows), kWideRows otherwise, and kLowRows where the
+// launch would have fewer items than the chip has CUs.
+constexpr int kLowRows = 128, kWideRows = 256;
+constexpr int kAbsorbRows = 32;  // rows past kWideRows that an item takes along
+constexpr int kTallRows = kWideRows + kAbsorbRows;
+
+__host__ __device__ inline int items_of(int n, int hmax) { return (n + hmax - 1) / hmax; }
+__device__ __forceinline__ int rows_of(int n, int c) { return (n + 32 * c - 1) / (32 * c) * 32; }
+
+struct Item {
+  int e;         // expert, or -1 (rows owned by no expert)
+  int row0;      // first row
+  int actual;    // routed rows of this piece (<= hmax): which tile runs the item
+  int n0;        // first output feature of the tile
+  int zero_end;  // pre-routed, the expert's last piece: rows [row0 + actual, zero_end) have no token
+  bool shared;   // other items of this launch read the same weight rows
+};
+
+// Fused launches: istart[e] = items per N tile of the experts below e, and XCD x
+// runs the items [xb[x], xb[x + 1]) (both written by align); e's rows are
+// [gpo[e], gpo[e] + gs[e]).  rows_cap: rows the caller's buffers hold.
+__device__ __forceinline__ bool item_fused(int g, const int32_t* __restrict__ istart, const int32_t* __restrict__ xb,
+                                           const int32_t* __restrict__ gs, const int32_t* __restrict__ gpo, int E,
+                                           int BN, int nt, int rows_cap, Item& it) {
+  const int v = xb[g % kNumXcd] + g / kNumXcd;
+  if (v >= xb[g % kNumXcd + 1]) return false;
   const int l = lane_id();
-  int cb0[C], cnb[C], cd[C];
-  uint64_t cm1[C], cm2[C], cm3[C];
-  int dtot = 0;
-#pragma unroll
-  for (int c = 0; c < C; ++c) {
-    const int e = 64 * c + l;
-    int b0 = 0, nb = 0, d = 0;
-    bool tri = false;
-    if (e < E) {
-      b0 = gpo[e] / BM;
-      nb = gpo[e + 1] / BM - b0;
-      const int n = gs[e];
-      const int v = (n + BM - 1) / BM;  // blocks holding routed rows
-      if (v >= (pair ? absorb : 1) + 1 && n - (v - 1) * BM <= kAbsorbRows && nb >= v && nb - (v - 1) <= 3)
-        d = nb - (v - 1);
-      const int nm = nb - d;
-      tri = triple && pair && nm >= 3 && (nm & 1) && (d == 0 || nm >= 5);
-    }
-    cb0[c] = b0;
-    cnb[c] = nb;
-    cd[c] = d + (tri ? 4 : 0);  // bit 2: the expert takes a triple item
-    cm1[c] = __ballot(d & 1);
-    cm2[c] = __ballot((d >> 1) & 1);
-    cm3[c] = __ballot(tri);
-    dtot += __popcll(cm1[c]) + 2 * __popcll(cm2[c]) + __popcll(cm3[c]);
+  int cnt = 0;
+  for (int base = 0; base < E; base += 64) {
+    const int e = base + l;
+    cnt += __popcll(__ballot(e < E && istart[e < E ? e : 0] * nt <= v));
   }
-  int expert_blocks = gpo[E] / BM;
-  expert_blocks = expert_blocks < host_blocks ? expert_blocks : host_blocks;
-  const int total = (expert_blocks - dtot) * nt;
-  const int per = (total + kNumXcd - 1) / kNumXcd;
-  const int slot = g / kNumXcd;
-  const int v = (g % kNumXcd) * per + slot;
-  if (total <= 0 || slot >= per || v >= total) return false;
-  const uint64_t below = (1ull << l) - 1;  // l <= 63
-  int e = -1, eb0 = 0, enb = 0, ed = 0, estart = 0, carry = 0;
-#pragma unroll
-  for (int c = 0; c < C; ++c) {
-    const int start = (cb0[c] - carry - __popcll(cm1[c] & below) - 2 * __popcll(cm2[c] & below) -
-                       __popcll(cm3[c] & below)) * nt;
-    const int k = __popcll(__ballot(64 * c + l < E && start <= v));
-    if (k > 0) {  // wave-uniform
-      e = 64 * c + k - 1;
-      eb0 = __shfl(cb0[c], k - 1);
-      enb = __shfl(cnb[c], k - 1);
-      ed = __shfl(cd[c], k - 1);
-      estart = __shfl(start, k - 1);
-    }
-    carry += __popcll(cm1[c]) + 2 * __popcll(cm2[c]) + __popcll(cm3[c]);
-  }
-  if (e < 0) return false;  // only with inconsistent metadata (gpo[0] > 0)
-  const int etri = triple ? ed >> 2 : 0;  // the expert takes a triple item
-  if (triple) ed &= 3;
-  const int nm = enb - ed;  // blocks with items
-  if (nm <= 0) return false;
-  const int ni = nm - etri;  // items per N tile
-  const int local = v - estart;
-  const int t = local / ni;  // N tile
-  const int r = local % ni;  // item within tile t
-  const int P = pair ? (nm - 3 * etri) / 2 : 0;  // pairs per half tile (besides the triple)
-  w.e = e;
-  w.shared = pair ? ni > 2 : ni > 1;
-  if (r < 2 * P) {
-    w.rows = 2 * BM;
-    w.row0 = (eb0 + 2 * (r % P)) * BM;
-    w.bn = BN / 2;
-    w.n0 = (2 * t + r / P) * (BN / 2);
-  } else if (etri) {  // r = 2P, 2P + 1: the triple on half tile r - 2P
-    w.rows = 3 * BM;
-    w.row0 = (eb0 + 2 * P) * BM;
-    w.bn = BN / 2;
-    w.n0 = (2 * t + r - 2 * P) * (BN / 2);
-  } else {
-    w.rows = BM;
-    w.row0 = (eb0 + r) * BM;
-    w.bn = BN;
-    w.n0 = t * BN;
-  }
-  w.ar0 = 0;
-  w.nar = 0;
-  if (ed > 0 && (P > 0 ? (r < 2 * P && r % P == 0) : r == 0)) {
-    w.ar0 = (eb0 + nm) * BM;
-    w.nar = gs[e] - nm * BM;  // 1 .. kAbsorbRows
-  }
-  return (w.row0 + w.rows) / BM <= host_blocks && (w.nar == 0 || w.ar0 / BM < host_blocks) && t < nt;
+  const int e = cnt - 1;  // an empty expert starts where the next one does, so e has items
+  const int i0 = istart[e], c = istart[e + 1] - i0;
+  if (c <= 0) return false;
+  const int n = gs[e], r = rows_of(n, c);
+  const int local = v - i0 * nt;
+  const int t = local / c, i = local % c;
+  it.e = e;
+  it.row0 = gpo[e] + i * r;
+  it.actual = n - i * r < r ? n - i * r : r;
+  it.n0 = t * BN;
+  it.zero_end = 0;
+  it.shared = c > 1;
+  return it.actual > 0 && it.row0 + it.actual <= rows_cap;
 }
 
-// Pre-routed launches (the reference operator): block b's expert is
-// gidx[b] (problem_detail.json:50 note 5; submission.py:1444), and the launch
-// covers blocks [0, nblk) with nblk = min(gidx entries, blocks of the row
-// buffers), as submission.py:2115 launches group_idx_for_bx.numel() blocks.
-// Item v belongs to block v / nt; the maximal run of consecutive blocks with
-// that block's gidx value is treated as one expert's blocks above (paired
-// items, N-tile-major order), so items [s * nt, (s + n) * nt) cover run
-// [s, s + n) exactly once whatever the values are.  Two blocks of one run
-// form a valid paired item for any group metadata: row m of the pair is
-// valid iff m < gs[e] - (row0 - gpo[e]), which is the per-block rule of each
-// half.  A gidx value outside [0, E) gives w.e = -1 (rows owned by no expert).
+// Pre-routed launches (the reference operator): block b of 128 rows belongs to
+// expert gidx[b] (problem_detail.json:50 note 5; submission.py:1444), and the
+// launch covers blocks [0, nblk) with nblk = min(gidx entries, blocks of the
+// row buffers), as submission.py:2115 launches group_idx_for_bx.numel()
+// blocks.  The maximal run [s, end) of consecutive blocks with one gidx value
+// is treated as one expert: its first n = clamp(gs[e] - (128 s - gpo[e]), 0,
+// 128 (end - s)) rows are routed (the per-block rule of each of its blocks),
+// and the rest have no token.  A run without tokens still has one item per N
+// tile, which writes its rows as 0.  A gidx value outside [0, E) gives e = -1
+// (rows owned by no expert).
 //
-// Absorbed rows here keep the numbering: with `absorb` set, a run of two or
-// more blocks whose last block holds 1..kAbsorbRows routed rows (by gs and
-// gpo) gives that block's items nothing to do (they end at once), and the
-// run's first item group takes its rows, as schedule_absorbed describes.
-__device__ __forceinline__ bool schedule_bx(int g, const int32_t* __restrict__ gidx, int nblk, int E, int BM,
-                                            int BN, int nt, bool pair, Work& w,
-                                            const int32_t* __restrict__ gs = nullptr,
-                                            const int32_t* __restrict__ gpo = nullptr, int absorb = 0) {
-  const int total = nblk * nt;
-  const int per = (total + kNumXcd - 1) / kNumXcd;
-  const int slot = g / kNumXcd;
-  const int v = (g % kNumXcd) * per + slot;
-  if (slot >= per || v >= total) return false;
-  const int bs = v / nt;
-  const int val = gidx[bs];
-  const int l = lane_id();
-  // run start: the nearest block below bs with another value (or -1)
-  int s = -1;
-  for (int base = bs - 1; base >= 0 && s < 0; base -= 64) {
-    const int b = base - l;
-    const bool diff = b < 0 || gidx[b] != val;
-    const uint64_t m = __ballot(diff);
-    if (m) s = base - (__ffsll((unsigned long long)m) - 1) + 1;
+// The items below a run are counted here, by the workgroup's 512 threads, 512
+// blocks at a time: block j of a run counts the pieces that its rows add,
+// items_of(min(n, 128 (j + 1))) - items_of(min(n, 128 j)), which sums to the
+// run's.  (Numbering by blocks instead, with the surplus items ending at once,
+// left the XCDs unequal work: 22 experts of 155 rows and 10 of 112, H 7168, I
+// 2048, Stage 1 551 us.)
+struct RunScan {
+  int smem_s[8], smem_p[8];
+};
+
+__device__ __forceinline__ bool item_bx(int g, const int32_t* __restrict__ gidx, int nblk, int E, int BN, int nt,
+                                        const int32_t* __restrict__ gs, const int32_t* __restrict__ gpo, int hmax,
+                                        char* smem, Item& it) {
+  constexpr int BM = 128, kThreads = 512;
+  RunScan* sh = reinterpret_cast<RunScan*>(smem);
+  const int l = lane_id(), w = wave_id();
+  // pass over all blocks; f(block, first of its run, items below it)
+  auto sweep = [&](auto&& f) {
+    int carry_s = 0, carry_p = 0;
+    for (int base = 0; base < nblk; base += kThreads) {
+      const int b = base + (int)threadIdx.x;
+      const int bc = b < nblk ? b : nblk - 1;
+      const int val = gidx[bc], before = gidx[bc > 0 ? bc - 1 : 0];
+      const bool first = b < nblk && (b == 0 || val != before);
+      const uint64_t m = __ballot(first);
+      if (l == 0) sh->smem_s[w] = m ? base + 64 * w + 63 - __builtin_clzll(m) : -1;
+      const bool owned = val >= 0 && val < E;
+      const int ec = owned ? val : 0;
+      const int gs_e = gs[ec], gpo_e = gpo[ec];
+      __syncthreads();
+      int s = carry_s;
+      for (int v = 0; v < w; ++v) s = sh->smem_s[v] >= 0 ? sh->smem_s[v] : s;
+      const uint64_t upto = m & (l == 63 ? ~0ull : (1ull << (l + 1)) - 1);
+      if (upto) s = base + 64 * w + 63 - __builtin_clzll(upto);
+      const int64_t left = owned ? (int64_t)gs_e - ((int64_t)s * BM - gpo_e) : 0;
+      const int64_t lo = (int64_t)(b - s) * BM, hi = lo + BM;
+      int c = 0;
+      if (b < nblk) {
+        if (left > 0) c = items_of((int)(left < hi ? left : hi), hmax) - items_of((int)(left < lo ? left : lo), hmax);
+        else c = first;
+      }
+      const int inc = wave_inclusive_scan(c);
+      if (l == 63) sh->smem_p[w] = inc;
+      __syncthreads();
+      int below = carry_p;
+      for (int v = 0; v < 8; ++v) {
+        if (v == w) f(b, first, below + inc - c);
+        below += sh->smem_p[v];
+        carry_s = sh->smem_s[v] >= 0 ? sh->smem_s[v] : carry_s;
+      }
+      carry_p = below;
+      __syncthreads();  // the next pass (or caller) writes the same memory
+    }
+    return carry_p;
+  };
+  int p0 = 0;
+  bool first0 = false;
+  const int total = sweep([&](int b, bool first, int below) {
+    if (b < kThreads) {
+      first0 = first;
+      p0 = below;
+    }
+  });
+  const int v = xcd_item(g, total * nt);
+  if (v < 0) return false;
+  // the last run whose first item is <= v: block s, items below it ps
+  int s = -1, ps = 0;
+  auto find = [&](int b, bool first, int below) {
+    const uint64_t m = __ballot(first && below * nt <= v);
+    if (m) {
+      const int lane = 63 - __builtin_clzll(m);
+      s = __shfl(b, lane);
+      ps = __shfl(below, lane);
+    }
+  };
+  if (nblk <= kThreads) find((int)threadIdx.x, first0, p0);
+  else sweep(find);
+  if (l == 0) {
+    sh->smem_s[w] = s;
+    sh->smem_p[w] = ps;
   }
-  if (s < 0) s = 0;
-  // run end: the nearest block above bs with another value (or nblk)
+  __syncthreads();
+  for (int u = 0; u < 8; ++u)
+    if (sh->smem_s[u] > s) {
+      s = sh->smem_s[u];
+      ps = sh->smem_p[u];
+    }
+  s = __builtin_amdgcn_readfirstlane(s);
+  ps = __builtin_amdgcn_readfirstlane(ps);
+  __syncthreads();  // the caller reuses smem
+  const int val = gidx[s];
+  // run end: the nearest block above s with another value (or nblk)
   int end = -1;
-  for (int base = bs + 1; end < 0; base += 64) {
+  for (int base = s + 1; end < 0; base += 64) {
     const int b = base + l;
     const bool diff = b >= nblk || gidx[b] != val;
     const uint64_t m = __ballot(diff);
     if (m) end = base + (__ffsll((unsigned long long)m) - 1);
   }
-  const int nb = end - s;
-  w.e = val >= 0 && val < E ? val : -1;
-  int nm = nb, last = 0;  // blocks with items; routed rows of an absorbed last block
-  if (absorb > 0 && w.e >= 0 && nb >= (pair ? absorb : 1) + 1) {
-    last = gs[w.e] - ((s + nb - 1) * BM - gpo[w.e]);
-    if (last >= 1 && last <= kAbsorbRows) nm = nb - 1;
+  it.e = val >= 0 && val < E ? val : -1;
+  int n = 0;
+  if (it.e >= 0) {
+    const int64_t left = (int64_t)gs[it.e] - ((int64_t)s * BM - gpo[it.e]);
+    const int64_t cap = (int64_t)(end - s) * BM;
+    n = (int)(left < 0 ? 0 : (left > cap ? cap : left));
   }
-  const int local = v - s * nt;
-  const int t = local / nb;
-  const int r = local % nb;
-  if (r >= nm) return false;  // the absorbed block's item: its rows ride with the run's first items
-  const int P = pair ? nm / 2 : 0;
-  w.shared = pair ? nm > 2 : nm > 1;
-  if (r < 2 * P) {
-    w.rows = 2 * BM;
-    w.row0 = (s + 2 * (r % P)) * BM;
-    w.bn = BN / 2;
-    w.n0 = (2 * t + r / P) * (BN / 2);
-  } else {
-    w.rows = BM;
-    w.row0 = (s + r) * BM;
-    w.bn = BN;
-    w.n0 = t * BN;
-  }
-  w.ar0 = 0;
-  w.nar = 0;
-  if (nm < nb && (P > 0 ? (r < 2 * P && r % P == 0) : r == 0)) {
-    w.ar0 = (s + nm) * BM;
-    w.nar = last;
-  }
-  return true;
+  const int c = n > 0 ? items_of(n, hmax) : 1;
+  const int local = v - ps * nt;
+  const int t = local / c, i = local % c;
+  const int r = n > 0 ? rows_of(n, c) : 0;
+  it.row0 = s * BM + i * r;
+  it.actual = n - i * r < r ? n - i * r : r;
+  it.n0 = t * BN;
+  it.zero_end = i == c - 1 ? end * BM : 0;
+  it.shared = c > 1;
+  return t < nt;
 }
 
-// Upper bound on the workgroups `schedule` needs for `blocks` M blocks.
+// XCD shares of a fused launch's items, for one lane: the first item of XCD x
+// (x = 8: the end) and the cost of the items before it.  `weighted`: the items
+// are cut where the cost is an eighth each; otherwise into equal numbers.  An
+// item of r rows costs kItemCost + r: at 256 experts of H 7168, I 2048 a Stage 1
+// step took 1.28 us at 32 rows, 1.42 at 128, 1.64 at 160 and 2.2 at 256.  The
+// experts below e cost K(e) = kItemCost * ist[e] + gof[e] per N tile.
+constexpr int kItemCost = 256;
+struct XcdCut {
+  int item;
+  double cost;
+};
+__device__ __forceinline__ XcdCut xcd_cut(int x, bool weighted, const int* ist, const int* gof, int E, int nt) {
+  const int total = ist[E] * nt;
+  auto K = [&](int e) { return (double)kItemCost * ist[e] + (double)gof[e]; };
+  const double all = K(E) * nt;
+  XcdCut r;
+  const int per = (total + kNumXcd - 1) / kNumXcd;
+  r.item = x * per < total ? x * per : total;
+  r.cost = all * x / kNumXcd;
+  if (x == kNumXcd || (!weighted && r.item == total)) return XcdCut{total, all};
+  // the last expert that starts at or before the cut
+  int lo = 0, hi = E;
+  while (hi - lo > 1) {
+    const int mid = (lo + hi) / 2;
+    if (weighted ? K(mid) * nt <= r.cost : ist[mid] * nt <= r.item) lo = mid;
+    else hi = mid;
+  }
+  const int c = ist[lo + 1] - ist[lo];
+  const double ce = K(lo + 1) - K(lo);  // of its c pieces
+  if (weighted) {
+    const int in = c > 0 ? (int)((r.cost - K(lo) * nt) * c / ce) : 0;
+    r.item = ist[lo] * nt + (in < c * nt ? in : c * nt);
+  } else {
+    r.cost = K(lo) * nt + (c > 0 ? (r.item - ist[lo] * nt) * ce / c : 0.0);
+  }
+  return r;
+}
+// Both cuts of one launch on lanes 0..8 (equal numbers) and 9..17 (equal cost)
+// of a wave, and the better one written to xb[0..8]: the one whose slowest XCD
+// needs less time, an XCD running its items kCusPerXcd at a time.  Equal cost
+// pays where experts differ and there are many rounds; with two rounds of like
+// items it would leave some XCD a third.
+constexpr int kCusPerXcd = 32;
+__device__ __forceinline__ void xcd_shares(const int* ist, const int* gof, int E, int nt, int32_t* __restrict__ xb) {
+  const int l = lane_id();
+  const int x = l % 9;
+  XcdCut cut = {0, 0.0};
+  if (l < 18) cut = xcd_cut(x, l >= 9, ist, gof, E, nt);
+  const int items = __shfl_down(cut.item, 1) - cut.item;
+  const float cost = __shfl_down((float)cut.cost, 1) - (float)cut.cost;
+  float t = 0.0f;
+  if (l < 18 && x < 8 && items > 0) t = (float)((items + kCusPerXcd - 1) / kCusPerXcd) * cost / (float)items;
+  float slow[2] = {0.0f, 0.0f};
+  for (int q = 0; q < 18; ++q) slow[q / 9] = fmaxf(slow[q / 9], __shfl(t, q));
+  const bool weighted = slow[1] < slow[0];
+  if (l < 18 && (l >= 9) == weighted) xb[x] = cut.item;
+}
+// An upper bound on an XCD's items either way, for `pieces` items per N tile and
+// `rows` routed rows in all.
+inline int64_t xcd_items_bound(int64_t pieces, int64_t rows, int64_t nt) {
+  return (pieces * kItemCost + rows) * nt / (kNumXcd * kItemCost) + 2;
+}
+
+// Workgroups of a launch of `blocks` blocks (or row pieces) x `ntiles` items.
 inline int64_t schedule_grid(int64_t blocks, int64_t ntiles) {
   const int64_t total = blocks * ntiles;
   const int64_t per = (total + kNumXcd - 1) / kNumXcd;

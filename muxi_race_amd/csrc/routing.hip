@@ -118,28 +118,21 @@ __device__ __forceinline__ void align_place_range(const int32_t* __restrict__ id
   }
 }
 
-// Inclusive prefix sum over the wave's 64 lanes: Hillis-Steele inside each
-// 16-lane row with DPP row shifts (lanes shifted in from outside the row read
-// 0), then each row adds the totals of the rows before it (read from lanes 15,
-// 31, 47).  Integer adds, so the order of the terms does not matter.
-__device__ __forceinline__ int wave_inclusive_scan(int v) {
-  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xF, 0xF, false);  // row_shr:1
-  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xF, 0xF, false);  // row_shr:2
-  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xF, 0xF, false);  // row_shr:4
-  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xF, 0xF, false);  // row_shr:8
-  const int r0 = __builtin_amdgcn_readlane(v, 15), r1 = __builtin_amdgcn_readlane(v, 31),
-            r2 = __builtin_amdgcn_readlane(v, 47);
-  const int row = lane_id() >> 4;
-  return v + (row > 0 ? r0 : 0) + (row > 1 ? r1 : 0) + (row > 2 ? r2 : 0);
-}
+// The wide items' plan: see launch_align.
+struct ItemPlan {
+  int32_t* istart;
+  int hmax, nt1, nt2;
+};
 
 // Expert scan by one wave: tot[E] -> padded offsets pstart[E+1] in LDS, and
-// (when `out`) group sizes / offsets / padded offsets in global memory.
+// (when `out`) group sizes / offsets / padded offsets, and the wide items' plan
+// when one is asked for, in global memory.  ist, gof: [E+1] ints of LDS each.
 __device__ __forceinline__ void align_expert_scan(const int* tot, int E, int BM, int* pstart, bool out,
                                                   int32_t* __restrict__ gs, int32_t* __restrict__ go,
-                                                  int32_t* __restrict__ gpo) {
+                                                  int32_t* __restrict__ gpo, const ItemPlan& plan, int* ist,
+                                                  int* gof) {
   const int l = lane_id();
-  int carry = 0, carry_p = 0;
+  int carry = 0, carry_p = 0, carry_i = 0;
   for (int base = 0; base < E; base += 64) {
     const int e = base + l;
     const int c = e < E ? tot[e] : 0;
@@ -153,6 +146,14 @@ __device__ __forceinline__ void align_expert_scan(const int* tot, int E, int BM,
         gpo[e] = carry_p + ip - pc;
       }
     }
+    if (out && plan.istart) {  // uniform
+      const int ni = items_of(c, plan.hmax), ii = wave_inclusive_scan(ni);
+      if (e < E) {
+        plan.istart[e] = ist[e] = carry_i + ii - ni;
+        gof[e] = carry + ic - c;
+      }
+      carry_i += __builtin_amdgcn_readlane(ii, 63);
+    }
     carry += __builtin_amdgcn_readlane(ic, 63);
     carry_p += __builtin_amdgcn_readlane(ip, 63);
   }
@@ -162,6 +163,15 @@ __device__ __forceinline__ void align_expert_scan(const int* tot, int E, int BM,
       go[E] = carry;
       gpo[E] = carry_p;
     }
+  }
+  if (out && plan.istart) {
+    if (l == 0) {
+      plan.istart[E] = ist[E] = carry_i;
+      gof[E] = carry;
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");  // this wave's LDS writes, before other lanes read them
+    xcd_shares(ist, gof, E, plan.nt1, plan.istart + E + 1);
+    xcd_shares(ist, gof, E, plan.nt2, plan.istart + E + 10);
   }
 }
 
@@ -195,11 +205,13 @@ template <int NW>
 __global__ __launch_bounds__(64 * NW) void align_small_kernel(
     const int32_t* __restrict__ ids, int P, int E, int e_off, int BM, int32_t* __restrict__ sorted_ids,
     int32_t* __restrict__ block_expert, int32_t* __restrict__ gs, int32_t* __restrict__ go,
-    int32_t* __restrict__ gpo) {
+    int32_t* __restrict__ gpo, ItemPlan plan) {
   extern __shared__ int sm[];
   int* hist = sm;                 // [NW][E]: wave w's count of expert e, then its first row among e's
   int* tot = sm + NW * E;         // [E]
   int* pstart = tot + E;          // [E+1] padded offsets
+  int* ist = pstart + E + 1;      // [E+1], with an item plan only
+  int* gof = ist + E + 1;         // [E+1]
   const int tid = threadIdx.x, w = tid >> 6, l = lane_id();
   const int nbits = bits_for(E);
   const int R = ((P + NW - 1) / NW + 63) / 64 * 64;  // <= 64 * kAlignUnroll (launch_align checks)
@@ -242,7 +254,7 @@ __global__ __launch_bounds__(64 * NW) void align_small_kernel(
     tot[e] = run;
   }
   __syncthreads();
-  if (w == 0) align_expert_scan(tot, E, BM, pstart, true, gs, go, gpo);
+  if (w == 0) align_expert_scan(tot, E, BM, pstart, true, gs, go, gpo, plan, ist, gof);
   __syncthreads();
   const int rows = pstart[E];
   for (int r = tid; r < rows; r += 64 * NW) sorted_ids[r] = P;
@@ -266,11 +278,13 @@ template <int NW>
 __global__ __launch_bounds__(64 * NW) void align_kernel(
     const int32_t* __restrict__ ids, int P, int E, int e_off, int BM, int32_t* __restrict__ sorted_ids,
     int32_t* __restrict__ block_expert, int32_t* __restrict__ gs, int32_t* __restrict__ go,
-    int32_t* __restrict__ gpo) {
+    int32_t* __restrict__ gpo, ItemPlan plan) {
   extern __shared__ int sm[];
   int* hist = sm;                 // [NW][E]
   int* tot = sm + NW * E;         // [E]
   int* pstart = tot + E;          // [E+1] padded offsets
+  int* ist = pstart + E + 1;      // [E+1], with an item plan only
+  int* gof = ist + E + 1;         // [E+1]
   const int tid = threadIdx.x, w = tid >> 6;
   const int nbits = bits_for(E);
   const int R = ((P + NW - 1) / NW + 63) / 64 * 64;
@@ -288,7 +302,7 @@ __global__ __launch_bounds__(64 * NW) void align_kernel(
     tot[e] = run;
   }
   __syncthreads();
-  if (w == 0) align_expert_scan(tot, E, BM, pstart, true, gs, go, gpo);
+  if (w == 0) align_expert_scan(tot, E, BM, pstart, true, gs, go, gpo, plan, ist, gof);
   __syncthreads();
   for (int e = tid; e < E; e += 64 * NW)
     for (int v = 0; v < NW; ++v) hist[v * E + e] += pstart[e];
@@ -324,12 +338,14 @@ template <int NW>
 __global__ __launch_bounds__(64 * NW) void align_place_kernel(
     const int32_t* __restrict__ ids, int P, int E, int e_off, int BM, int RW, const int32_t* __restrict__ whist,
     int32_t* __restrict__ sorted_ids, int32_t* __restrict__ block_expert, int32_t* __restrict__ gs,
-    int32_t* __restrict__ go, int32_t* __restrict__ gpo) {
+    int32_t* __restrict__ go, int32_t* __restrict__ gpo, ItemPlan plan) {
   extern __shared__ int sm[];
   int* hist = sm;                 // [NW][E]
   int* tot = sm + NW * E;         // [E]
   int* pstart = tot + E;          // [E+1]
   int* before = pstart + E + 1;   // [E] pairs of expert e in the workgroups before this one
+  int* ist = before + E;          // [E+1], with an item plan only
+  int* gof = ist + E + 1;         // [E+1]
   const int tid = threadIdx.x, w = tid >> 6;
   const int G = gridDim.x, g = blockIdx.x;
   // Every workgroup's count of expert e, loaded kBatch at a time before any is
@@ -357,7 +373,7 @@ __global__ __launch_bounds__(64 * NW) void align_place_kernel(
   int* hw = hist + w * E;
   align_count_range(ids, p0, p1, E, e_off, nbits, hw);
   __syncthreads();
-  if (w == 0) align_expert_scan(tot, E, BM, pstart, g == 0, gs, go, gpo);
+  if (w == 0) align_expert_scan(tot, E, BM, pstart, g == 0, gs, go, gpo, plan, ist, gof);
   __syncthreads();
   for (int e = tid; e < E; e += 64 * NW) {
     int run = pstart[e] + before[e];
@@ -374,44 +390,47 @@ __global__ __launch_bounds__(64 * NW) void align_place_kernel(
 
 hipError_t launch_align(const int32_t* ids, int P, int E, int BM, int32_t* sorted_ids,
                         int32_t* block_expert, int32_t* gs, int32_t* go, int32_t* gpo,
-                        int32_t* whist, hipStream_t s, int e_off) {
+                        int32_t* whist, hipStream_t s, int e_off, int32_t* istart, int hmax,
+                        int nt1, int nt2) {
+  const ItemPlan plan{istart, hmax, nt1, nt2};
+  const size_t lds_plan = istart ? 2 * sizeof(int) * ((size_t)E + 1) : 0;
   // 16 waves while the histograms fit 48 KiB of LDS, else 8 (E <= 1024)
   const bool w16 = 16 * E <= 12288;
   const int nw = w16 ? 16 : 8;
   const int per_wave = (P + nw - 1) / nw;  // pairs per wave in one workgroup
   if (per_wave <= 64 * kAlignUnroll) {  // one workgroup, each wave's pairs held in registers
-    const size_t lds = sizeof(int) * (nw * (size_t)E + 2 * (size_t)E + 1);
+    const size_t lds = sizeof(int) * (nw * (size_t)E + 2 * (size_t)E + 1) + lds_plan;
     if (w16)
       hipLaunchKernelGGL(align_small_kernel<16>, dim3(1), dim3(1024), lds, s, ids, P, E, e_off, BM, sorted_ids,
-                         block_expert, gs, go, gpo);
+                         block_expert, gs, go, gpo, plan);
     else
       hipLaunchKernelGGL(align_small_kernel<8>, dim3(1), dim3(512), lds, s, ids, P, E, e_off, BM, sorted_ids,
-                         block_expert, gs, go, gpo);
+                         block_expert, gs, go, gpo, plan);
     return hipGetLastError();
   }
   const int G = align_groups(P);
   if (whist && G > 1) {
     const int RW = align_pairs_per_group(P, G, nw);
     const size_t lds1 = sizeof(int) * ((size_t)nw * E);
-    const size_t lds2 = sizeof(int) * ((size_t)nw * E + 3 * (size_t)E + 1);
+    const size_t lds2 = sizeof(int) * ((size_t)nw * E + 3 * (size_t)E + 1) + lds_plan;
     if (w16) {
       hipLaunchKernelGGL(align_count_kernel<16>, dim3(G), dim3(1024), lds1, s, ids, P, E, e_off, RW, whist);
       hipLaunchKernelGGL(align_place_kernel<16>, dim3(G), dim3(1024), lds2, s, ids, P, E, e_off, BM, RW, whist,
-                         sorted_ids, block_expert, gs, go, gpo);
+                         sorted_ids, block_expert, gs, go, gpo, plan);
     } else {
       hipLaunchKernelGGL(align_count_kernel<8>, dim3(G), dim3(512), lds1, s, ids, P, E, e_off, RW, whist);
       hipLaunchKernelGGL(align_place_kernel<8>, dim3(G), dim3(512), lds2, s, ids, P, E, e_off, BM, RW, whist,
-                         sorted_ids, block_expert, gs, go, gpo);
+                         sorted_ids, block_expert, gs, go, gpo, plan);
     }
     return hipGetLastError();
   }
-  const size_t lds = sizeof(int) * (nw * (size_t)E + 2 * (size_t)E + 1);
+  const size_t lds = sizeof(int) * (nw * (size_t)E + 2 * (size_t)E + 1) + lds_plan;
   if (w16)
     hipLaunchKernelGGL(align_kernel<16>, dim3(1), dim3(1024), lds, s, ids, P, E, e_off, BM, sorted_ids,
-                       block_expert, gs, go, gpo);
+                       block_expert, gs, go, gpo, plan);
   else
     hipLaunchKernelGGL(align_kernel<8>, dim3(1), dim3(512), lds, s, ids, P, E, e_off, BM, sorted_ids,
-                       block_expert, gs, go, gpo);
+                       block_expert, gs, go, gpo, plan);
   return hipGetLastError();
 }
 
