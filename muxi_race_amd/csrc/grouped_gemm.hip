@@ -570,16 +570,28 @@ struct Ring {
   }
 };
 
-// Wave placement: TR / 64 waves along the tokens, each owning 64 rows (two
-// 32-row blocks), and the rest along the weight rows.
-template <int TR>
+// Wave placement: WM = TR / 64 waves along the tokens, each owning two 32-row
+// blocks, and the rest along the weight rows.  Waves w and w + 4 share a SIMD.
+// A wave owns blocks wm and wm + WM, so that an item of 192 rows gives every
+// SIMD three of them per weight column, where two neighbouring blocks per wave
+// gave two SIMDs four and two SIMDs two (64 experts, H 7168, I 2048: fp8 at 2048
+// tokens 731 -> 715 us, int8 at 1000 tokens 554 -> 542).  Items with absorbed
+// rows have all blocks full and keep neighbouring ones (measured 0.7% faster).
+template <class R>
 struct WaveGrid {
-  static constexpr int WM = TR / 64, WN = 8 / WM;
+  static constexpr int WM = R::TR / 64, WN = 8 / WM;
+  static constexpr int kStep = R::ABS ? 32 : 32 * WM;  // rows between a wave's two blocks
   int wm, wn;
   __device__ __forceinline__ WaveGrid() {
     const int wave = threadIdx.x >> 6;
     wm = wave / WN;
     wn = wave % WN;
+  }
+  __device__ __forceinline__ int x0() const { return (R::ABS ? 64 : 32) * wm; }  // first row of the first block
+  // this wave's blocks that hold one of the first n rows
+  __device__ __forceinline__ int live(int n) const {
+    const int rows = n - x0();
+    return rows <= 0 ? 0 : (rows <= kStep ? 1 : 2);
   }
 };
 
@@ -598,6 +610,7 @@ __device__ __forceinline__ void wide_k_loop(const R& ring, int nk, char* smem, i
   constexpr bool F8 = QT == kQF8;
   constexpr int DT = R::DT, DW = R::DW, SW = R::SW, NIW = R::NIW;
   constexpr bool kWork = NB > 0 || A;
+  constexpr int kBlock = WaveGrid<R>::kStep * kRowBytes;  // LDS bytes between the wave's token blocks
   constexpr int kHalf = NWB > 1 ? NWB / 2 : 1;
   ScaleBytes<SCB> sc[2];
 #pragma unroll
@@ -632,7 +645,7 @@ __device__ __forceinline__ void wide_k_loop(const R& ring, int nk, char* smem, i
       const uint32_t xab = A ? row_base(ts, R::TR) : 0, wab = A ? row_base(wsl, wa) : 0;
       auto load_frags = [&](int buf, int s) {
 #pragma unroll
-        for (int b = 0; b < NB; ++b) xf[buf][b] = frag_at(xb + 4096 * b, fl.off[s]);
+        for (int b = 0; b < NB; ++b) xf[buf][b] = frag_at(xb + kBlock * b, fl.off[s]);
         if constexpr (NB > 0) {
 #pragma unroll
           for (int j = 0; j < NWB; ++j)
@@ -657,7 +670,7 @@ __device__ __forceinline__ void wide_k_loop(const R& ring, int nk, char* smem, i
 #pragma unroll
           for (int q = 0; q < 2; ++q)
 #pragma unroll
-            for (int b = 0; b < NB; ++b) xf[q][b] = frag_at(xb + 4096 * b, fl.off[2 * h + q]);
+            for (int b = 0; b < NB; ++b) xf[q][b] = frag_at(xb + kBlock * b, fl.off[2 * h + q]);
           if (kSpreadT && pt) ring.issue_t(td, ks + DT, h * R::NIT / 2, (h + 1) * R::NIT / 2);
           if (kSpread && pw) ring.template issue_w<STREAM>(wd, ks + DW, h * NIW / 2, (h + 1) * NIW / 2);
 #pragma unroll
@@ -704,7 +717,7 @@ template <int QT, bool GATHER, int TR, bool ABS, bool STREAM>
 __device__ __forceinline__ void stage1_item(const Stage1Params& p, const Item& it, char* smem) {
   constexpr bool I8 = QT != kQF16, F8 = QT == kQF8;  // 8-bit operands with row scales
   using R = Ring<TR, 2 * kBN, ABS>;
-  using G = WaveGrid<TR>;
+  using G = WaveGrid<R>;
   using Acc = typename std::conditional<I8 && !F8, i32x16, f32x16>::type;
   constexpr int WTN = kBN / G::WN;  // gate (and up) features per wave
   constexpr int NBN = WTN / 32;     // gate (and up) blocks per wave
@@ -741,8 +754,7 @@ __device__ __forceinline__ void stage1_item(const Stage1Params& p, const Item& i
   }
 
   const G g;
-  const int live = (actual - 64 * g.wm + 31) / 32;
-  const int xr0 = 64 * g.wm;            // slot row of this wave's first token row
+  const int xr0 = g.x0();               // slot row of this wave's first token row
   const int gr0 = WTN * g.wn;           // ... first gate row; up rows follow the kBN gate rows
   const FragLane fl;
   const int l = lane_id();
@@ -761,7 +773,7 @@ __device__ __forceinline__ void stage1_item(const Stage1Params& p, const Item& i
     int pid[2];
 #pragma unroll
     for (int b = 0; b < 2; ++b) {
-      const int m = xr0 + 32 * b + (l & 31);
+      const int m = xr0 + G::kStep * b + (l & 31);
       pid[b] = p.sorted_ids[row0 + (m < actual ? m : 0)];
     }
 #pragma unroll
@@ -790,7 +802,7 @@ __device__ __forceinline__ void stage1_item(const Stage1Params& p, const Item& i
   const int aj = g.wm & 1;
   const int awr0 = (agate ? gr0 : kBN + gr0) + 32 * aj;
   const uint8_t* const no_scale[2] = {nullptr, nullptr};
-  with_live<2>(live < 0 ? 0 : live, [&](auto nb_c) {
+  with_live<2>(g.live(actual), [&](auto nb_c) {
     wide_k_loop<QT, false, R, STREAM, 2 * NBN, decltype(nb_c)::value, ABS>(ring, nk, smem, xr0, gr0, kBN + gr0, awr0, fl,
                                                                           acc, aa, no_scale);
   });
@@ -803,7 +815,7 @@ __device__ __forceinline__ void stage1_item(const Stage1Params& p, const Item& i
     // Stage 2 accumulates in int32 over the whole of K.
 #pragma unroll
     for (int b = 0; b < 2; ++b) {
-      const int m = xr0 + 32 * b + (l & 31);
+      const int m = xr0 + G::kStep * b + (l & 31);
       if (m < actual) {
         _Float16* hrow = reinterpret_cast<_Float16*>(p.h) + (int64_t)(row0 + m) * p.h_ld;
 #pragma unroll
@@ -867,7 +879,7 @@ __device__ __forceinline__ void stage1_item(const Stage1Params& p, const Item& i
     float hv[2][NBN][16];
 #pragma unroll
     for (int b = 0; b < 2; ++b) {
-      const int m = xr0 + 32 * b + (l & 31);
+      const int m = xr0 + G::kStep * b + (l & 31);
       const float sx = m < actual ? sxv[b] : 0.0f;
       float amax = 0.0f;
 #pragma unroll
@@ -893,12 +905,12 @@ __device__ __forceinline__ void stage1_item(const Stage1Params& p, const Item& i
           }
         }
       amax = fmaxf(amax, __shfl_xor(amax, 32));
-      if (l < 32) red[g.wn * TR + xr0 + 32 * b + l] = amax;
+      if (l < 32) red[g.wn * TR + xr0 + G::kStep * b + l] = amax;
     }
     __syncthreads();
 #pragma unroll
     for (int b = 0; b < 2; ++b) {
-      const int m = xr0 + 32 * b + (l & 31);
+      const int m = xr0 + G::kStep * b + (l & 31);
       float amax = 0.0f;
 #pragma unroll
       for (int j = 0; j < G::WN; ++j) amax = fmaxf(amax, red[j * TR + m]);
@@ -948,7 +960,7 @@ template <int QT, bool FUSED, int BN, int TR, bool ABS, bool STREAM>
 __device__ __forceinline__ void stage2_item(const Stage2Params& p, const Item& it, char* smem) {
   constexpr bool I8 = QT == kQI8, F8 = QT == kQF8;
   using R = Ring<TR, BN, ABS>;
-  using G = WaveGrid<TR>;
+  using G = WaveGrid<R>;
   // int8: exact int32 accumulation over the whole of K (the intermediate has
   // one scale per row, applied in the epilogue); fp16 / fp8: fp32
   using Acc = typename std::conditional<I8, i32x16, f32x16>::type;
@@ -984,8 +996,7 @@ __device__ __forceinline__ void stage2_item(const Stage2Params& p, const Item& i
 
   const G g;
   const int l = lane_id();
-  const int live = (actual - 64 * g.wm + 31) / 32;  // see Stage 1
-  const int xr0 = 64 * g.wm;   // slot row of this wave's first token row
+  const int xr0 = g.x0();      // slot row of this wave's first token row
   const int wr0 = WTN * g.wn;  // ... of its first weight row
   const FragLane fl;
 
@@ -1017,7 +1028,7 @@ __device__ __forceinline__ void stage2_item(const Stage2Params& p, const Item& i
   const uint8_t* sp[2] = {nullptr, nullptr};
 #pragma unroll
   for (int b = 0; b < 2; ++b) {
-    const int m = xr0 + 32 * b + (l & 31);
+    const int m = xr0 + G::kStep * b + (l & 31);
     const int mc = m < actual ? m : 0;
     wr[b] = weight_of(m, m < actual);
     if constexpr (I8) shv[b] = p.a_scale[row0 + mc];
@@ -1046,13 +1057,13 @@ __device__ __forceinline__ void stage2_item(const Stage2Params& p, const Item& i
     if (awave) loop(std::integral_constant<int, 2>{}, std::true_type{});
     else loop(std::integral_constant<int, 2>{}, std::false_type{});
   } else {
-    with_live<2>(live < 0 ? 0 : live, [&](auto nb_c) { loop(nb_c, std::false_type{}); });
+    with_live<2>(g.live(actual), [&](auto nb_c) { loop(nb_c, std::false_type{}); });
   }
 
   __syncthreads();  // every wave is done with the ring
 #pragma unroll
   for (int b = 0; b < 2; ++b) {
-    const int m = xr0 + 32 * b + (l & 31);
+    const int m = xr0 + G::kStep * b + (l & 31);
     if (m >= actual) continue;
 #pragma unroll
     for (int a = 0; a < NWB; ++a)

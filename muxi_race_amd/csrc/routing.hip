@@ -118,19 +118,21 @@ __device__ __forceinline__ void align_place_range(const int32_t* __restrict__ id
   }
 }
 
-// The wide items' plan: see launch_align.
+// The wide items' plan: see launch_align.  A workgroup of its own, the launch's
+// last, counts and scans as the others do and writes it (3 us of one wave's
+// work, which would otherwise end the launch).
 struct ItemPlan {
   int32_t* istart;
   int hmax, nt1, nt2;
 };
 
 // Expert scan by one wave: tot[E] -> padded offsets pstart[E+1] in LDS, and
-// (when `out`) group sizes / offsets / padded offsets, and the wide items' plan
-// when one is asked for, in global memory.  ist, gof: [E+1] ints of LDS each.
+// (when `out`) group sizes / offsets / padded offsets, and (when `plan`) the wide
+// items' plan, in global memory.  ist, gof: [E+1] ints of LDS each.
 __device__ __forceinline__ void align_expert_scan(const int* tot, int E, int BM, int* pstart, bool out,
                                                   int32_t* __restrict__ gs, int32_t* __restrict__ go,
-                                                  int32_t* __restrict__ gpo, const ItemPlan& plan, int* ist,
-                                                  int* gof) {
+                                                  int32_t* __restrict__ gpo, const ItemPlan* plan = nullptr,
+                                                  int* ist = nullptr, int* gof = nullptr) {
   const int l = lane_id();
   int carry = 0, carry_p = 0, carry_i = 0;
   for (int base = 0; base < E; base += 64) {
@@ -146,10 +148,10 @@ __device__ __forceinline__ void align_expert_scan(const int* tot, int E, int BM,
         gpo[e] = carry_p + ip - pc;
       }
     }
-    if (out && plan.istart) {  // uniform
-      const int ni = items_of(c, plan.hmax), ii = wave_inclusive_scan(ni);
+    if (plan) {
+      const int ni = items_of(c, plan->hmax), ii = wave_inclusive_scan(ni);
       if (e < E) {
-        plan.istart[e] = ist[e] = carry_i + ii - ni;
+        plan->istart[e] = ist[e] = carry_i + ii - ni;
         gof[e] = carry + ic - c;
       }
       carry_i += __builtin_amdgcn_readlane(ii, 63);
@@ -164,14 +166,14 @@ __device__ __forceinline__ void align_expert_scan(const int* tot, int E, int BM,
       gpo[E] = carry_p;
     }
   }
-  if (out && plan.istart) {
+  if (plan) {
     if (l == 0) {
-      plan.istart[E] = ist[E] = carry_i;
+      plan->istart[E] = ist[E] = carry_i;
       gof[E] = carry;
     }
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");  // this wave's LDS writes, before other lanes read them
-    xcd_shares(ist, gof, E, plan.nt1, plan.istart + E + 1);
-    xcd_shares(ist, gof, E, plan.nt2, plan.istart + E + 10);
+    xcd_shares(ist, gof, E, plan->nt1, plan->istart + E + 1);
+    xcd_shares(ist, gof, E, plan->nt2, plan->istart + E + 10);
   }
 }
 
@@ -254,7 +256,12 @@ __global__ __launch_bounds__(64 * NW) void align_small_kernel(
     tot[e] = run;
   }
   __syncthreads();
-  if (w == 0) align_expert_scan(tot, E, BM, pstart, true, gs, go, gpo, plan, ist, gof);
+  const bool planner = blockIdx.x > 0;
+  if (w == 0) {
+    if (planner) align_expert_scan(tot, E, BM, pstart, false, gs, go, gpo, &plan, ist, gof);
+    else align_expert_scan(tot, E, BM, pstart, true, gs, go, gpo);
+  }
+  if (planner) return;
   __syncthreads();
   const int rows = pstart[E];
   for (int r = tid; r < rows; r += 64 * NW) sorted_ids[r] = P;
@@ -302,7 +309,12 @@ __global__ __launch_bounds__(64 * NW) void align_kernel(
     tot[e] = run;
   }
   __syncthreads();
-  if (w == 0) align_expert_scan(tot, E, BM, pstart, true, gs, go, gpo, plan, ist, gof);
+  const bool planner = blockIdx.x > 0;
+  if (w == 0) {
+    if (planner) align_expert_scan(tot, E, BM, pstart, false, gs, go, gpo, &plan, ist, gof);
+    else align_expert_scan(tot, E, BM, pstart, true, gs, go, gpo);
+  }
+  if (planner) return;
   __syncthreads();
   for (int e = tid; e < E; e += 64 * NW)
     for (int v = 0; v < NW; ++v) hist[v * E + e] += pstart[e];
@@ -347,7 +359,7 @@ __global__ __launch_bounds__(64 * NW) void align_place_kernel(
   int* ist = before + E;          // [E+1], with an item plan only
   int* gof = ist + E + 1;         // [E+1]
   const int tid = threadIdx.x, w = tid >> 6;
-  const int G = gridDim.x, g = blockIdx.x;
+  const int G = gridDim.x - (plan.istart ? 1 : 0), g = blockIdx.x;  // g == G: the plan's workgroup
   // Every workgroup's count of expert e, loaded kBatch at a time before any is
   // added, so one load latency is exposed per batch rather than per workgroup.
   constexpr int kBatch = 16;
@@ -373,7 +385,11 @@ __global__ __launch_bounds__(64 * NW) void align_place_kernel(
   int* hw = hist + w * E;
   align_count_range(ids, p0, p1, E, e_off, nbits, hw);
   __syncthreads();
-  if (w == 0) align_expert_scan(tot, E, BM, pstart, g == 0, gs, go, gpo, plan, ist, gof);
+  if (w == 0) {
+    if (g == G) align_expert_scan(tot, E, BM, pstart, false, gs, go, gpo, &plan, ist, gof);
+    else align_expert_scan(tot, E, BM, pstart, g == 0, gs, go, gpo);
+  }
+  if (g == G) return;
   __syncthreads();
   for (int e = tid; e < E; e += 64 * NW) {
     int run = pstart[e] + before[e];
@@ -393,6 +409,7 @@ hipError_t launch_align(const int32_t* ids, int P, int E, int BM, int32_t* sorte
                         int32_t* whist, hipStream_t s, int e_off, int32_t* istart, int hmax,
                         int nt1, int nt2) {
   const ItemPlan plan{istart, hmax, nt1, nt2};
+  const unsigned extra = istart ? 1 : 0;  // the plan's workgroup
   const size_t lds_plan = istart ? 2 * sizeof(int) * ((size_t)E + 1) : 0;
   // 16 waves while the histograms fit 48 KiB of LDS, else 8 (E <= 1024)
   const bool w16 = 16 * E <= 12288;
@@ -401,10 +418,10 @@ hipError_t launch_align(const int32_t* ids, int P, int E, int BM, int32_t* sorte
   if (per_wave <= 64 * kAlignUnroll) {  // one workgroup, each wave's pairs held in registers
     const size_t lds = sizeof(int) * (nw * (size_t)E + 2 * (size_t)E + 1) + lds_plan;
     if (w16)
-      hipLaunchKernelGGL(align_small_kernel<16>, dim3(1), dim3(1024), lds, s, ids, P, E, e_off, BM, sorted_ids,
+      hipLaunchKernelGGL(align_small_kernel<16>, dim3(1 + extra), dim3(1024), lds, s, ids, P, E, e_off, BM, sorted_ids,
                          block_expert, gs, go, gpo, plan);
     else
-      hipLaunchKernelGGL(align_small_kernel<8>, dim3(1), dim3(512), lds, s, ids, P, E, e_off, BM, sorted_ids,
+      hipLaunchKernelGGL(align_small_kernel<8>, dim3(1 + extra), dim3(512), lds, s, ids, P, E, e_off, BM, sorted_ids,
                          block_expert, gs, go, gpo, plan);
     return hipGetLastError();
   }
@@ -415,21 +432,21 @@ hipError_t launch_align(const int32_t* ids, int P, int E, int BM, int32_t* sorte
     const size_t lds2 = sizeof(int) * ((size_t)nw * E + 3 * (size_t)E + 1) + lds_plan;
     if (w16) {
       hipLaunchKernelGGL(align_count_kernel<16>, dim3(G), dim3(1024), lds1, s, ids, P, E, e_off, RW, whist);
-      hipLaunchKernelGGL(align_place_kernel<16>, dim3(G), dim3(1024), lds2, s, ids, P, E, e_off, BM, RW, whist,
+      hipLaunchKernelGGL(align_place_kernel<16>, dim3(G + extra), dim3(1024), lds2, s, ids, P, E, e_off, BM, RW, whist,
                          sorted_ids, block_expert, gs, go, gpo, plan);
     } else {
       hipLaunchKernelGGL(align_count_kernel<8>, dim3(G), dim3(512), lds1, s, ids, P, E, e_off, RW, whist);
-      hipLaunchKernelGGL(align_place_kernel<8>, dim3(G), dim3(512), lds2, s, ids, P, E, e_off, BM, RW, whist,
+      hipLaunchKernelGGL(align_place_kernel<8>, dim3(G + extra), dim3(512), lds2, s, ids, P, E, e_off, BM, RW, whist,
                          sorted_ids, block_expert, gs, go, gpo, plan);
     }
     return hipGetLastError();
   }
   const size_t lds = sizeof(int) * (nw * (size_t)E + 2 * (size_t)E + 1) + lds_plan;
   if (w16)
-    hipLaunchKernelGGL(align_kernel<16>, dim3(1), dim3(1024), lds, s, ids, P, E, e_off, BM, sorted_ids,
+    hipLaunchKernelGGL(align_kernel<16>, dim3(1 + extra), dim3(1024), lds, s, ids, P, E, e_off, BM, sorted_ids,
                        block_expert, gs, go, gpo, plan);
   else
-    hipLaunchKernelGGL(align_kernel<8>, dim3(1), dim3(512), lds, s, ids, P, E, e_off, BM, sorted_ids,
+    hipLaunchKernelGGL(align_kernel<8>, dim3(1 + extra), dim3(512), lds, s, ids, P, E, e_off, BM, sorted_ids,
                        block_expert, gs, go, gpo, plan);
   return hipGetLastError();
 }
