@@ -1,0 +1,160 @@
+"""GPU parity of the wide items (more than 32 rows per expert): every item of a
+launch runs exactly once however the routing is skewed, at the row counts where
+an expert's split or its tile changes, over both cuts of the items over the
+XCDs, for every format; run_kernel's item count over more than 512 blocks; and
+the one-launch routing and alignment of small batches against the two
+launches."""
+import pytest
+import torch
+
+from _cases import prerouted_inputs
+from conftest import assert_close
+from oracle import fused_moe_forward, prerouted_forward, w8a8_forward
+
+pytestmark = pytest.mark.gpu
+
+# Rows per expert around every change of the split and of the tile (up to 32 /
+# 128 / 256 / 288 rows per item; two and three pieces), for 20 experts
+EDGES = [1, 31, 32, 33, 64, 65, 127, 128, 129, 160, 161, 192, 255, 256, 257, 288, 289, 576, 577, 0]
+
+
+def _logits(sizes, k):
+    """Router logits whose top-k gives expert e exactly sizes[e] rows, top-1,
+    and (k > 1) spreads the further choices round-robin over the experts."""
+    E, T = len(sizes), sum(sizes)
+    first = torch.repeat_interleave(torch.arange(E), torch.tensor(sizes))
+    first = first[torch.randperm(T, generator=torch.Generator().manual_seed(T))]
+    lg = torch.zeros(T, E)
+    t = torch.arange(T)
+    lg[t, first] = 4.0
+    for j in range(1, k):
+        lg[t, (first + 1 + (t + j) % (E - 1)) % E] += 2.0 - 0.1 * j
+    return lg
+
+
+def _case(sizes, H, I, k, seed):
+    g = torch.Generator().manual_seed(seed)
+    T, E = sum(sizes), len(sizes)
+    mk = lambda *sh: (torch.randn(sh, generator=g) * 0.05).half()
+    return torch.randn(T, H, generator=g).half(), _logits(sizes, k), mk(E, I, H), mk(E, I, H), mk(E, H, I)
+
+
+def _close_8bit(out, ref, x, lg, wg, wu, wd, what):
+    """Against the 8-bit oracle, which sums in another order: a code of the
+    intermediate at a rounding tie may fall the other way.  One flip changes an
+    output by at most one code step of that h (amax_h / 8 for e4m3, less for
+    int8) times a down weight, and flips are rare: the relative L2 stays far
+    below the quantisation's own 2.5e-2 / 4.6e-2."""
+    got, ref = out.float().cpu(), ref.float()
+    assert bool(torch.isfinite(got).all()), what
+    e = lg.argmax(1)
+    hmax = max(float((torch.nn.functional.silu(x[e == j].float() @ wg[j].float().T) * (x[e == j].float() @ wu[j].float().T)).abs().max())
+               for j in range(wg.shape[0]) if bool((e == j).any()))
+    d = (got - ref).abs()
+    bound = hmax / 8 * float(wd.float().abs().max()) + 1e-2
+    rel = float(d.norm() / ref.norm())
+    print(f"{what}: max|d| {float(d.max()):.4f} (bound {bound:.4f}), rel L2 {rel:.5f}")
+    assert float(d.max()) <= bound and rel < 5e-3, what
+
+
+@pytest.mark.parametrize("H,I,bm", [(256, 128, 64), (384, 256, 128), (512, 2048, 0)])
+def test_rows_at_every_edge_fp16(H, I, bm):
+    """H 384 is no multiple of 256 (Stage 2 on 128-wide tiles); I 2048 has 16
+    Stage 1 tiles, enough for full-height items, the others take short ones."""
+    from muxi_race_amd import fused_moe
+    x, lg, wg, wu, wd = _case(EDGES, H, I, 1, 5)
+    out = torch.full((x.shape[0], H), float("nan"), dtype=torch.float16, device="cuda")
+    out = fused_moe(x.cuda(), lg.cuda(), wg.cuda(), wu.cuda(), wd.cuda(), 1, block_m=bm, out=out)
+    torch.cuda.synchronize()
+    assert_close(out, fused_moe_forward(x, lg, wg, wu, wd, 1), what=f"edge rows H={H} I={I} bm={bm}")
+
+
+@pytest.mark.parametrize("fmt", ["int8", "fp8"])
+@pytest.mark.parametrize("H,I", [(256, 2048), (384, 256)])
+def test_rows_at_every_edge_8bit(fmt, H, I):
+    """I 2048: 16 scale bytes per fp8 intermediate row, one register load."""
+    from muxi_race_amd import fused_moe, quantize_w8a8_weights
+    x, lg, wg, wu, wd = _case(EDGES, H, I, 1, 6)
+    qw = quantize_w8a8_weights(wg.cuda(), wu.cuda(), wd.cuda(), fmt=fmt)
+    out = torch.full((x.shape[0], H), float("nan"), dtype=torch.float16, device="cuda")
+    out = fused_moe(x.cuda(), lg.cuda(), None, None, None, 1, w8a8=qw, block_m=64, out=out)
+    torch.cuda.synchronize()
+    codes = lambda t: (t.view(torch.uint8) if fmt == "fp8" else t).cpu().numpy()
+    ref = w8a8_forward(x, lg, codes(qw.q_gate), qw.s_gate.cpu().numpy(), codes(qw.q_up), qw.s_up.cpu().numpy(),
+                       codes(qw.q_down), qw.s_down.cpu().numpy(), 1, fmt=fmt)
+    _close_8bit(out, ref, x, lg, wg, wu, wd, f"{fmt} edge rows H={H} I={I}")
+
+
+@pytest.mark.parametrize("bm", [32, 64])
+def test_fp8_scale_bytes_reload(bm):
+    """I 2304: 18 scale bytes per row, loaded 16 K steps at a time (narrow and
+    wide items)."""
+    from muxi_race_amd import fused_moe, quantize_w8a8_weights
+    x, lg, wg, wu, wd = _case([40, 3, 150, 7], 128, 2304, 2, 7)
+    qw = quantize_w8a8_weights(wg.cuda(), wu.cuda(), wd.cuda(), fmt="fp8")
+    out = fused_moe(x.cuda(), lg.cuda(), None, None, None, 2, w8a8=qw, block_m=bm)
+    codes = lambda t: t.view(torch.uint8).cpu().numpy()
+    ref = w8a8_forward(x, lg, codes(qw.q_gate), qw.s_gate.cpu().numpy(), codes(qw.q_up), qw.s_up.cpu().numpy(),
+                       codes(qw.q_down), qw.s_down.cpu().numpy(), 2, fmt="fp8")
+    _close_8bit(out, ref, x, lg, wg, wu, wd, f"fp8 I=2304 bm={bm}")
+
+
+@pytest.mark.parametrize("skew", ["first", "last", "even"])
+def test_xcd_shares_cover_every_item(skew):
+    """70 experts, 16 Stage 1 tiles: a few experts of hundreds of rows at one
+    end (the items are cut over the XCDs by cost) or like ones (cut into equal
+    numbers)."""
+    from muxi_race_amd import fused_moe
+    sizes = [40 + e % 7 for e in range(70)]
+    if skew != "even":
+        heavy = [700, 410, 300, 277, 259]
+        sizes = heavy + sizes[5:] if skew == "first" else sizes[5:] + heavy
+    H, I = 256, 2048
+    g = torch.Generator(device="cuda").manual_seed(3)
+    T, E = sum(sizes), 70
+    x = torch.randn(T, H, generator=g, device="cuda").half()
+    w = [(torch.randn(sh, generator=g, device="cuda") * 0.05).half() for sh in ((E, I, H), (E, I, H), (E, H, I))]
+    lg = _logits(sizes, 2)
+    out = torch.full((T, H), float("nan"), dtype=torch.float16, device="cuda")
+    out = fused_moe(x, lg.cuda(), *w, 2, block_m=64, out=out)
+    torch.cuda.synchronize()
+    assert_close(out, fused_moe_forward(x.cpu(), lg, *(m.cpu() for m in w), 2), what=f"XCD shares {skew}")
+
+
+def test_run_kernel_over_512_blocks():
+    """650 experts (more than 512 blocks: two passes of the item count), with
+    empty, single-block and multi-block experts."""
+    g = torch.Generator().manual_seed(11)
+    sizes = [int(v) for v in torch.randint(0, 140, (650,), generator=g)]
+    sizes[3], sizes[200], sizes[649] = 600, 0, 290
+    args = prerouted_inputs(sizes, 128, 128, seed=12)
+    from muxi_race_amd import run_kernel
+    out = torch.full(args[0].shape, float("nan"), dtype=torch.float16, device="cuda")
+    run_kernel(*args, out)
+    torch.cuda.synchronize()
+    assert_close(out, prerouted_forward(*args), what="650 experts")
+
+
+@pytest.mark.parametrize("E,k,T", [(1, 1, 1), (8, 2, 1), (8, 8, 256), (8, 2, 257), (5, 3, 77), (16, 4, 200), (9, 2, 256),
+                                   (17, 2, 16)])
+@pytest.mark.parametrize("bias", [False, True])
+def test_small_batches_route_and_align_in_one_launch(E, k, T, bias):
+    """At most 16 experts and 256 tokens: the same ids, weights (bits) and
+    output as route_topk and the routed entry, with ties and infinities."""
+    from muxi_race_amd import fused_moe, fused_moe_routed, route_topk
+    g = torch.Generator(device="cuda").manual_seed(T)
+    mk = lambda *sh: torch.randn(sh, generator=g, device="cuda")
+    lg = mk(T, E)
+    lg[0] = 1.0  # all tied
+    if T > 2 and k < E:
+        lg[1], lg[2, E - 1] = -float("inf"), float("inf")
+        lg[1, :k] = 0.5
+    b = mk(E) if bias else None
+    x = mk(T, 128).half()
+    w = [(mk(*sh) * 0.05).half() for sh in ((E, 128, 128), (E, 128, 128), (E, 128, 128))]
+    rid, rw = route_topk(lg, k, b)
+    out, (ids, wts) = fused_moe(x, lg, *w, k, expert_bias=b, return_routing=True)
+    want = fused_moe_routed(x, rid, rw, *w)
+    torch.cuda.synchronize()
+    assert torch.equal(ids, rid) and torch.equal(wts.view(torch.int32), rw.view(torch.int32))
+    assert torch.equal(torch.nan_to_num(out), torch.nan_to_num(want))
