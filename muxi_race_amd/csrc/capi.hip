@@ -394,7 +394,17 @@ static int fused_common(int qt, const void* x, const float* logits, const void* 
   // 8-bit operands from logits: the routing and the per-token quantisation of
   // x run as one launch (route_quant_kernel)
   const bool route_quant = w8 && !given && !w_router;
-  if (given) {
+  const int nt1 = (int)(I / moe::kBN), nt2 = (int)wide.nt2;
+  int32_t* const plan = narrow ? nullptr : istart;
+  // small batches from logits: routing and alignment run as one launch
+  hipError_t ra = hipSuccess;
+  const bool route_align =
+      !w8 && !given && !w_router &&
+      moe::launch_route_align(logits, bias, (int)T, (int)E_route, (int)k, ids, wts, e_shared, (int)Ee, (int)block_m, sorted,
+                              (int32_t*)(ws + L.bexp), gs, go, gpo, s, (int)e_begin, plan, wide.hmax, nt1, nt2, &ra);
+  if (route_align) {
+    if ((rc = check_launch(ra, "route_align"))) return rc;
+  } else if (given) {
     // routed by the caller: nothing to launch (ids and weights are only read)
   } else if (route_quant) {
     if ((rc = check_launch(moe::launch_route_quant(logits, bias, (int)T, (int)E_route, (int)k, ids, wts, x, H,
@@ -406,7 +416,8 @@ static int fused_common(int qt, const void* x, const float* logits, const void* 
     return rc;
   }
   mark(1);
-  if ((rc = check_launch(moe::launch_align(rids, (int)(T * ke), (int)Ee, (int)block_m, sorted, (int32_t*)(ws + L.bexp), gs, go, gpo, (int32_t*)(ws + L.whist), s, (int)e_begin, narrow ? nullptr : istart, wide.hmax, (int)(I / moe::kBN), (int)wide.nt2), "align"))) return rc;
+  if (!route_align &&
+      (rc = check_launch(moe::launch_align(rids, (int)(T * ke), (int)Ee, (int)block_m, sorted, (int32_t*)(ws + L.bexp), gs, go, gpo, (int32_t*)(ws + L.whist), s, (int)e_begin, plan, wide.hmax, nt1, nt2), "align"))) return rc;
   mark(2);
   if (w8 && !route_quant && (rc = check_launch(moe::launch_quant_rows(x, T, H, ws + L.xq, (float*)(ws + L.sx), qt, s), "quantize_x"))) return rc;
   mark(3);

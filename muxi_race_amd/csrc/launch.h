@@ -135,6 +135,12 @@ hipError_t launch_align(const int32_t* ids, int P, int E, int BM, int32_t* sorte
                         int32_t* block_expert, int32_t* gs, int32_t* go, int32_t* gpo,
                         int32_t* whist, hipStream_t stream, int e_off = 0, int32_t* istart = nullptr,
                         int hmax = 1, int nt1 = 0, int nt2 = 0);
+// launch_route_topk and launch_align in one launch, for small batches (see
+// route_align_kernel); false, with nothing launched, for others.
+bool launch_route_align(const float* logits, const float* bias, int T, int E_route, int k, int32_t* ids, float* w,
+                        int e_shared, int E, int BM, int32_t* sorted_ids, int32_t* block_expert, int32_t* gs,
+                        int32_t* go, int32_t* gpo, hipStream_t stream, int e_off, int32_t* istart, int hmax, int nt1,
+                        int nt2, hipError_t* err);
 // Router GEMM (x . w_router^T, K split in router_splits parts) + routing of
 // the summed partials; `part` holds router_partial_floats fp32, `logits`
 // (fp32 [T, E]) may be null.

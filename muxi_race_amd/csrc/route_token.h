@@ -164,4 +164,63 @@ __device__ __forceinline__ void route_token_row(const float* __restrict__ row, c
   route_token_values<VPL>(v, valid, t, k, ids, wout, kout == 0 ? k : kout, e_shared);
 }
 
+// Routes token t by one lane, for E <= EL experts (EL 8 or 16): the choices of
+// route_token_values (k rounds of the largest key, ties to the lower expert)
+// and its softmax sum in the same order (wave_sum's tree, whose lanes past E add
+// 0), so the same bits.  Loads are unconditional at clamped experts.
+template <int EL>
+__device__ __forceinline__ void route_token_lane(const float* __restrict__ row, const float* __restrict__ bias, int t,
+                                                 int E, int k, int32_t* __restrict__ ids, float* __restrict__ wout,
+                                                 int kout, int e_shared) {
+  const float* bsrc = bias ? bias : row;
+  float v[EL], bv[EL];
+#pragma unroll
+  for (int j = 0; j < EL; ++j) {
+    v[j] = row[j < E ? j : E - 1];
+    bv[j] = bsrc[j < E ? j : E - 1];
+  }
+  uint32_t key[EL];
+  float m = 0.0f;
+#pragma unroll
+  for (int j = 0; j < EL; ++j) {
+    v[j] = bias ? v[j] + bv[j] : v[j];
+    key[j] = j < E ? order_key(v[j]) : 0u;
+  }
+  uint32_t top = 0;
+#pragma unroll
+  for (int j = 0; j < EL; ++j) top = key[j] > top ? key[j] : top;
+  m = key_value(top);
+  float e[EL];
+#pragma unroll
+  for (int j = 0; j < EL; ++j) e[j] = j < E ? expf(v[j] - m) : 0.0f;
+#pragma unroll
+  for (int o = EL / 2; o >= 1; o >>= 1)
+#pragma unroll
+    for (int j = 0; j < o; ++j) e[j] += e[j + o];
+  const float s = e[0];
+  float denom = 0.0f;
+  for (int c = 0; c < k; ++c) {
+    uint32_t best = 0;
+    int at = 0;
+#pragma unroll
+    for (int j = 0; j < EL; ++j) {
+      if (key[j] > best) {
+        best = key[j];
+        at = j;
+      }
+    }
+    const float pr = expf(key_value(best) - m) / s;
+    denom = denom + pr;
+    ids[(int64_t)t * kout + c] = at;
+    wout[(int64_t)t * kout + c] = pr;
+#pragma unroll
+    for (int j = 0; j < EL; ++j) key[j] = j == at ? 0u : key[j];
+  }
+  for (int c = 0; c < k; ++c) wout[(int64_t)t * kout + c] = wout[(int64_t)t * kout + c] / denom;
+  if (e_shared >= 0) {
+    ids[(int64_t)t * kout + k] = e_shared;
+    wout[(int64_t)t * kout + k] = 1.0f;
+  }
+}
+
 }  // namespace moe
