@@ -196,7 +196,7 @@ int moe_run_prerouted_events(const void* x, const void* w_gate, const void* w_up
   // optional stage markers: ev[0] start, [1] stage 1, [2] stage 2
   auto mark = [&](int i) { if (stage_events && stage_events[i]) (void)hipEventRecord((hipEvent_t)stage_events[i], s); };
   mark(0);
-  int rc = check_launch(moe::launch_stage1(p1, false, moe::kQF16, false, blocks, 0, s), "stage1");
+  int rc = check_launch(moe::launch_stage1(p1, false, moe::kQF16, false, blocks, 128 * blocks, s), "stage1");
   if (rc) return rc;
   mark(1);
 
@@ -215,7 +215,7 @@ int moe_run_prerouted_events(const void* x, const void* w_gate, const void* w_up
   p2.I = I;
   p2.V = V;
   p2.hmax = wide.hmax;
-  rc = check_launch(moe::launch_stage2(p2, false, moe::kQF16, false, wide.bn256, blocks, 0, s), "stage2");
+  rc = check_launch(moe::launch_stage2(p2, false, moe::kQF16, false, wide.bn256, blocks, 128 * blocks, s), "stage2");
   mark(2);
   return rc;
 }

@@ -939,19 +939,24 @@ template <int QT, bool GATHER>
 __global__ __launch_bounds__(512) void stage1_wide_kernel(Stage1Params p) {
   __shared__ __attribute__((aligned(16))) char smem[kLdsBytes];
   const int nt = (int)(p.I / kBN);
+  auto run = [&](const Item& it) {
+    if (it.actual <= 0) return;  // no token: Stage 2 writes the rows as 0
+    if (it.actual <= kLowRows) {
+      if (it.shared) stage1_item<QT, GATHER, kLowRows, false, false>(p, it, smem);
+      else stage1_item<QT, GATHER, kLowRows, false, true>(p, it, smem);
+    } else if (QT != kQF16 || it.actual <= kWideRows) {
+      if (it.shared) stage1_item<QT, GATHER, kWideRows, false, false>(p, it, smem);
+      else stage1_item<QT, GATHER, kWideRows, false, true>(p, it, smem);
+    } else if constexpr (QT == kQF16) {
+      if (it.shared) stage1_item<QT, GATHER, kWideRows, true, false>(p, it, smem);
+      else stage1_item<QT, GATHER, kWideRows, true, true>(p, it, smem);
+    }
+  };
   Item it;
-  if (GATHER ? !item_fused(blockIdx.x, p.istart, p.xb, p.gs, p.gpo, p.E, kBN, nt, p.rows_cap, it)
-             : !item_bx(blockIdx.x, p.gidx, p.host_blocks, p.E, kBN, nt, p.gs, p.gpo, p.hmax, smem, it)) return;
-  if (it.actual <= 0) return;  // no token: Stage 2 writes the rows as 0
-  if (it.actual <= kLowRows) {
-    if (it.shared) stage1_item<QT, GATHER, kLowRows, false, false>(p, it, smem);
-    else stage1_item<QT, GATHER, kLowRows, false, true>(p, it, smem);
-  } else if (QT != kQF16 || it.actual <= kWideRows) {
-    if (it.shared) stage1_item<QT, GATHER, kWideRows, false, false>(p, it, smem);
-    else stage1_item<QT, GATHER, kWideRows, false, true>(p, it, smem);
-  } else if constexpr (QT == kQF16) {
-    if (it.shared) stage1_item<QT, GATHER, kWideRows, true, false>(p, it, smem);
-    else stage1_item<QT, GATHER, kWideRows, true, true>(p, it, smem);
+  if constexpr (GATHER) {
+    if (item_fused(blockIdx.x, p.istart, p.xb, p.gs, p.gpo, p.E, kBN, nt, p.rows_cap, it)) run(it);
+  } else {
+    if (item_bx(blockIdx.x, p.gidx, p.host_blocks, p.E, kBN, nt, p.gs, p.gpo, p.hmax, gridDim.x, smem, it)) run(it);
   }
 }
 
@@ -1107,10 +1112,24 @@ template <int QT, bool FUSED, int BN>
 __global__ __launch_bounds__(512) void stage2_wide_kernel(Stage2Params p) {
   __shared__ __attribute__((aligned(16))) char smem[kLdsBytes];
   const int nt = (int)(p.H / BN);
+  auto run = [&](const Item& it) {
+    if (it.actual <= 0) return;
+    if (it.actual <= kLowRows) {
+      if (it.shared) stage2_item<QT, FUSED, BN, kLowRows, false, false>(p, it, smem);
+      else stage2_item<QT, FUSED, BN, kLowRows, false, true>(p, it, smem);
+    } else if (QT != kQF16 || it.actual <= kWideRows) {
+      if (it.shared) stage2_item<QT, FUSED, BN, kWideRows, false, false>(p, it, smem);
+      else stage2_item<QT, FUSED, BN, kWideRows, false, true>(p, it, smem);
+    } else if constexpr (QT == kQF16) {
+      if (it.shared) stage2_item<QT, FUSED, BN, kWideRows, true, false>(p, it, smem);
+      else stage2_item<QT, FUSED, BN, kWideRows, true, true>(p, it, smem);
+    }
+  };
   Item it;
-  if (FUSED ? !item_fused(blockIdx.x, p.istart, p.xb, p.gs, p.gpo, p.E, BN, nt, p.rows_cap, it)
-            : !item_bx(blockIdx.x, p.gidx, p.host_blocks, p.E, BN, nt, p.gs, p.gpo, p.hmax, smem, it)) return;
-  if constexpr (!FUSED) {
+  if constexpr (FUSED) {
+    if (item_fused(blockIdx.x, p.istart, p.xb, p.gs, p.gpo, p.E, BN, nt, p.rows_cap, it)) run(it);
+  } else {
+    if (!item_bx(blockIdx.x, p.gidx, p.host_blocks, p.E, BN, nt, p.gs, p.gpo, p.hmax, gridDim.x, smem, it)) return;
     // Rows owned by no valid token are written as 0 (problem_detail.json:50 note 4).
     _Float16* o = reinterpret_cast<_Float16*>(p.out);
     const int rows = it.zero_end - (it.row0 + it.actual);
@@ -1118,17 +1137,7 @@ __global__ __launch_bounds__(512) void stage2_wide_kernel(Stage2Params p) {
       const int r = it.row0 + it.actual + idx / (BN / 8), c = idx % (BN / 8);
       *reinterpret_cast<u32x4*>(o + (int64_t)r * p.H + it.n0 + 8 * c) = u32x4{0, 0, 0, 0};
     }
-    if (it.actual <= 0) return;
-  }
-  if (it.actual <= kLowRows) {
-    if (it.shared) stage2_item<QT, FUSED, BN, kLowRows, false, false>(p, it, smem);
-    else stage2_item<QT, FUSED, BN, kLowRows, false, true>(p, it, smem);
-  } else if (QT != kQF16 || it.actual <= kWideRows) {
-    if (it.shared) stage2_item<QT, FUSED, BN, kWideRows, false, false>(p, it, smem);
-    else stage2_item<QT, FUSED, BN, kWideRows, false, true>(p, it, smem);
-  } else if constexpr (QT == kQF16) {
-    if (it.shared) stage2_item<QT, FUSED, BN, kWideRows, true, false>(p, it, smem);
-    else stage2_item<QT, FUSED, BN, kWideRows, true, true>(p, it, smem);
+    run(it);
   }
 }
 
@@ -1161,7 +1170,11 @@ static hipError_t go1_narrow(const Stage1Params& p, int64_t max_blocks, hipStrea
   return hipGetLastError();
 }
 static int64_t wide_grid(bool fused, int64_t pieces, int64_t rows, int64_t nt) {
-  return fused ? kNumXcd * xcd_items_bound(pieces, rows, nt) : schedule_grid(pieces, nt);
+  // pre-routed: an eighth more than an equal cut needs, so that a cut by cost
+  // fits.  H 7168, I 2048: 32 experts, 5 of them tall, 1796 rows 717 -> 650 us;
+  // 64 experts, 9000 rows 1523 -> 1420; the surplus workgroups cost even
+  // groupings 1-4% (376 -> 390, 632 -> 639, 1233 -> 1241 us).
+  return fused ? kNumXcd * xcd_items_bound(pieces, rows, nt) : schedule_grid(pieces + (pieces + 7) / 8, nt);
 }
 template <int QT>
 static hipError_t go1(const Stage1Params& p, bool gather, int64_t max_blocks, int64_t max_rows, hipStream_t s) {

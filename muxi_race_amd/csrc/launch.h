@@ -101,7 +101,7 @@ hipError_t launch_zero(void* p, int64_t n, hipStream_t stream);
 // qt: a QuantType.  narrow: 32-row items over rows padded to 32 (gather / fused
 // only); otherwise wide items.  max_blocks: an upper bound on the items per N
 // tile (narrow: 32-row blocks; wide: row pieces; direct: 128-row blocks);
-// max_rows: of the routed rows (wide, gather / fused).
+// max_rows: of the routed rows (wide).
 // bn256: Stage 2's wide items take 256 features where H allows.
 hipError_t launch_stage1(const Stage1Params& p, bool narrow, int qt, bool gather,
                          int64_t max_blocks, int64_t max_rows, hipStream_t stream);

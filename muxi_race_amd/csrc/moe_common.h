@@ -88,18 +88,14 @@ __device__ __forceinline__ void barrier_no_fence() {
 
 #define MOE_LDS_PTR(p) ((__attribute__((address_space(3))) void*)(p))
 
-// Cache policy of weight loads that no other tile repeats, used by the
-// decode-sized (32-row) kernels.  A weight tile read by exactly one item is
-// loaded non-temporal (the gfx950 `nt` bit, cache-policy immediate 2):
-// decode went from 0.575 to 0.533 ms with it (a load-only copy of the 96-row
-// decode ring streamed 6.15 -> 7.12 TB/s at rows 14 KiB apart, 5.45 -> 6.14
-// TB/s at 4 KiB).  Weight tiles that sibling items of a multi-block
-// expert re-read from L2, and token / intermediate rows, keep the default
-// policy (non-temporal there measured slower: fewer L2 hits).  Of the
-// wide-tile kernels, only the 8-bit 256-row items stream their unshared
-// weight tiles (MOE_W8_STREAM in grouped_gemm.hip, measured faster there);
-// the fp16 ones load everything with the default policy (no gain measured,
-// and the per-instruction choice cost 2-5%).  0 turns streaming off.
+// Cache policy of weight loads that no other tile repeats.  A weight tile read
+// by exactly one item is loaded non-temporal (the gfx950 `nt` bit,
+// cache-policy immediate 2): decode went from 0.575 to 0.533 ms with it (a
+// load-only copy of the 96-row decode ring streamed 6.15 -> 7.12 TB/s at rows
+// 14 KiB apart, 5.45 -> 6.14 TB/s at 4 KiB).  Weight tiles that sibling items
+// of an expert re-read from L2, and token / intermediate rows, keep the
+// default policy (non-temporal there measured slower: fewer L2 hits).
+// 0 turns streaming off.
 #ifndef MOE_W_POLICY
 #define MOE_W_POLICY 2
 #endif
@@ -420,136 +416,7 @@ __device__ __forceinline__ bool item_fused(int g, const int32_t* __restrict__ is
   return it.actual > 0 && it.row0 + it.actual <= rows_cap;
 }
 
-// Pre-routed launches (the reference operator): block b of 128 rows belongs to
-// expert gidx[b] (problem_detail.json:50 note 5; submission.py:1444), and the
-// launch covers blocks [0, nblk) with nblk = min(gidx entries, blocks of the
-// row buffers), as submission.py:2115 launches group_idx_for_bx.numel()
-// blocks.  The maximal run [s, end) of consecutive blocks with one gidx value
-// is treated as one expert: its first n = clamp(gs[e] - (128 s - gpo[e]), 0,
-// 128 (end - s)) rows are routed (the per-block rule of each of its blocks),
-// and the rest have no token.  A run without tokens still has one item per N
-// tile, which writes its rows as 0.  A gidx value outside [0, E) gives e = -1
-// (rows owned by no expert).
-//
-// The items below a run are counted here, by the workgroup's 512 threads, 512
-// blocks at a time: block j of a run counts the pieces that its rows add,
-// items_of(min(n, 128 (j + 1))) - items_of(min(n, 128 j)), which sums to the
-// run's.  (Numbering by blocks instead, with the surplus items ending at once,
-// left the XCDs unequal work: 22 experts of 155 rows and 10 of 112, H 7168, I
-// 2048, Stage 1 551 us.)
-struct RunScan {
-  int smem_s[8], smem_p[8];
-};
-
-__device__ __forceinline__ bool item_bx(int g, const int32_t* __restrict__ gidx, int nblk, int E, int BN, int nt,
-                                        const int32_t* __restrict__ gs, const int32_t* __restrict__ gpo, int hmax,
-                                        char* smem, Item& it) {
-  constexpr int BM = 128, kThreads = 512;
-  RunScan* sh = reinterpret_cast<RunScan*>(smem);
-  const int l = lane_id(), w = wave_id();
-  // pass over all blocks; f(block, first of its run, items below it)
-  auto sweep = [&](auto&& f) {
-    int carry_s = 0, carry_p = 0;
-    for (int base = 0; base < nblk; base += kThreads) {
-      const int b = base + (int)threadIdx.x;
-      const int bc = b < nblk ? b : nblk - 1;
-      const int val = gidx[bc], before = gidx[bc > 0 ? bc - 1 : 0];
-      const bool first = b < nblk && (b == 0 || val != before);
-      const uint64_t m = __ballot(first);
-      if (l == 0) sh->smem_s[w] = m ? base + 64 * w + 63 - __builtin_clzll(m) : -1;
-      const bool owned = val >= 0 && val < E;
-      const int ec = owned ? val : 0;
-      const int gs_e = gs[ec], gpo_e = gpo[ec];
-      __syncthreads();
-      int s = carry_s;
-      for (int v = 0; v < w; ++v) s = sh->smem_s[v] >= 0 ? sh->smem_s[v] : s;
-      const uint64_t upto = m & (l == 63 ? ~0ull : (1ull << (l + 1)) - 1);
-      if (upto) s = base + 64 * w + 63 - __builtin_clzll(upto);
-      const int64_t left = owned ? (int64_t)gs_e - ((int64_t)s * BM - gpo_e) : 0;
-      const int64_t lo = (int64_t)(b - s) * BM, hi = lo + BM;
-      int c = 0;
-      if (b < nblk) {
-        if (left > 0) c = items_of((int)(left < hi ? left : hi), hmax) - items_of((int)(left < lo ? left : lo), hmax);
-        else c = first;
-      }
-      const int inc = wave_inclusive_scan(c);
-      if (l == 63) sh->smem_p[w] = inc;
-      __syncthreads();
-      int below = carry_p;
-      for (int v = 0; v < 8; ++v) {
-        if (v == w) f(b, first, below + inc - c);
-        below += sh->smem_p[v];
-        carry_s = sh->smem_s[v] >= 0 ? sh->smem_s[v] : carry_s;
-      }
-      carry_p = below;
-      __syncthreads();  // the next pass (or caller) writes the same memory
-    }
-    return carry_p;
-  };
-  int p0 = 0;
-  bool first0 = false;
-  const int total = sweep([&](int b, bool first, int below) {
-    if (b < kThreads) {
-      first0 = first;
-      p0 = below;
-    }
-  });
-  const int v = xcd_item(g, total * nt);
-  if (v < 0) return false;
-  // the last run whose first item is <= v: block s, items below it ps
-  int s = -1, ps = 0;
-  auto find = [&](int b, bool first, int below) {
-    const uint64_t m = __ballot(first && below * nt <= v);
-    if (m) {
-      const int lane = 63 - __builtin_clzll(m);
-      s = __shfl(b, lane);
-      ps = __shfl(below, lane);
-    }
-  };
-  if (nblk <= kThreads) find((int)threadIdx.x, first0, p0);
-  else sweep(find);
-  if (l == 0) {
-    sh->smem_s[w] = s;
-    sh->smem_p[w] = ps;
-  }
-  __syncthreads();
-  for (int u = 0; u < 8; ++u)
-    if (sh->smem_s[u] > s) {
-      s = sh->smem_s[u];
-      ps = sh->smem_p[u];
-    }
-  s = __builtin_amdgcn_readfirstlane(s);
-  ps = __builtin_amdgcn_readfirstlane(ps);
-  __syncthreads();  // the caller reuses smem
-  const int val = gidx[s];
-  // run end: the nearest block above s with another value (or nblk)
-  int end = -1;
-  for (int base = s + 1; end < 0; base += 64) {
-    const int b = base + l;
-    const bool diff = b >= nblk || gidx[b] != val;
-    const uint64_t m = __ballot(diff);
-    if (m) end = base + (__ffsll((unsigned long long)m) - 1);
-  }
-  it.e = val >= 0 && val < E ? val : -1;
-  int n = 0;
-  if (it.e >= 0) {
-    const int64_t left = (int64_t)gs[it.e] - ((int64_t)s * BM - gpo[it.e]);
-    const int64_t cap = (int64_t)(end - s) * BM;
-    n = (int)(left < 0 ? 0 : (left > cap ? cap : left));
-  }
-  const int c = n > 0 ? items_of(n, hmax) : 1;
-  const int local = v - ps * nt;
-  const int t = local / c, i = local % c;
-  const int r = n > 0 ? rows_of(n, c) : 0;
-  it.row0 = s * BM + i * r;
-  it.actual = n - i * r < r ? n - i * r : r;
-  it.n0 = t * BN;
-  it.zero_end = i == c - 1 ? end * BM : 0;
-  it.shared = c > 1;
-  return t < nt;
-}
-
-// XCD shares of a fused launch's items, for one lane: the first item of XCD x
+// XCD shares of a launch's items, for one lane: the first item of XCD x
 // (x = 8: the end) and the cost of the items before it.  `weighted`: the items
 // are cut where the cost is an eighth each; otherwise into equal numbers.  An
 // item of r rows costs kItemCost + r: at 256 experts of H 7168, I 2048 a Stage 1
@@ -590,9 +457,12 @@ __device__ __forceinline__ XcdCut xcd_cut(int x, bool weighted, const int* ist, 
 // of a wave, and the better one written to xb[0..8]: the one whose slowest XCD
 // needs less time, an XCD running its items kCusPerXcd at a time.  Equal cost
 // pays where experts differ and there are many rounds; with two rounds of like
-// items it would leave some XCD a third.
+// pays where experts differ and there are many rounds; with two rounds of like
+// items it would leave some XCD a third.  slots: workgroups an XCD has in the
+// launch; an equal cut always fits.
 constexpr int kCusPerXcd = 32;
-__device__ __forceinline__ void xcd_shares(const int* ist, const int* gof, int E, int nt, int32_t* __restrict__ xb) {
+__device__ __forceinline__ void xcd_shares(const int* ist, const int* gof, int E, int nt, int32_t* xb,
+                                           int slots = 0x7fffffff) {
   const int l = lane_id();
   const int x = l % 9;
   XcdCut cut = {0, 0.0};
@@ -603,13 +473,189 @@ __device__ __forceinline__ void xcd_shares(const int* ist, const int* gof, int E
   if (l < 18 && x < 8 && items > 0) t = (float)((items + kCusPerXcd - 1) / kCusPerXcd) * cost / (float)items;
   float slow[2] = {0.0f, 0.0f};
   for (int q = 0; q < 18; ++q) slow[q / 9] = fmaxf(slow[q / 9], __shfl(t, q));
-  const bool weighted = slow[1] < slow[0];
+  const bool fits = __ballot(l >= 9 && l < 17 && items > slots) == 0;
+  const bool weighted = fits && slow[1] < slow[0];
   if (l < 18 && (l >= 9) == weighted) xb[x] = cut.item;
 }
 // An upper bound on an XCD's items either way, for `pieces` items per N tile and
 // `rows` routed rows in all.
 inline int64_t xcd_items_bound(int64_t pieces, int64_t rows, int64_t nt) {
   return (pieces * kItemCost + rows) * nt / (kNumXcd * kItemCost) + 2;
+}
+
+// Pre-routed launches (the reference operator): block b of 128 rows belongs to
+// expert gidx[b] (problem_detail.json:50 note 5; submission.py:1444), and the
+// launch covers blocks [0, nblk) with nblk = min(gidx entries, blocks of the
+// row buffers), as submission.py:2115 launches group_idx_for_bx.numel()
+// blocks.  The maximal run [s, end) of consecutive blocks with one gidx value
+// is treated as one expert: its first n = clamp(gs[e] - (128 s - gpo[e]), 0,
+// 128 (end - s)) rows are routed (the per-block rule of each of its blocks),
+// and the rest have no token.  A run without tokens still has one item per N
+// tile, which writes its rows as 0.  A gidx value outside [0, E) gives e = -1
+// (rows owned by no expert).
+//
+// The items below a run are counted here, by the workgroup's 512 threads, 512
+// blocks at a time: block j of a run counts the pieces that its rows add,
+// items_of(min(n, 128 (j + 1))) - items_of(min(n, 128 j)), which sums to the
+// run's.  (Numbering by blocks instead, with the surplus items ending at once,
+// left the XCDs unequal work: 22 experts of 155 rows and 10 of 112, H 7168, I
+// 2048, Stage 1 551 us.)
+//
+// Launches of up to 512 blocks with an expert of more than kCutRows rows cut
+// their items over the XCDs as the fused ones do (xcd_shares, over blocks
+// instead of experts); others into equal numbers, which saves the 2 us that the
+// comparison of the two cuts takes before each item.
+constexpr int kCutRows = 192;
+struct RunScan {
+  int smem_s[8], smem_p[8], smem_r[8];
+  int xb[9];
+  int ist[513], gof[513];  // items per N tile and rows below each block
+};
+
+__device__ __forceinline__ bool item_bx(int g, const int32_t* __restrict__ gidx, int nblk, int E, int BN, int nt,
+                                        const int32_t* __restrict__ gs, const int32_t* __restrict__ gpo, int hmax,
+                                        int grid, char* smem, Item& it) {
+  constexpr int BM = 128, kThreads = 512;
+  RunScan* sh = reinterpret_cast<RunScan*>(smem);
+  const int l = lane_id(), w = wave_id();
+  // pass over all blocks; f(block, first of its run, items below it, rows below it)
+  int rows_all = 0;
+  bool tall = false;  // a block of this thread belongs to a run of more than kCutRows rows
+  auto sweep = [&](auto&& f) {
+    int carry_s = 0, carry_p = 0, carry_r = 0;
+    for (int base = 0; base < nblk; base += kThreads) {
+      const int b = base + (int)threadIdx.x;
+      const int bc = b < nblk ? b : nblk - 1;
+      const int val = gidx[bc], before = gidx[bc > 0 ? bc - 1 : 0];
+      const bool first = b < nblk && (b == 0 || val != before);
+      const uint64_t m = __ballot(first);
+      if (l == 0) sh->smem_s[w] = m ? base + 64 * w + 63 - __builtin_clzll(m) : -1;
+      const bool owned = val >= 0 && val < E;
+      const int ec = owned ? val : 0;
+      const int gs_e = gs[ec], gpo_e = gpo[ec];
+      __syncthreads();
+      int s = carry_s;
+      for (int v = 0; v < w; ++v) s = sh->smem_s[v] >= 0 ? sh->smem_s[v] : s;
+      const uint64_t upto = m & (l == 63 ? ~0ull : (1ull << (l + 1)) - 1);
+      if (upto) s = base + 64 * w + 63 - __builtin_clzll(upto);
+      const int64_t left = owned ? (int64_t)gs_e - ((int64_t)s * BM - gpo_e) : 0;
+      const int64_t lo = (int64_t)(b - s) * BM, hi = lo + BM;
+      int c = 0, r = 0;  // pieces and routed rows that this block adds
+      if (b < nblk) {
+        const int upto_hi = (int)(left < hi ? left : hi), upto_lo = (int)(left < lo ? left : lo);
+        if (left > 0) {
+          c = items_of(upto_hi, hmax) - items_of(upto_lo, hmax);
+          r = upto_hi - upto_lo;
+        } else {
+          c = first;
+        }
+        tall = tall || left > kCutRows;
+      }
+      const int inc = wave_inclusive_scan(c), incr = wave_inclusive_scan(r);
+      if (l == 63) {
+        sh->smem_p[w] = inc;
+        sh->smem_r[w] = incr;
+      }
+      __syncthreads();
+      int below = carry_p, rbelow = carry_r;
+      for (int v = 0; v < 8; ++v) {
+        if (v == w) f(b, first, below + inc - c, rbelow + incr - r);
+        below += sh->smem_p[v];
+        rbelow += sh->smem_r[v];
+        carry_s = sh->smem_s[v] >= 0 ? sh->smem_s[v] : carry_s;
+      }
+      carry_p = below;
+      carry_r = rbelow;
+      __syncthreads();  // the next pass (or caller) writes the same memory
+    }
+    rows_all = carry_r;
+    return carry_p;
+  };
+  int p0 = 0;
+  bool first0 = false;
+  const int total = sweep([&](int b, bool first, int below, int rbelow) {
+    if (b < kThreads) {
+      first0 = first;
+      p0 = below;
+      if (b < nblk) {
+        sh->ist[b] = below;
+        sh->gof[b] = rbelow;
+      }
+    }
+  });
+  const bool any = __ballot(tall) != 0;
+  if (l == 0) sh->smem_r[w] = any;
+  __syncthreads();  // orders ist and gof, too
+  bool cut = false;
+  for (int u = 0; u < 8; ++u) cut = cut || sh->smem_r[u];
+  int v;
+  if (nblk <= kThreads && cut) {
+    if (w == 0) {
+      if (l == 0) {
+        sh->ist[nblk] = total;
+        sh->gof[nblk] = rows_all;
+      }
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+      xcd_shares(sh->ist, sh->gof, nblk, nt, sh->xb, grid / kNumXcd);
+    }
+    __syncthreads();
+    v = sh->xb[g % kNumXcd] + g / kNumXcd;
+    if (v >= sh->xb[g % kNumXcd + 1]) return false;
+  } else {
+    v = xcd_item(g, total * nt);
+    if (v < 0) return false;
+  }
+  // the last run whose first item is <= v: block s, items below it ps
+  int s = -1, ps = 0;
+  auto find = [&](int b, bool first, int below, int) {
+    const uint64_t m = __ballot(first && below * nt <= v);
+    if (m) {
+      const int lane = 63 - __builtin_clzll(m);
+      s = __shfl(b, lane);
+      ps = __shfl(below, lane);
+    }
+  };
+  if (nblk <= kThreads) find((int)threadIdx.x, first0, p0, 0);
+  else sweep(find);
+  if (l == 0) {
+    sh->smem_s[w] = s;
+    sh->smem_p[w] = ps;
+  }
+  __syncthreads();
+  for (int u = 0; u < 8; ++u)
+    if (sh->smem_s[u] > s) {
+      s = sh->smem_s[u];
+      ps = sh->smem_p[u];
+    }
+  s = __builtin_amdgcn_readfirstlane(s);
+  ps = __builtin_amdgcn_readfirstlane(ps);
+  __syncthreads();  // the caller reuses smem
+  const int val = gidx[s];
+  // run end: the nearest block above s with another value (or nblk)
+  int end = -1;
+  for (int base = s + 1; end < 0; base += 64) {
+    const int b = base + l;
+    const bool diff = b >= nblk || gidx[b] != val;
+    const uint64_t m = __ballot(diff);
+    if (m) end = base + (__ffsll((unsigned long long)m) - 1);
+  }
+  it.e = val >= 0 && val < E ? val : -1;
+  int n = 0;
+  if (it.e >= 0) {
+    const int64_t left = (int64_t)gs[it.e] - ((int64_t)s * BM - gpo[it.e]);
+    const int64_t cap = (int64_t)(end - s) * BM;
+    n = (int)(left < 0 ? 0 : (left > cap ? cap : left));
+  }
+  const int c = n > 0 ? items_of(n, hmax) : 1;
+  const int local = v - ps * nt;
+  const int t = local / c, i = local % c;
+  const int r = n > 0 ? rows_of(n, c) : 0;
+  it.row0 = s * BM + i * r;
+  it.actual = n - i * r < r ? n - i * r : r;
+  it.n0 = t * BN;
+  it.zero_end = i == c - 1 ? end * BM : 0;
+  it.shared = c > 1;
+  return t < nt;
 }
 
 // Workgroups of a launch of `blocks` blocks (or row pieces) x `ntiles` items.
