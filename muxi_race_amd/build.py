@@ -56,7 +56,7 @@ def _compile(src: Path, obj: Path, extra=()) -> tuple[Path, str]:
 def build(verbose: bool = False, defines: dict | None = None, out: Path | None = None) -> Path:
     """Compile every csrc/*.hip and link the shared library; returns its path.
 
-    ``defines`` adds -DNAME=VALUE tuning macros (e.g. MOE_S2_STAGES_128) and
+    ``defines`` adds -DNAME=VALUE tuning macros (e.g. MOE_S1N_STAGES) and
     ``out`` redirects the library (default: muxi_race_amd/libmoe_gfx950.so)."""
     lib = LIB if out is None else Path(out)
     objdir = OBJDIR if out is None else lib.parent / "_build"

@@ -153,7 +153,7 @@ __global__ __launch_bounds__(256) void stage1_narrow_kernel(Stage1Params p) {
 
   const int64_t kbytes = p.H * (I8 ? 1 : 2);
   const int nk = (int)(kbytes / kRowBytes);
-  const bool sh = p.e_shared >= 0 && e == p.e_shared;  // see stage1_kernel
+  const bool sh = p.e_shared >= 0 && e == p.e_shared;  // the shared expert's own tensors, same row stride
   const char* gexp = sh ? p.wg_shared : p.wg + (int64_t)e * p.w_es;
   const char* uexp = sh ? p.wu_shared : p.wu + (int64_t)e * p.w_es;
   LD ld;

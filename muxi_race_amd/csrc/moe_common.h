@@ -457,7 +457,6 @@ __device__ __forceinline__ XcdCut xcd_cut(int x, bool weighted, const int* ist, 
 // of a wave, and the better one written to xb[0..8]: the one whose slowest XCD
 // needs less time, an XCD running its items kCusPerXcd at a time.  Equal cost
 // pays where experts differ and there are many rounds; with two rounds of like
-// pays where experts differ and there are many rounds; with two rounds of like
 // items it would leave some XCD a third.  slots: workgroups an XCD has in the
 // launch; an equal cut always fits.
 constexpr int kCusPerXcd = 32;
