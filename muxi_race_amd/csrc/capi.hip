@@ -126,6 +126,10 @@ WidePlan wide_plan(int64_t rows, int64_t experts, int64_t H, int64_t I, int qt) 
   return w;
 }
 
+// run_kernel: average rows of an expert up to which more blocks than experts
+// mean short items.
+constexpr int64_t kSkewRows = 112;
+
 bool aligned16(const void* p) { return ((uintptr_t)p & 15) == 0; }
 
 int check_dims(int64_t T, int64_t H, int64_t I, int64_t E, int64_t k, int64_t bm) {
@@ -191,7 +195,14 @@ int moe_run_prerouted_events(const void* x, const void* w_gate, const void* w_up
   p1.H = H;
   p1.I = I;
   const int64_t experts = E < blocks ? E : blocks;
-  const WidePlan wide = wide_plan(V > experts ? V : experts, experts, H, I, moe::kQF16);
+  WidePlan wide = wide_plan(V > experts ? V : experts, experts, H, I, moe::kQF16);
+  // A low average beside more blocks than experts: a few tall experts among
+  // short ones.  Items of up to 288 rows then end long after the short ones.
+  // Up to 288 rows, up to 128: 32 experts (H 7168, I 2048) of 3 rows but 8 of 336
+  // 735 -> 653 us, of 11 but 5 of 300 632 -> 604, of 60 but 3 of 380 654 -> 619; 16
+  // (H 2048, I 8192) of 19 but 4 of 350 448 -> 415: averages of 56 to 102.  At
+  // 141 (64 experts of 30 but 41 of 203) 1331 -> 1390, so the line lies between.
+  if (V <= kSkewRows * experts && blocks > experts) wide.hmax = moe::kLowRows;
   p1.hmax = wide.hmax;
   // optional stage markers: ev[0] start, [1] stage 1, [2] stage 2
   auto mark = [&](int i) { if (stage_events && stage_events[i]) (void)hipEventRecord((hipEvent_t)stage_events[i], s); };

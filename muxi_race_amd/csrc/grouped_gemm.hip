@@ -1169,16 +1169,15 @@ static hipError_t go1_narrow(const Stage1Params& p, int64_t max_blocks, hipStrea
   }
   return hipGetLastError();
 }
-static int64_t wide_grid(bool fused, int64_t pieces, int64_t rows, int64_t nt) {
-  // pre-routed: an eighth more than an equal cut needs, so that a cut by cost
-  // fits.  H 7168, I 2048: 32 experts, 5 of them tall, 1796 rows 717 -> 650 us;
-  // 64 experts, 9000 rows 1523 -> 1420; the surplus workgroups cost even
+static int64_t wide_grid(bool fused, int64_t pieces, int64_t rows, int64_t nt, int hmax) {
+  // pre-routed, where item_bx may cut by cost: an eighth more than an equal cut needs, so that a cut by cost
+  // fits.  H 7168, I 2048, 64 experts, 9000 rows 1523 -> 1420 us; the surplus workgroups cost even
   // groupings 1-4% (376 -> 390, 632 -> 639, 1233 -> 1241 us).
-  return fused ? kNumXcd * xcd_items_bound(pieces, rows, nt) : schedule_grid(pieces + (pieces + 7) / 8, nt);
+  return fused ? kNumXcd * xcd_items_bound(pieces, rows, nt) : schedule_grid(pieces + (hmax > kLowRows ? (pieces + 7) / 8 : 0), nt);
 }
 template <int QT>
 static hipError_t go1(const Stage1Params& p, bool gather, int64_t max_blocks, int64_t max_rows, hipStream_t s) {
-  const dim3 grid((unsigned)wide_grid(gather, max_blocks, max_rows, p.I / kBN));
+  const dim3 grid((unsigned)wide_grid(gather, max_blocks, max_rows, p.I / kBN, p.hmax));
   if (gather) hipLaunchKernelGGL((stage1_wide_kernel<QT, true>), grid, dim3(512), 0, s, p);
   else if constexpr (QT == kQF16) hipLaunchKernelGGL((stage1_wide_kernel<QT, false>), grid, dim3(512), 0, s, p);
   else return hipErrorInvalidValue;
@@ -1186,7 +1185,7 @@ static hipError_t go1(const Stage1Params& p, bool gather, int64_t max_blocks, in
 }
 template <int QT, int BN>
 static hipError_t go2(const Stage2Params& p, bool fused, int64_t max_blocks, int64_t max_rows, hipStream_t s) {
-  const dim3 grid((unsigned)wide_grid(fused, max_blocks, max_rows, p.H / BN));
+  const dim3 grid((unsigned)wide_grid(fused, max_blocks, max_rows, p.H / BN, p.hmax));
   if (fused) hipLaunchKernelGGL((stage2_wide_kernel<QT, true, BN>), grid, dim3(512), 0, s, p);
   else if constexpr (QT == kQF16) hipLaunchKernelGGL((stage2_wide_kernel<QT, false, BN>), grid, dim3(512), 0, s, p);
   else return hipErrorInvalidValue;

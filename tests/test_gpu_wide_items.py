@@ -158,3 +158,18 @@ def test_small_batches_route_and_align_in_one_launch(E, k, T, bias):
     torch.cuda.synchronize()
     assert torch.equal(ids, rid) and torch.equal(wts.view(torch.int32), rw.view(torch.int32))
     assert torch.equal(torch.nan_to_num(out), torch.nan_to_num(want))
+
+
+@pytest.mark.parametrize("tall", [129, 288, 289, 380])
+@pytest.mark.parametrize("low", [1, 100])
+def test_prerouted_few_tall_experts(tall, low):
+    """A few tall experts among short ones: items of up to 128 rows where the
+    average is at most 112 rows and there are more blocks than experts."""
+    from muxi_race_amd import run_kernel
+    sizes = [low] * 18
+    sizes[2] = sizes[17] = tall
+    args = prerouted_inputs(sizes, 256, 2048, seed=tall + low)
+    out = torch.full(args[0].shape, float("nan"), dtype=torch.float16, device="cuda")
+    run_kernel(*args, out)
+    torch.cuda.synchronize()
+    assert_close(out, prerouted_forward(*args), what=f"{tall} rows beside {low}")
