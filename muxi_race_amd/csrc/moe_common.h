@@ -363,10 +363,14 @@ __device__ __forceinline__ bool schedule(int g, const int32_t* __restrict__ gpo,
 }
 
 // Wide items (more than 32 rows per expert).  An expert of n routed rows runs
-// c = ceil(n / hmax) items per N tile, of rows_of(n, c) rows each (the last one
-// of what is left): its rows split evenly in multiples of 32, so an item
-// streams a weight tile for as many rows as the tallest tile holds and no item
-// is left with a few.  All items span the whole N tile; item v of expert e is
+// c = ceil(n / hmax) items per N tile, of rows_of(n, c) rows each, n / c rounded
+// up to a multiple of 32; the last one takes what is left, at least one row (385
+// rows with hmax 128: 128, 128, 128, 1).  Dealing the 32-row blocks out evenly
+// instead (128, 96, 96, 65) was slower, since waves and token loads work in
+// 64-row steps and three short pieces then cost what full ones do: H 7168, I
+// 2048, 32 experts of 11 rows but 5 of 300 (128, 128, 44 -> 128, 96, 76) 611 ->
+// 638 us, 64 of 20 but 10 of 300 1180 -> 1203.
+// All items span the whole N tile; item v of expert e is
 // N tile (v - first) / c, row piece (v - first) % c, so the c items reading one
 // weight tile are adjacent.  hmax is kTallRows where the tiles take absorbed
 // rows (moe_common.h kAbsorbRows), kWideRows otherwise, and kLowRows where the

@@ -173,3 +173,22 @@ def test_prerouted_few_tall_experts(tall, low):
     run_kernel(*args, out)
     torch.cuda.synchronize()
     assert_close(out, prerouted_forward(*args), what=f"{tall} rows beside {low}")
+
+
+@pytest.mark.parametrize("I", [256, 4096])
+def test_last_piece_of_one_row(I):
+    """Row counts that leave an expert's last piece one row: 385 in pieces of
+    up to 128, 2305 in pieces of up to 288, through fused_moe and run_kernel
+    (I 256: short items, 4096: tall ones)."""
+    from muxi_race_amd import fused_moe, run_kernel
+    sizes = [385, 2305, 1, 33, 300, 417]
+    x, lg, wg, wu, wd = _case(sizes, 256, I, 1, 8)
+    out = torch.full((x.shape[0], 256), float("nan"), dtype=torch.float16, device="cuda")
+    out = fused_moe(x.cuda(), lg.cuda(), wg.cuda(), wu.cuda(), wd.cuda(), 1, block_m=64, out=out)
+    torch.cuda.synchronize()
+    assert_close(out, fused_moe_forward(x, lg, wg, wu, wd, 1), what=f"last piece I={I}")
+    args = prerouted_inputs(sizes, 256, I, seed=9)
+    out = torch.full(args[0].shape, float("nan"), dtype=torch.float16, device="cuda")
+    run_kernel(*args, out)
+    torch.cuda.synchronize()
+    assert_close(out, prerouted_forward(*args), what=f"prerouted last piece I={I}")
