@@ -37,7 +37,7 @@ int64_t cap_rows(int64_t T, int64_t k, int64_t E, int64_t bm) {
 }
 
 struct FusedLayout {
-  int64_t ids, w, sorted, bexp, gs, go, gpo, istart, whist, h, hq, hs, xq, sx, ypair, pos, total;
+  int64_t ids, w, sorted, bexp, gs, go, gpo, plan, whist, h, hq, hs, xq, sx, ypair, pos, total;
 };
 
 // qt: moe::kQF16, kQI8 or kQF8.  The intermediate h is fp16 for fp16 and int8
@@ -57,7 +57,7 @@ FusedLayout fused_layout(int64_t T, int64_t H, int64_t I, int64_t E, int64_t k, 
   L.gs = o; o += up(E * 4);
   L.go = o; o += up((E + 1) * 4);
   L.gpo = o; o += up((E + 1) * 4);
-  L.istart = o; o += up((E + 19) * 4);                   // wide items per N tile below each expert, XCD bounds
+  L.plan = o; o += up(moe::ItemPlan::ints(E) * 4);        // the wide items' plan
   L.whist = o; o += up((int64_t)moe::align_groups((int)P) * E * 4);  // align workgroup histograms
   L.h = o; o += up(rows * I * (qt == moe::kQF8 ? 1 : 2));
   L.hq = o; o += i8 ? up(rows * I) : 0;                   // int8: per-row codes of h
@@ -103,26 +103,64 @@ int64_t align_bm(int64_t T, int64_t E, int64_t k, int64_t H, int64_t I, int64_t 
   return bm == 128 && H % 256 == 0 && avg >= 192 ? 256 : bm;
 }
 
-// How the wide items split `rows` routed rows over at most `experts` experts:
-// the most rows of an item, whether Stage 2 takes 256 features, and an upper
-// bound on the items per N tile.  An expert is assumed to hold the average.
-// Launches that would not give every CU an item take shorter and narrower ones.
+constexpr int64_t kCus = 256;
+
+// What a fused launch's plan (launch.h ItemPlan) may choose from, for any
+// routing of `pairs` pairs over `experts` experts of which `rows` are expected
+// here (an expert shard's share).  With every expert at the average:
+//   - heights below the tallest for launches of up to kPlanRounds items per CU.
+//     With more, the last round is a small part of the launch: up to 4 rounds
+//     the choice won 5-25% on skewed routings (Stage 1 of 60 experts of H 2048, I
+//     1408, 400 tokens top-4, Zipf 112 -> 79 us), at 7 it was level or lost
+//     (Stage 2 of 64 experts of H 7168, I 2048, 200 tokens top-6, Zipf 208 -> 224).
+//   - Stage 2 in 128-feature items as well up to 1.5 items of 256 features per
+//     CU; past it none of those cases gained by them.  Its K loop is short
+//     (I / 64 steps), so 256 features are right where they fill the chip: half
+//     the re-reads of the intermediate and twice the work behind each item's fill
+//     and epilogue.
+// The launches hold the workgroups that the tallest, widest items may need with
+// any routing, and at least one per CU if shorter ones could use them; the plan
+// takes what fits.  A launch sized for the shortest items lost more to surplus
+// workgroups, about 3 us of a CU each (8 experts of H 4096, I 14336, 2048 tokens
+// top-2: Stage 2 500 us, with three times the workgroups 523), and the choice
+// that it left to these was no better.
+constexpr int64_t kPlanRounds = 4;
+moe::ItemPlan fused_plan(int64_t pairs, int64_t rows, int64_t experts, int64_t H, int64_t I, int qt) {
+  const int64_t used = rows < experts ? rows : experts, held = pairs < experts ? pairs : experts;
+  const int64_t avg = used > 0 ? (rows + used - 1) / used : 0;
+  moe::ItemPlan p;
+  p.tall = qt == moe::kQF16 ? moe::kTallRows : moe::kWideRows;
+  p.nt1 = (int)(I / moe::kBN);
+  p.nt2 = (int)(H / moe::kBN);
+  const int64_t items = used * moe::items_of((int)avg, p.tall);
+  p.any1 = items * p.nt1 <= kPlanRounds * kCus;
+  p.any2 = items * ((p.nt2 + 1) / 2) <= kPlanRounds * kCus;
+  p.bn2 = H % 256 ? 128 : (2 * items * (H / 256) <= 3 * kCus ? 0 : 256);
+  auto slots = [&](bool any, int64_t nt, int64_t nt_most) {
+    // sum of ceil(n / hmax) over `held` experts: at most pairs / hmax + held
+    const int64_t least = moe::xcd_items_bound(pairs / p.tall + held, pairs, nt);
+    const int64_t most = moe::xcd_items_bound(pairs / (any ? moe::kLowRows : p.tall) + held, pairs, nt_most);
+    const int64_t one = most < moe::kCusPerXcd ? most : moe::kCusPerXcd;
+    return (int)(least > one ? least : one);
+  };
+  p.slots1 = slots(p.any1, p.nt1, p.nt1);
+  p.slots2 = slots(p.any2, p.bn2 == 128 ? p.nt2 : p.nt2 / 2, p.bn2 == 256 ? p.nt2 / 2 : p.nt2);
+  return p;
+}
+
+// run_kernel: the tallest item and Stage 2's features per item, every expert
+// taken to hold the average of `rows` rows.  Launches that would not give every
+// CU an item take shorter and narrower ones.
 struct WidePlan {
   int hmax;
-  bool bn256;
-  int64_t nt2;        // Stage 2's N tiles
-  int64_t max_items;
+  int bn;
 };
-WidePlan wide_plan(int64_t rows, int64_t experts, int64_t H, int64_t I, int qt) {
-  constexpr int64_t kCus = 256;
-  const int64_t used = rows < experts ? rows : experts;
-  const int64_t avg = used > 0 ? (rows + used - 1) / used : 0;
+WidePlan wide_plan(int64_t rows, int64_t experts, int64_t H, int64_t I) {
+  const int64_t avg = (rows + experts - 1) / experts;
   WidePlan w;
-  w.hmax = qt == moe::kQF16 ? moe::kTallRows : moe::kWideRows;
-  if (used * moe::items_of((int)avg, w.hmax) * (I / moe::kBN) < kCus) w.hmax = moe::kLowRows;
-  w.bn256 = H % 256 == 0 && used * moe::items_of((int)avg, w.hmax) * (H / 256) >= kCus;
-  w.nt2 = H / (w.bn256 ? 256 : 128);
-  w.max_items = rows / w.hmax + used;  // sum of ceil(n / hmax) over `used` experts
+  w.hmax = moe::kTallRows;
+  if (experts * moe::items_of((int)avg, w.hmax) * (I / moe::kBN) < kCus) w.hmax = moe::kLowRows;
+  w.bn = H % 256 == 0 && experts * moe::items_of((int)avg, w.hmax) * (H / 256) >= kCus ? 256 : 128;
   return w;
 }
 
@@ -195,7 +233,7 @@ int moe_run_prerouted_events(const void* x, const void* w_gate, const void* w_up
   p1.H = H;
   p1.I = I;
   const int64_t experts = E < blocks ? E : blocks;
-  WidePlan wide = wide_plan(V > experts ? V : experts, experts, H, I, moe::kQF16);
+  WidePlan wide = wide_plan(V > experts ? V : experts, experts, H, I);
   // A low average beside more blocks than experts: a few tall experts among
   // short ones.  Items of up to 288 rows then end long after the short ones.
   // Up to 288 rows, up to 128: 32 experts (H 7168, I 2048) of 3 rows but 8 of 336
@@ -207,7 +245,7 @@ int moe_run_prerouted_events(const void* x, const void* w_gate, const void* w_up
   // optional stage markers: ev[0] start, [1] stage 1, [2] stage 2
   auto mark = [&](int i) { if (stage_events && stage_events[i]) (void)hipEventRecord((hipEvent_t)stage_events[i], s); };
   mark(0);
-  int rc = check_launch(moe::launch_stage1(p1, false, moe::kQF16, false, blocks, 128 * blocks, s), "stage1");
+  int rc = check_launch(moe::launch_stage1(p1, false, moe::kQF16, false, blocks, s), "stage1");
   if (rc) return rc;
   mark(1);
 
@@ -226,7 +264,8 @@ int moe_run_prerouted_events(const void* x, const void* w_gate, const void* w_up
   p2.I = I;
   p2.V = V;
   p2.hmax = wide.hmax;
-  rc = check_launch(moe::launch_stage2(p2, false, moe::kQF16, false, wide.bn256, blocks, 128 * blocks, s), "stage2");
+  p2.bn = wide.bn;
+  rc = check_launch(moe::launch_stage2(p2, false, moe::kQF16, false, blocks, s), "stage2");
   mark(2);
   return rc;
 }
@@ -389,13 +428,10 @@ static int fused_common(int qt, const void* x, const float* logits, const void* 
   int32_t* gs = (int32_t*)(ws + L.gs);
   int32_t* go = (int32_t*)(ws + L.go);
   int32_t* gpo = (int32_t*)(ws + L.gpo);
-  int32_t* istart = (int32_t*)(ws + L.istart);
   const int64_t rows = cap_rows(T, ke, Ee, block_m);
-  // (a shard's share of the pairs decides how its items are shaped; the bound
-  // on their number holds for any routing)
-  WidePlan wide = wide_plan(shard ? (T * ke * E + E_route - 1) / E_route : T * ke, Ee, H, I, qt);
-  wide.max_items = T * ke / wide.hmax + (T * ke < Ee ? T * ke : Ee);
-  const int64_t max_blocks = narrow ? rows / 32 : wide.max_items;
+  // (a shard is expected to get its share of the pairs)
+  moe::ItemPlan plan = fused_plan(T * ke, shard ? (T * ke * E + E_route - 1) / E_route : T * ke, Ee, H, I, qt);
+  if (!narrow) plan.out = (int32_t*)(ws + L.plan);
   const int e_shared = shared ? (int)E : -1;
 
   // optional stage markers: ev[0] start, [1] routed, [2] aligned, [3] x quantised,
@@ -405,14 +441,12 @@ static int fused_common(int qt, const void* x, const float* logits, const void* 
   // 8-bit operands from logits: the routing and the per-token quantisation of
   // x run as one launch (route_quant_kernel)
   const bool route_quant = w8 && !given && !w_router;
-  const int nt1 = (int)(I / moe::kBN), nt2 = (int)wide.nt2;
-  int32_t* const plan = narrow ? nullptr : istart;
   // small batches from logits: routing and alignment run as one launch
   hipError_t ra = hipSuccess;
   const bool route_align =
       !w8 && !given && !w_router &&
       moe::launch_route_align(logits, bias, (int)T, (int)E_route, (int)k, ids, wts, e_shared, (int)Ee, (int)block_m, sorted,
-                              (int32_t*)(ws + L.bexp), gs, go, gpo, s, (int)e_begin, plan, wide.hmax, nt1, nt2, &ra);
+                              (int32_t*)(ws + L.bexp), gs, go, gpo, s, (int)e_begin, plan, &ra);
   if (route_align) {
     if ((rc = check_launch(ra, "route_align"))) return rc;
   } else if (given) {
@@ -428,7 +462,7 @@ static int fused_common(int qt, const void* x, const float* logits, const void* 
   }
   mark(1);
   if (!route_align &&
-      (rc = check_launch(moe::launch_align(rids, (int)(T * ke), (int)Ee, (int)block_m, sorted, (int32_t*)(ws + L.bexp), gs, go, gpo, (int32_t*)(ws + L.whist), s, (int)e_begin, plan, wide.hmax, nt1, nt2), "align"))) return rc;
+      (rc = check_launch(moe::launch_align(rids, (int)(T * ke), (int)Ee, (int)block_m, sorted, (int32_t*)(ws + L.bexp), gs, go, gpo, (int32_t*)(ws + L.whist), s, (int)e_begin, plan), "align"))) return rc;
   mark(2);
   if (w8 && !route_quant && (rc = check_launch(moe::launch_quant_rows(x, T, H, ws + L.xq, (float*)(ws + L.sx), qt, s), "quantize_x"))) return rc;
   mark(3);
@@ -455,11 +489,12 @@ static int fused_common(int qt, const void* x, const float* logits, const void* 
   p1.E = (int)Ee;
   p1.H = H;
   p1.I = I;
-  p1.istart = istart;
-  p1.xb = istart + Ee + 1;
+  if (!narrow) {
+    p1.istart = plan.out;
+    p1.xb = plan.out + moe::ItemPlan::xb1(Ee);
+  }
   p1.rows_cap = (int)rows;
-  p1.hmax = wide.hmax;
-  if ((rc = check_launch(moe::launch_stage1(p1, narrow, qt, true, max_blocks, T * ke, s), "stage1"))) return rc;
+  if ((rc = check_launch(moe::launch_stage1(p1, narrow, qt, true, narrow ? rows / 32 : plan.slots1, s), "stage1"))) return rc;
   // int8: h (fp16) -> per-row int8 codes + scales, for the routed rows only
   // (sorted id below the sentinel T * ke, row below gpo[E])
   if (qt == moe::kQI8 &&
@@ -478,10 +513,12 @@ static int fused_common(int qt, const void* x, const float* logits, const void* 
   p2.out = MOE_S2_SCATTER ? (char*)out : ws + L.ypair;
   p2.topk = (int)ke;
   p2.pos = (int32_t*)(ws + L.pos);
-  p2.istart = istart;
-  p2.xb = istart + Ee + 10;
+  if (!narrow) {
+    p2.istart = plan.out + moe::ItemPlan::istart2(Ee);
+    p2.xb = plan.out + moe::ItemPlan::xb2(Ee);
+    p2.bn_plan = plan.out + moe::ItemPlan::bn(Ee);
+  }
   p2.rows_cap = (int)rows;
-  p2.hmax = wide.hmax;
   p2.routed = rwts;
   p2.routed_f16 = 0;
   p2.gs = gs;
@@ -496,7 +533,7 @@ static int fused_common(int qt, const void* x, const float* logits, const void* 
   p2.H = H;
   p2.I = I;
   if (MOE_S2_SCATTER && (rc = check_launch(moe::launch_zero(out, T * H * 2, s), "zero_out"))) return rc;
-  if ((rc = check_launch(moe::launch_stage2(p2, narrow, qt, true, wide.bn256, max_blocks, T * ke, s), "stage2"))) return rc;
+  if ((rc = check_launch(moe::launch_stage2(p2, narrow, qt, true, narrow ? rows / 32 : plan.slots2, s), "stage2"))) return rc;
   mark(5);
   if (MOE_S2_SCATTER) {  // Stage 2 added every pair row into `out`
     mark(6);

@@ -1108,12 +1108,13 @@ __device__ __forceinline__ void stage2_item(const Stage2Params& p, const Item& i
   }
 }
 
-template <int QT, bool FUSED, int BN>
+template <int QT, bool FUSED>
 __global__ __launch_bounds__(512) void stage2_wide_kernel(Stage2Params p) {
   __shared__ __attribute__((aligned(16))) char smem[kLdsBytes];
-  const int nt = (int)(p.H / BN);
-  auto run = [&](const Item& it) {
-    if (it.actual <= 0) return;
+  const int bn = FUSED ? *p.bn_plan : p.bn;
+  const int nt = (int)(p.H / bn);
+  auto run_bn = [&](const Item& it, auto bn_c) {
+    constexpr int BN = decltype(bn_c)::value;
     if (it.actual <= kLowRows) {
       if (it.shared) stage2_item<QT, FUSED, BN, kLowRows, false, false>(p, it, smem);
       else stage2_item<QT, FUSED, BN, kLowRows, false, true>(p, it, smem);
@@ -1125,16 +1126,22 @@ __global__ __launch_bounds__(512) void stage2_wide_kernel(Stage2Params p) {
       else stage2_item<QT, FUSED, BN, kWideRows, true, true>(p, it, smem);
     }
   };
+  auto run = [&](const Item& it) {
+    if (it.actual <= 0) return;
+    if (bn == 256) run_bn(it, std::integral_constant<int, 256>{});
+    else run_bn(it, std::integral_constant<int, 128>{});
+  };
   Item it;
   if constexpr (FUSED) {
-    if (item_fused(blockIdx.x, p.istart, p.xb, p.gs, p.gpo, p.E, BN, nt, p.rows_cap, it)) run(it);
+    if (item_fused(blockIdx.x, p.istart, p.xb, p.gs, p.gpo, p.E, bn, nt, p.rows_cap, it)) run(it);
   } else {
-    if (!item_bx(blockIdx.x, p.gidx, p.host_blocks, p.E, BN, nt, p.gs, p.gpo, p.hmax, gridDim.x, smem, it)) return;
+    if (!item_bx(blockIdx.x, p.gidx, p.host_blocks, p.E, bn, nt, p.gs, p.gpo, p.hmax, gridDim.x, smem, it)) return;
     // Rows owned by no valid token are written as 0 (problem_detail.json:50 note 4).
     _Float16* o = reinterpret_cast<_Float16*>(p.out);
     const int rows = it.zero_end - (it.row0 + it.actual);
-    for (int idx = threadIdx.x; idx < rows * (BN / 8); idx += 512) {
-      const int r = it.row0 + it.actual + idx / (BN / 8), c = idx % (BN / 8);
+    const int shift = bn == 256 ? 5 : 4;  // 16-byte chunks per row
+    for (int idx = threadIdx.x; idx < rows << shift; idx += 512) {
+      const int r = it.row0 + it.actual + (idx >> shift), c = idx & ((1 << shift) - 1);
       *reinterpret_cast<u32x4*>(o + (int64_t)r * p.H + it.n0 + 8 * c) = u32x4{0, 0, 0, 0};
     }
     run(it);
@@ -1169,31 +1176,30 @@ static hipError_t go1_narrow(const Stage1Params& p, int64_t max_blocks, hipStrea
   }
   return hipGetLastError();
 }
-static int64_t wide_grid(bool fused, int64_t pieces, int64_t rows, int64_t nt, int hmax) {
+static int64_t wide_grid(bool fused, int64_t max_blocks, int64_t nt, int hmax) {
   // pre-routed, where item_bx may cut by cost: an eighth more than an equal cut needs, so that a cut by cost
   // fits.  H 7168, I 2048, 64 experts, 9000 rows 1523 -> 1420 us; the surplus workgroups cost even
   // groupings 1-4% (376 -> 390, 632 -> 639, 1233 -> 1241 us).
-  return fused ? kNumXcd * xcd_items_bound(pieces, rows, nt) : schedule_grid(pieces + (hmax > kLowRows ? (pieces + 7) / 8 : 0), nt);
+  return fused ? kNumXcd * max_blocks : schedule_grid(max_blocks + (hmax > kLowRows ? (max_blocks + 7) / 8 : 0), nt);
 }
 template <int QT>
-static hipError_t go1(const Stage1Params& p, bool gather, int64_t max_blocks, int64_t max_rows, hipStream_t s) {
-  const dim3 grid((unsigned)wide_grid(gather, max_blocks, max_rows, p.I / kBN, p.hmax));
+static hipError_t go1(const Stage1Params& p, bool gather, int64_t max_blocks, hipStream_t s) {
+  const dim3 grid((unsigned)wide_grid(gather, max_blocks, p.I / kBN, p.hmax));
   if (gather) hipLaunchKernelGGL((stage1_wide_kernel<QT, true>), grid, dim3(512), 0, s, p);
   else if constexpr (QT == kQF16) hipLaunchKernelGGL((stage1_wide_kernel<QT, false>), grid, dim3(512), 0, s, p);
   else return hipErrorInvalidValue;
   return hipGetLastError();
 }
-template <int QT, int BN>
-static hipError_t go2(const Stage2Params& p, bool fused, int64_t max_blocks, int64_t max_rows, hipStream_t s) {
-  const dim3 grid((unsigned)wide_grid(fused, max_blocks, max_rows, p.H / BN, p.hmax));
-  if (fused) hipLaunchKernelGGL((stage2_wide_kernel<QT, true, BN>), grid, dim3(512), 0, s, p);
-  else if constexpr (QT == kQF16) hipLaunchKernelGGL((stage2_wide_kernel<QT, false, BN>), grid, dim3(512), 0, s, p);
+template <int QT>
+static hipError_t go2(const Stage2Params& p, bool fused, int64_t max_blocks, hipStream_t s) {
+  const dim3 grid((unsigned)wide_grid(fused, max_blocks, p.H / (fused ? kBN : p.bn), p.hmax));
+  if (fused) hipLaunchKernelGGL((stage2_wide_kernel<QT, true>), grid, dim3(512), 0, s, p);
+  else if constexpr (QT == kQF16) hipLaunchKernelGGL((stage2_wide_kernel<QT, false>), grid, dim3(512), 0, s, p);
   else return hipErrorInvalidValue;
   return hipGetLastError();
 }
 
-hipError_t launch_stage1(const Stage1Params& params, bool narrow, int qt, bool gather, int64_t max_blocks,
-                         int64_t max_rows, hipStream_t s) {
+hipError_t launch_stage1(const Stage1Params& params, bool narrow, int qt, bool gather, int64_t max_blocks, hipStream_t s) {
   Stage1Params p = params;
   p.host_blocks = (int)max_blocks;
   if (p.w_ld == 0) p.w_ld = p.H * (qt != kQF16 ? 1 : 2);
@@ -1205,20 +1211,12 @@ hipError_t launch_stage1(const Stage1Params& params, bool narrow, int qt, bool g
     return qt == kQF8 ? go1_narrow<kQF8>(p, max_blocks, s)
                       : (qt == kQI8 ? go1_narrow<kQI8>(p, max_blocks, s) : go1_narrow<kQF16>(p, max_blocks, s));
   }
-  return qt == kQF8 ? go1<kQF8>(p, gather, max_blocks, max_rows, s)
-                    : (qt == kQI8 ? go1<kQI8>(p, gather, max_blocks, max_rows, s) : go1<kQF16>(p, gather, max_blocks, max_rows, s));
+  return qt == kQF8 ? go1<kQF8>(p, gather, max_blocks, s)
+                    : (qt == kQI8 ? go1<kQI8>(p, gather, max_blocks, s) : go1<kQF16>(p, gather, max_blocks, s));
 }
 
-// Stage 2's K loop is short (I / 64 steps), so its items take 256 features
-// when H allows and the launch still has an item per CU: half the re-reads of
-// the intermediate and twice the work behind each item's fill and epilogue.
-template <int QT>
-static hipError_t go2_wide(const Stage2Params& p, bool fused, bool bn256, int64_t mb, int64_t max_rows, hipStream_t s) {
-  return bn256 ? go2<QT, 256>(p, fused, mb, max_rows, s) : go2<QT, 128>(p, fused, mb, max_rows, s);
-}
-
-hipError_t launch_stage2(const Stage2Params& params, bool narrow, int qt, bool fused, bool bn256,
-                         int64_t max_blocks, int64_t max_rows, hipStream_t s) {
+hipError_t launch_stage2(const Stage2Params& params, bool narrow, int qt, bool fused,
+                         int64_t max_blocks, hipStream_t s) {
   Stage2Params p = params;
   p.host_blocks = (int)max_blocks;
   if (p.a_ld == 0) p.a_ld = p.I * (qt != kQF16 ? 1 : 2);
@@ -1233,9 +1231,9 @@ hipError_t launch_stage2(const Stage2Params& params, bool narrow, int qt, bool f
     else hipLaunchKernelGGL((stage2_narrow_kernel<MOE_S2N_STAGES, kQF16>), grid, dim3(256), 0, s, p);
     return hipGetLastError();
   }
-  return qt == kQF8 ? go2_wide<kQF8>(p, fused, bn256, max_blocks, max_rows, s)
-                    : (qt == kQI8 ? go2_wide<kQI8>(p, fused, bn256, max_blocks, max_rows, s)
-                                  : go2_wide<kQF16>(p, fused, bn256, max_blocks, max_rows, s));
+  if (!fused && p.bn != 128 && (p.bn != 256 || p.H % 256)) return hipErrorInvalidValue;
+  return qt == kQF8 ? go2<kQF8>(p, fused, max_blocks, s)
+                    : (qt == kQI8 ? go2<kQI8>(p, fused, max_blocks, s) : go2<kQF16>(p, fused, max_blocks, s));
 }
 
 }  // namespace moe

@@ -24,6 +24,29 @@ namespace moe {
 // accumulation).
 enum QuantType : int { kQF16 = 0, kQI8 = 1, kQF8 = 2 };
 
+// The wide items of a fused launch (moe_common.h Item) are planned by align from
+// the routed rows themselves: the height of each stage's tallest item, and how
+// many features Stage 2's take.  A launch of few rounds ends when its slowest
+// CU does, which depends on how the counts fall: 16 experts of H 4096, I 2048 at
+// 1500 tokens top-2 with Zipf popularity ran Stage 1 in 217 us in items of up to
+// 288 rows, 182 in 128 and 168 in 192, and 138, 142 and 128 (224 rows) on an even
+// routing.  `out`, int32: [E+1] items per N tile below each expert for Stage 1,
+// [E+1] for Stage 2, the 9 XCD bounds of each, Stage 2's features per item.
+struct ItemPlan {
+  int32_t* out = nullptr;  // null: no plan
+  int tall = 0;            // rows of the tallest item
+  int nt1 = 0, nt2 = 0;    // N tiles of Stage 1, and of Stage 2 at 128 features
+  bool any1 = false, any2 = false;  // may take shorter items (moe_common.h plan_height)
+  int bn2 = 0;             // Stage 2's features per item: 128, 256 or either (0)
+  int slots1 = 0, slots2 = 0;  // workgroups of each stage's launch per XCD: what a choice has to fit in
+
+  static constexpr int64_t ints(int64_t E) { return 2 * E + 21; }
+  static constexpr int64_t istart2(int64_t E) { return E + 1; }
+  static constexpr int64_t xb1(int64_t E) { return 2 * E + 2; }
+  static constexpr int64_t xb2(int64_t E) { return 2 * E + 11; }
+  static constexpr int64_t bn(int64_t E) { return 2 * E + 20; }
+};
+
 // Stage 1: h = silu(X Wg^T) * (X Wu^T) for the rows of every M block.
 struct Stage1Params {
   const char* x;            // fp16 [rows, H] (direct) / fp16|int8 [T, H] (gather)
@@ -54,7 +77,7 @@ struct Stage1Params {
   const int32_t* istart = nullptr;  // wide, gather: [E+1] items per N tile below each expert
   const int32_t* xb = nullptr;      // wide, gather: [9] first item of each XCD
   int rows_cap = 0;         // wide, gather: rows the buffers hold
-  int hmax = 0;             // wide: most rows of an item (moe_common.h Item)
+  int hmax = 0;             // wide, direct: most rows of an item (moe_common.h Item)
 };
 
 // Stage 2: y = h Wd^T, scaled by the routing weight of each row.
@@ -87,6 +110,8 @@ struct Stage2Params {
   int host_blocks;          // as Stage 1's
   const int32_t* istart = nullptr;
   const int32_t* xb = nullptr;
+  const int32_t* bn_plan = nullptr;  // wide, fused: features of an item, 128 or 256 (the plan's)
+  int bn = 0;               // wide, pre-routed: features of an item, 128 or 256
   int rows_cap = 0;
   int hmax = 0;
   int topk = 0;             // fused, built with MOE_S2_SCATTER: choices per token; `out` is then
@@ -99,14 +124,12 @@ struct Stage2Params {
 hipError_t launch_zero(void* p, int64_t n, hipStream_t stream);
 
 // qt: a QuantType.  narrow: 32-row items over rows padded to 32 (gather / fused
-// only); otherwise wide items.  max_blocks: an upper bound on the items per N
-// tile (narrow: 32-row blocks; wide: row pieces; direct: 128-row blocks);
-// max_rows: of the routed rows (wide).
-// bn256: Stage 2's wide items take 256 features where H allows.
+// only); otherwise wide items.  max_blocks: narrow, 32-row blocks of the launch
+// at most; wide, the plan's slots (gather / fused) or 128-row blocks (pre-routed).
 hipError_t launch_stage1(const Stage1Params& p, bool narrow, int qt, bool gather,
-                         int64_t max_blocks, int64_t max_rows, hipStream_t stream);
-hipError_t launch_stage2(const Stage2Params& p, bool narrow, int qt, bool fused, bool bn256,
-                         int64_t max_blocks, int64_t max_rows, hipStream_t stream);
+                         int64_t max_blocks, hipStream_t stream);
+hipError_t launch_stage2(const Stage2Params& p, bool narrow, int qt, bool fused,
+                         int64_t max_blocks, hipStream_t stream);
 
 // With e_shared >= 0 every token also gets the shared expert as choice k
 // (id e_shared, weight 1): ids / w rows hold k + 1 entries.
@@ -127,20 +150,16 @@ inline int align_pairs_per_group(int P, int groups, int nw) {
   return (per + 64 * nw - 1) / (64 * nw) * (64 * nw);
 }
 // e_off: pairs are bucketed by id - e_off; ids outside [e_off, e_off + E)
-// are dropped (an expert shard of a wider routing).  With `istart` (int32
-// [E + 1], may be null) the items of hmax rows per N tile below each expert
-// are written there (moe_common.h Item), and behind it, at istart + E + 1, the 9
-// XCD bounds of Stage 1's items (nt1 N tiles) and the 9 of Stage 2's (nt2).
+// are dropped (an expert shard of a wider routing).  With `plan.out` the wide
+// items' plan is written there (moe_common.h ItemPlan).
 hipError_t launch_align(const int32_t* ids, int P, int E, int BM, int32_t* sorted_ids,
                         int32_t* block_expert, int32_t* gs, int32_t* go, int32_t* gpo,
-                        int32_t* whist, hipStream_t stream, int e_off = 0, int32_t* istart = nullptr,
-                        int hmax = 1, int nt1 = 0, int nt2 = 0);
+                        int32_t* whist, hipStream_t stream, int e_off = 0, const ItemPlan& plan = ItemPlan{});
 // launch_route_topk and launch_align in one launch, for small batches (see
 // route_align_kernel); false, with nothing launched, for others.
 bool launch_route_align(const float* logits, const float* bias, int T, int E_route, int k, int32_t* ids, float* w,
                         int e_shared, int E, int BM, int32_t* sorted_ids, int32_t* block_expert, int32_t* gs,
-                        int32_t* go, int32_t* gpo, hipStream_t stream, int e_off, int32_t* istart, int hmax, int nt1,
-                        int nt2, hipError_t* err);
+                        int32_t* go, int32_t* gpo, hipStream_t stream, int e_off, const ItemPlan& plan, hipError_t* err);
 // Router GEMM (x . w_router^T, K split in router_splits parts) + routing of
 // the summed partials; `part` holds router_partial_floats fp32, `logits`
 // (fp32 [T, E]) may be null.

@@ -372,15 +372,20 @@ __device__ __forceinline__ bool schedule(int g, const int32_t* __restrict__ gpo,
 // 638 us, 64 of 20 but 10 of 300 1180 -> 1203.
 // All items span the whole N tile; item v of expert e is
 // N tile (v - first) / c, row piece (v - first) % c, so the c items reading one
-// weight tile are adjacent.  hmax is kTallRows where the tiles take absorbed
-// rows (moe_common.h kAbsorbRows), kWideRows otherwise, and kLowRows where the
-// launch would have fewer items than the chip has CUs.
+// weight tile are adjacent.  hmax is kTallRows at most where the tiles take
+// absorbed rows (kAbsorbRows), kWideRows otherwise; shorter where that ends a
+// launch of few rounds earlier (fused: launch.h ItemPlan; run_kernel: capi.hip).
 constexpr int kLowRows = 128, kWideRows = 256;
 constexpr int kAbsorbRows = 32;  // rows past kWideRows that an item takes along
 constexpr int kTallRows = kWideRows + kAbsorbRows;
 
 __host__ __device__ inline int items_of(int n, int hmax) { return (n + hmax - 1) / hmax; }
 __device__ __forceinline__ int rows_of(int n, int c) { return (n + 32 * c - 1) / (32 * c) * 32; }
+
+// The heights that a plan chooses from: the tallest, 256, 224, .., 128.
+constexpr int kPlanHeights = 6;
+__device__ __forceinline__ int plan_height(int j, int tall) { return j == 0 ? tall : kWideRows - 32 * (j - 1); }
+static_assert(kWideRows - 32 * (kPlanHeights - 2) == kLowRows, "the shortest is the one the host's bounds assume");
 
 struct Item {
   int e;         // expert, or -1 (rows owned by no expert)
@@ -457,31 +462,45 @@ __device__ __forceinline__ XcdCut xcd_cut(int x, bool weighted, const int* ist, 
   }
   return r;
 }
-// Both cuts of one launch on lanes 0..8 (equal numbers) and 9..17 (equal cost)
-// of a wave, and the better one written to xb[0..8]: the one whose slowest XCD
-// needs less time, an XCD running its items kCusPerXcd at a time.  Equal cost
-// pays where experts differ and there are many rounds; with two rounds of like
-// items it would leave some XCD a third.  slots: workgroups an XCD has in the
-// launch; an equal cut always fits.
+// Both cuts of a launch's items on 18 lanes of a wave -- lanes 0..8 of them equal
+// numbers, 9..17 equal cost; up to three launches at once, one per 18 lanes --
+// and the better one: the one whose slowest XCD needs less time, an XCD running
+// its items kCusPerXcd at a time.  Equal cost pays where experts differ and
+// there are many rounds; with two rounds of like items it would leave some XCD a
+// third.  slots: workgroups an XCD has in the launch, which a cut has to fit in.
 constexpr int kCusPerXcd = 32;
-__device__ __forceinline__ void xcd_shares(const int* ist, const int* gof, int E, int nt, int32_t* xb,
-                                           int slots = 0x7fffffff) {
-  const int l = lane_id();
-  const int x = l % 9;
+struct XcdPick {
+  int item;     // first item of XCD (lane % 18) % 9
+  bool chosen;  // this lane's cut is the better one
+  float slow;   // its slowest XCD's time, in rows of cost; INFINITY: neither fits
+};
+__device__ __forceinline__ XcdPick xcd_pick(const int* ist, const int* gof, int E, int nt, bool active, int slots) {
+  const int l = lane_id(), q = l % 18, base = l - q, x = q % 9;
   XcdCut cut = {0, 0.0};
-  if (l < 18) cut = xcd_cut(x, l >= 9, ist, gof, E, nt);
+  if (active) cut = xcd_cut(x, q >= 9, ist, gof, E, nt);
   const int items = __shfl_down(cut.item, 1) - cut.item;
   const float cost = __shfl_down((float)cut.cost, 1) - (float)cut.cost;
   float t = 0.0f;
-  if (l < 18 && x < 8 && items > 0) t = (float)((items + kCusPerXcd - 1) / kCusPerXcd) * cost / (float)items;
-  float slow[2] = {0.0f, 0.0f};
-  for (int q = 0; q < 18; ++q) slow[q / 9] = fmaxf(slow[q / 9], __shfl(t, q));
-  const bool fits = __ballot(l >= 9 && l < 17 && items > slots) == 0;
-  const bool weighted = fits && slow[1] < slow[0];
-  if (l < 18 && (l >= 9) == weighted) xb[x] = cut.item;
+  if (active && x < 8 && items > 0) t = (float)((items + kCusPerXcd - 1) / kCusPerXcd) * cost / (float)items;
+  float equal = 0.0f, weighted = 0.0f;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    equal = fmaxf(equal, __shfl(t, base + j));
+    weighted = fmaxf(weighted, __shfl(t, base + 9 + j));
+  }
+  const uint64_t over = __ballot(active && x < 8 && items > slots) >> base;
+  if (over & 0x1ff) equal = INFINITY;
+  if (over & 0x3fe00) weighted = INFINITY;
+  const bool take = weighted < equal;
+  return XcdPick{cut.item, active && (q >= 9) == take, take ? weighted : equal};
 }
-// An upper bound on an XCD's items either way, for `pieces` items per N tile and
-// `rows` routed rows in all.
+// xb[0..8]: the better cut of one launch.
+__device__ __forceinline__ void xcd_shares(const int* ist, const int* gof, int E, int nt, int32_t* xb, int slots) {
+  const XcdPick p = xcd_pick(ist, gof, E, nt, lane_id() < 18, slots);
+  if (p.chosen) xb[lane_id() % 9] = p.item;
+}
+// An upper bound on an XCD's items with either cut, for `pieces` items per N tile
+// and `rows` routed rows in all.
 inline int64_t xcd_items_bound(int64_t pieces, int64_t rows, int64_t nt) {
   return (pieces * kItemCost + rows) * nt / (kNumXcd * kItemCost) + 2;
 }

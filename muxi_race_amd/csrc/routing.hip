@@ -118,23 +118,13 @@ __device__ __forceinline__ void align_place_range(const int32_t* __restrict__ id
   }
 }
 
-// The wide items' plan: see launch_align.  A workgroup of its own, the launch's
-// last, counts and scans as the others do and writes it (3 us of one wave's
-// work, which would otherwise end the launch).
-struct ItemPlan {
-  int32_t* istart;
-  int hmax, nt1, nt2;
-};
-
 // Expert scan by one wave: tot[E] -> padded offsets pstart[E+1] in LDS, and
-// (when `out`) group sizes / offsets / padded offsets, and (when `plan`) the wide
-// items' plan, in global memory.  ist, gof: [E+1] ints of LDS each.
+// (when `out`) group sizes / offsets / padded offsets in global memory.
 __device__ __forceinline__ void align_expert_scan(const int* tot, int E, int BM, int* pstart, bool out,
                                                   int32_t* __restrict__ gs, int32_t* __restrict__ go,
-                                                  int32_t* __restrict__ gpo, const ItemPlan* plan = nullptr,
-                                                  int* ist = nullptr, int* gof = nullptr) {
+                                                  int32_t* __restrict__ gpo) {
   const int l = lane_id();
-  int carry = 0, carry_p = 0, carry_i = 0;
+  int carry = 0, carry_p = 0;
   for (int base = 0; base < E; base += 64) {
     const int e = base + l;
     const int c = e < E ? tot[e] : 0;
@@ -148,14 +138,6 @@ __device__ __forceinline__ void align_expert_scan(const int* tot, int E, int BM,
         gpo[e] = carry_p + ip - pc;
       }
     }
-    if (plan) {
-      const int ni = items_of(c, plan->hmax), ii = wave_inclusive_scan(ni);
-      if (e < E) {
-        plan->istart[e] = ist[e] = carry_i + ii - ni;
-        gof[e] = carry + ic - c;
-      }
-      carry_i += __builtin_amdgcn_readlane(ii, 63);
-    }
     carry += __builtin_amdgcn_readlane(ic, 63);
     carry_p += __builtin_amdgcn_readlane(ip, 63);
   }
@@ -166,16 +148,78 @@ __device__ __forceinline__ void align_expert_scan(const int* tot, int E, int BM,
       gpo[E] = carry_p;
     }
   }
-  if (plan) {
-    if (l == 0) {
-      plan->istart[E] = ist[E] = carry_i;
-      gof[E] = carry;
-    }
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");  // this wave's LDS writes, before other lanes read them
-    xcd_shares(ist, gof, E, plan->nt1, plan->istart + E + 1);
-    xcd_shares(ist, gof, E, plan->nt2, plan->istart + E + 10);
-  }
 }
+
+// The wide items' plan (launch.h ItemPlan) from the routed rows tot[E], by a
+// workgroup of its own, the launch's last, which counts as the others do (a few
+// us of serial work that would otherwise end the launch).  Wave j scans the
+// items of height j and weighs the launches that may use it -- Stage 1, Stage 2
+// with 256 features, with 128 -- on 18 lanes each; the fastest of a stage is
+// written.  A 128-feature item is taken to cost kHalfTile of a 256-feature one:
+// half the weight rows, the same token rows.  Over 456 cases that run wide items
+// (9 layers of 8 to 128 experts, 200 to 4096 tokens, even and Zipf routing, each
+// format) the choice is 1% slower on average than the best height and width
+// measured, and the rules before it (tallest, or 128 rows where that left CUs
+// without an item; 256 features where that gave every CU one) 6% in Stage 1 and
+// 8% in Stage 2, 55% at most.
+// sm: plan_lds_ints(E) of LDS.
+constexpr float kHalfTile = 0.7f;
+constexpr int kPlanLaunches = 3 * kPlanHeights;
+__host__ __device__ inline int plan_lds_ints(int E) { return (kPlanHeights + 1) * (E + 1) + 10 * kPlanLaunches; }
+__device__ void item_plan(const int* tot, int E, const ItemPlan& p, int* sm) {
+  const int tid = threadIdx.x, w = wave_id(), l = lane_id();
+  int* ist = sm;                             // [kPlanHeights][E+1]
+  int* gof = sm + kPlanHeights * (E + 1);    // [E+1] rows below each expert
+  int* xbs = gof + E + 1;                    // [kPlanLaunches][9]
+  float* est = reinterpret_cast<float*>(xbs + 9 * kPlanLaunches);  // [kPlanLaunches]
+  const int nh = p.any1 || p.any2 ? kPlanHeights : 1;
+  int* mine = ist + (w < nh ? w : 0) * (E + 1);
+  if (w < nh) {
+    int items = 0, rows = 0;
+    for (int base = 0; base < E; base += 64) {
+      const int e = base + l;
+      const int c = e < E ? tot[e] : 0, ni = items_of(c, plan_height(w, p.tall));
+      const int ii = wave_inclusive_scan(ni), ir = wave_inclusive_scan(c);
+      if (e < E) {
+        mine[e] = items + ii - ni;
+        if (w == 0) gof[e] = rows + ir - c;
+      }
+      items += __builtin_amdgcn_readlane(ii, 63);
+      rows += __builtin_amdgcn_readlane(ir, 63);
+    }
+    if (l == 0) {
+      mine[E] = items;
+      if (w == 0) gof[E] = rows;
+    }
+  }
+  __syncthreads();
+  if (w < nh) {
+    const int k = l / 18;  // 0: Stage 1, 1: Stage 2 with 256 features, 2: with 128
+    const bool may = k == 0 ? w == 0 || p.any1 : (w == 0 || p.any2) && p.bn2 != (k == 1 ? 128 : 256);
+    const int nt = k == 0 ? p.nt1 : (k == 1 ? p.nt2 / 2 : p.nt2);
+    const XcdPick pick = xcd_pick(mine, gof, E, nt, k < 3 && may, k == 0 ? p.slots1 : p.slots2);
+    if (pick.chosen) xbs[9 * (3 * w + k) + l % 18 % 9] = pick.item;
+    if (k < 3 && l % 18 == 0) est[3 * w + k] = may ? pick.slow * (k == 2 ? kHalfTile : 1.0f) : INFINITY;
+  }
+  __syncthreads();
+  int s1 = 0, s2 = p.bn2 == 128 ? 2 : 1;
+  for (int j = 0; j < nh; ++j) {
+    if (est[3 * j] < est[s1]) s1 = 3 * j;
+    for (int k = 1; k < 3; ++k)
+      if (est[3 * j + k] < est[s2]) s2 = 3 * j + k;
+  }
+  for (int e = tid; e <= E; e += blockDim.x) {
+    p.out[e] = ist[s1 / 3 * (E + 1) + e];
+    p.out[ItemPlan::istart2(E) + e] = ist[s2 / 3 * (E + 1) + e];
+  }
+  if (tid < 9) {
+    p.out[ItemPlan::xb1(E) + tid] = xbs[9 * s1 + tid];
+    p.out[ItemPlan::xb2(E) + tid] = xbs[9 * s2 + tid];
+  }
+  if (tid == 0) p.out[ItemPlan::bn(E)] = s2 % 3 == 1 ? 256 : 128;
+}
+// LDS of item_plan: over the NW histograms, which it no longer needs, where those are as large; else at `end`.
+__host__ __device__ inline bool plan_over_hist(int nw, int E) { return nw * E >= plan_lds_ints(E); }
 
 // padding rows of experts e0, e0 + step, ... -> sentinel P; their blocks ->
 // owning expert (rows disjoint from the placed ones); by one wave
@@ -211,8 +255,7 @@ __device__ __forceinline__ void align_small(
   int* hist = sm;                 // [NW][E]: wave w's count of expert e, then its first row among e's
   int* tot = sm + NW * E;         // [E]
   int* pstart = tot + E;          // [E+1] padded offsets
-  int* ist = pstart + E + 1;      // [E+1], with an item plan only
-  int* gof = ist + E + 1;         // [E+1]
+  int* plan_sm = plan_over_hist(NW, E) ? hist : pstart + E + 1;
   const int tid = threadIdx.x, w = tid >> 6, l = lane_id();
   const int nbits = bits_for(E);
   const int R = ((P + NW - 1) / NW + 63) / 64 * 64;  // <= 64 * kAlignUnroll (launch_align checks)
@@ -255,12 +298,11 @@ __device__ __forceinline__ void align_small(
     tot[e] = run;
   }
   __syncthreads();
-  const bool planner = blockIdx.x > 0;
-  if (w == 0) {
-    if (planner) align_expert_scan(tot, E, BM, pstart, false, gs, go, gpo, &plan, ist, gof);
-    else align_expert_scan(tot, E, BM, pstart, true, gs, go, gpo);
+  if (blockIdx.x > 0) {
+    item_plan(tot, E, plan, plan_sm);
+    return;
   }
-  if (planner) return;
+  if (w == 0) align_expert_scan(tot, E, BM, pstart, true, gs, go, gpo);
   __syncthreads();
   const int rows = pstart[E];
   for (int r = tid; r < rows; r += 64 * NW) sorted_ids[r] = P;
@@ -316,15 +358,18 @@ __global__ __launch_bounds__(1024) void route_align_kernel(
   align_small<16>(lids, P, E, e_off, BM, sorted_ids, block_expert, gs, go, gpo, plan, sm + 2 * P);
 }
 
+// LDS bytes that a launch of nw waves adds for the plan.
+static size_t plan_extra_lds(const ItemPlan& plan, int nw, int E) {
+  return plan.out && !plan_over_hist(nw, E) ? sizeof(int) * (size_t)plan_lds_ints(E) : 0;
+}
+
 bool launch_route_align(const float* logits, const float* bias, int T, int E_route, int k, int32_t* ids, float* w,
                         int e_shared, int E, int BM, int32_t* sorted_ids, int32_t* block_expert, int32_t* gs,
-                        int32_t* go, int32_t* gpo, hipStream_t s, int e_off, int32_t* istart, int hmax, int nt1,
-                        int nt2, hipError_t* err) {
+                        int32_t* go, int32_t* gpo, hipStream_t s, int e_off, const ItemPlan& plan, hipError_t* err) {
   const int kout = e_shared >= 0 ? k + 1 : k, P = T * kout;
   if (E_route > 16 || T > kRouteAlignTokens) return false;
-  const ItemPlan plan{istart, hmax, nt1, nt2};
-  const dim3 grid(istart ? 2 : 1), block(1024);
-  const size_t lds = sizeof(int) * (2 * (size_t)P + 16 * (size_t)E + 2 * (size_t)E + 1 + (istart ? 2 * ((size_t)E + 1) : 0));
+  const dim3 grid(plan.out ? 2 : 1), block(1024);
+  const size_t lds = sizeof(int) * (2 * (size_t)P + 16 * (size_t)E + 2 * (size_t)E + 1) + plan_extra_lds(plan, 16, E);
 #define MOE_RA(L) hipLaunchKernelGGL((route_align_kernel<L>), grid, block, lds, s, logits, bias, T, E_route, k, ids, w, \
                                      e_shared, E, e_off, BM, sorted_ids, block_expert, gs, go, gpo, plan)
   if (E_route <= 8) MOE_RA(8);
@@ -346,8 +391,7 @@ __global__ __launch_bounds__(64 * NW) void align_kernel(
   int* hist = sm;                 // [NW][E]
   int* tot = sm + NW * E;         // [E]
   int* pstart = tot + E;          // [E+1] padded offsets
-  int* ist = pstart + E + 1;      // [E+1], with an item plan only
-  int* gof = ist + E + 1;         // [E+1]
+  int* plan_sm = plan_over_hist(NW, E) ? hist : pstart + E + 1;
   const int tid = threadIdx.x, w = tid >> 6;
   const int nbits = bits_for(E);
   const int R = ((P + NW - 1) / NW + 63) / 64 * 64;
@@ -365,12 +409,11 @@ __global__ __launch_bounds__(64 * NW) void align_kernel(
     tot[e] = run;
   }
   __syncthreads();
-  const bool planner = blockIdx.x > 0;
-  if (w == 0) {
-    if (planner) align_expert_scan(tot, E, BM, pstart, false, gs, go, gpo, &plan, ist, gof);
-    else align_expert_scan(tot, E, BM, pstart, true, gs, go, gpo);
+  if (blockIdx.x > 0) {
+    item_plan(tot, E, plan, plan_sm);
+    return;
   }
-  if (planner) return;
+  if (w == 0) align_expert_scan(tot, E, BM, pstart, true, gs, go, gpo);
   __syncthreads();
   for (int e = tid; e < E; e += 64 * NW)
     for (int v = 0; v < NW; ++v) hist[v * E + e] += pstart[e];
@@ -412,10 +455,9 @@ __global__ __launch_bounds__(64 * NW) void align_place_kernel(
   int* tot = sm + NW * E;         // [E]
   int* pstart = tot + E;          // [E+1]
   int* before = pstart + E + 1;   // [E] pairs of expert e in the workgroups before this one
-  int* ist = before + E;          // [E+1], with an item plan only
-  int* gof = ist + E + 1;         // [E+1]
+  int* plan_sm = plan_over_hist(NW, E) ? hist : before + E;
   const int tid = threadIdx.x, w = tid >> 6;
-  const int G = gridDim.x - (plan.istart ? 1 : 0), g = blockIdx.x;  // g == G: the plan's workgroup
+  const int G = gridDim.x - (plan.out ? 1 : 0), g = blockIdx.x;  // g == G: the plan's workgroup
   // Every workgroup's count of expert e, loaded kBatch at a time before any is
   // added, so one load latency is exposed per batch rather than per workgroup.
   constexpr int kBatch = 16;
@@ -441,11 +483,11 @@ __global__ __launch_bounds__(64 * NW) void align_place_kernel(
   int* hw = hist + w * E;
   align_count_range(ids, p0, p1, E, e_off, nbits, hw);
   __syncthreads();
-  if (w == 0) {
-    if (g == G) align_expert_scan(tot, E, BM, pstart, false, gs, go, gpo, &plan, ist, gof);
-    else align_expert_scan(tot, E, BM, pstart, g == 0, gs, go, gpo);
+  if (g == G) {
+    item_plan(tot, E, plan, plan_sm);
+    return;
   }
-  if (g == G) return;
+  if (w == 0) align_expert_scan(tot, E, BM, pstart, g == 0, gs, go, gpo);
   __syncthreads();
   for (int e = tid; e < E; e += 64 * NW) {
     int run = pstart[e] + before[e];
@@ -462,14 +504,12 @@ __global__ __launch_bounds__(64 * NW) void align_place_kernel(
 
 hipError_t launch_align(const int32_t* ids, int P, int E, int BM, int32_t* sorted_ids,
                         int32_t* block_expert, int32_t* gs, int32_t* go, int32_t* gpo,
-                        int32_t* whist, hipStream_t s, int e_off, int32_t* istart, int hmax,
-                        int nt1, int nt2) {
-  const ItemPlan plan{istart, hmax, nt1, nt2};
-  const unsigned extra = istart ? 1 : 0;  // the plan's workgroup
-  const size_t lds_plan = istart ? 2 * sizeof(int) * ((size_t)E + 1) : 0;
+                        int32_t* whist, hipStream_t s, int e_off, const ItemPlan& plan) {
+  const unsigned extra = plan.out ? 1 : 0;  // the plan's workgroup
   // 16 waves while the histograms fit 48 KiB of LDS, else 8 (E <= 1024)
   const bool w16 = 16 * E <= 12288;
   const int nw = w16 ? 16 : 8;
+  const size_t lds_plan = plan_extra_lds(plan, nw, E);
   const int per_wave = (P + nw - 1) / nw;  // pairs per wave in one workgroup
   if (per_wave <= 64 * kAlignUnroll) {  // one workgroup, each wave's pairs held in registers
     const size_t lds = sizeof(int) * (nw * (size_t)E + 2 * (size_t)E + 1) + lds_plan;
