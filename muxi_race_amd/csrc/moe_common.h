@@ -101,7 +101,6 @@ __device__ __forceinline__ void barrier_no_fence() {
 #endif
 constexpr int kPolicyDefault = 0;
 constexpr int kPolicyWeights = MOE_W_POLICY;
-constexpr int kNoStream = 1 << 30;  // `weights_from` that streams no row
 
 // global_load_lds_dword[x4]: per-lane global address -> LDS at m0 + 4|16 * lane,
 // cache policy POLICY.  The host compilation pass only needs kernel
@@ -142,22 +141,21 @@ struct DmaTile {
   }
   // rowp: address of K-step 0 of tile row row_of(i).
   __device__ __forceinline__ void set(int i, const char* rowp) { src[i] = at(row_of(i), rowp); }
+  // STREAM: tile rows from FROM on under the streaming weight policy.  Both are
+  // known at compile time: chosen at run time, the policy costs two branches per
+  // instruction, which one wave per SIMD does not hide (Stage 2 of 32-row tiles at
+  // one token, 8 experts top-2, H 4096, I 14336: fp8 52.0 -> 44.5 us, int8 50.1 ->
+  // 41.6; int8 Stage 1 at 24 tokens, 64 experts top-6, H 7168, I 2048: 249 -> 246).
+  // PART of PARTS: that share of the instructions.
+  template <bool STREAM = false, int FROM = 0, int PART = 0, int PARTS = 1>
   __device__ __forceinline__ void issue(char* lds, int ks) const {
+    static_assert(FROM % (8 * NW) == 0, "an instruction's rows have one policy");
     const int w = wave_id();
 #pragma unroll
-    for (int i = 0; i < NI; ++i) dma_to_lds<16>(src[i] + (size_t)ks * kRowBytes, lds + 1024 * (NW * i + w));
-  }
-  // As issue(), with tile rows from `weights_from` on loaded under the
-  // streaming weight policy (kNoStream: none); an instruction's 8 rows never
-  // straddle that boundary when it is a multiple of 8, so the choice is
-  // wave-uniform.
-  __device__ __forceinline__ void issue(char* lds, int ks, int weights_from) const {
-    const int w = wave_id();
-#pragma unroll
-    for (int i = 0; i < NI; ++i) {
+    for (int i = PART * NI / PARTS; i < (PART + 1) * NI / PARTS; ++i) {
       const char* g = src[i] + (size_t)ks * kRowBytes;
       char* d = lds + 1024 * (NW * i + w);
-      if (8 * (NW * i + w) >= weights_from) dma_to_lds<16, kPolicyWeights>(g, d);
+      if (STREAM && 8 * NW * i >= FROM) dma_to_lds<16, kPolicyWeights>(g, d);
       else dma_to_lds<16>(g, d);
     }
   }
