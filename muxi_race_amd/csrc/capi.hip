@@ -430,8 +430,11 @@ static int fused_common(int qt, const void* x, const float* logits, const void* 
   int32_t* gpo = (int32_t*)(ws + L.gpo);
   const int64_t rows = cap_rows(T, ke, Ee, block_m);
   // (a shard is expected to get its share of the pairs)
-  moe::ItemPlan plan = fused_plan(T * ke, shard ? (T * ke * E + E_route - 1) / E_route : T * ke, Ee, H, I, qt);
-  if (!narrow) plan.out = (int32_t*)(ws + L.plan);
+  moe::ItemPlan plan;
+  if (!narrow) {
+    plan = fused_plan(T * ke, shard ? (T * ke * E + E_route - 1) / E_route : T * ke, Ee, H, I, qt);
+    plan.out = (int32_t*)(ws + L.plan);
+  }
   const int e_shared = shared ? (int)E : -1;
 
   // optional stage markers: ev[0] start, [1] routed, [2] aligned, [3] x quantised,

@@ -193,20 +193,32 @@ __device__ void item_plan(const int* tot, int E, const ItemPlan& p, int* sm) {
     }
   }
   __syncthreads();
-  if (w < nh) {
+  if (w < kPlanHeights) {
     const int k = l / 18;  // 0: Stage 1, 1: Stage 2 with 256 features, 2: with 128
     const bool may = k == 0 ? w == 0 || p.any1 : (w == 0 || p.any2) && p.bn2 != (k == 1 ? 128 : 256);
-    const int nt = k == 0 ? p.nt1 : (k == 1 ? p.nt2 / 2 : p.nt2);
-    const XcdPick pick = xcd_pick(mine, gof, E, nt, k < 3 && may, k == 0 ? p.slots1 : p.slots2);
+    XcdPick pick = {0, false, INFINITY};
+    if (w < nh) {
+      const int nt = k == 0 ? p.nt1 : (k == 1 ? p.nt2 / 2 : p.nt2);
+      pick = xcd_pick(mine, gof, E, nt, k < 3 && may, k == 0 ? p.slots1 : p.slots2);
+    }
     if (pick.chosen) xbs[9 * (3 * w + k) + l % 18 % 9] = pick.item;
     if (k < 3 && l % 18 == 0) est[3 * w + k] = may ? pick.slow * (k == 2 ? kHalfTile : 1.0f) : INFINITY;
   }
   __syncthreads();
+  float t[kPlanLaunches];  // all loads before the comparisons
+#pragma unroll
+  for (int j = 0; j < kPlanLaunches; ++j) t[j] = est[j];
   int s1 = 0, s2 = p.bn2 == 128 ? 2 : 1;
-  for (int j = 0; j < nh; ++j) {
-    if (est[3 * j] < est[s1]) s1 = 3 * j;
-    for (int k = 1; k < 3; ++k)
-      if (est[3 * j + k] < est[s2]) s2 = 3 * j + k;
+  float t1 = t[0], t2 = p.bn2 == 128 ? t[2] : t[1];
+#pragma unroll
+  for (int j = 1; j < kPlanLaunches; ++j) {
+    if (j % 3 == 0) {
+      s1 = t[j] < t1 ? j : s1;
+      t1 = fminf(t1, t[j]);
+    } else {
+      s2 = t[j] < t2 ? j : s2;
+      t2 = fminf(t2, t[j]);
+    }
   }
   for (int e = tid; e <= E; e += blockDim.x) {
     p.out[e] = ist[s1 / 3 * (E + 1) + e];
