@@ -105,6 +105,22 @@ int64_t align_bm(int64_t T, int64_t E, int64_t k, int64_t H, int64_t I, int64_t 
 
 constexpr int64_t kCus = 256;
 
+// Whether a call streams the weights that no other item reads past the caches.
+// Kernels of one workgroup per CU wait on each step's loads, and a layer whose
+// weights stay in the 256 MB Infinity Cache from one call to the next is faster
+// if they may.  Of `experts` experts the call touches this much:
+//   44 MB  8 of H 7168, I 1024, fp8, 1 token   repeated 54 -> 42 us, with other layers between 57 -> 58
+//   101    16 of H 2048, I 1024, fp8, 128      44 -> 41, 45 -> 48
+//   176    8 of H 7168, I 1024, int8, 128      81 -> 68, 83 -> 86
+//   201    16 of H 2048, I 1024, fp16, 128     58 -> 52, 62 -> 66
+//   264    6 of H 7168, I 2048, fp8, 1         74 -> 69
+//   403    16 of H 4096, I 2048, fp8, 300      105 -> 114, 104 -> 112
+// (32-row items of the other kernels, two workgroups per CU, lose 2-8% of a
+// first pass by it and gain nothing: they always stream.)
+bool stream_weights(int64_t experts, int64_t H, int64_t I, int qt) {
+  return experts * 3 * H * I * (qt == moe::kQF16 ? 2 : 1) > ((int64_t)320 << 20);
+}
+
 // What a fused launch's plan (launch.h ItemPlan) may choose from, for any
 // routing of `pairs` pairs over `experts` experts of which `rows` are expected
 // here (an expert shard's share).  With every expert at the average:
@@ -242,6 +258,7 @@ int moe_run_prerouted_events(const void* x, const void* w_gate, const void* w_up
   // 141 (64 experts of 30 but 41 of 203) 1331 -> 1390, so the line lies between.
   if (V <= kSkewRows * experts && blocks > experts) wide.hmax = moe::kLowRows;
   p1.hmax = wide.hmax;
+  p1.stream = stream_weights(experts, H, I, moe::kQF16);
   // optional stage markers: ev[0] start, [1] stage 1, [2] stage 2
   auto mark = [&](int i) { if (stage_events && stage_events[i]) (void)hipEventRecord((hipEvent_t)stage_events[i], s); };
   mark(0);
@@ -264,6 +281,7 @@ int moe_run_prerouted_events(const void* x, const void* w_gate, const void* w_up
   p2.I = I;
   p2.V = V;
   p2.hmax = wide.hmax;
+  p2.stream = p1.stream;
   p2.bn = wide.bn;
   rc = check_launch(moe::launch_stage2(p2, false, moe::kQF16, false, blocks, s), "stage2");
   mark(2);
@@ -497,6 +515,7 @@ static int fused_common(int qt, const void* x, const float* logits, const void* 
     p1.xb = plan.out + moe::ItemPlan::xb1(Ee);
   }
   p1.rows_cap = (int)rows;
+  p1.stream = stream_weights(T * ke < Ee ? T * ke : Ee, H, I, qt);
   if ((rc = check_launch(moe::launch_stage1(p1, narrow, qt, true, narrow ? rows / 32 : plan.slots1, s), "stage1"))) return rc;
   // int8: h (fp16) -> per-row int8 codes + scales, for the routed rows only
   // (sorted id below the sentinel T * ke, row below gpo[E])
@@ -522,6 +541,7 @@ static int fused_common(int qt, const void* x, const float* logits, const void* 
     p2.bn_plan = plan.out + moe::ItemPlan::bn(Ee);
   }
   p2.rows_cap = (int)rows;
+  p2.stream = p1.stream;
   p2.routed = rwts;
   p2.routed_f16 = 0;
   p2.gs = gs;

@@ -351,7 +351,7 @@ __global__ __launch_bounds__(256) void stage1_f8_kernel(Stage1Params p) {
       half(std::integral_constant<int, 1>{});
     }
   };
-  if (w.shared) k_loop(std::false_type{});
+  if (w.shared || !p.stream) k_loop(std::false_type{});
   else k_loop(std::true_type{});
   __syncthreads();  // every wave is done with the ring before LDS is reused
 
@@ -962,13 +962,13 @@ __global__ __launch_bounds__(512) void stage1_wide_kernel(Stage1Params p) {
   auto run = [&](const Item& it) {
     if (it.actual <= 0) return;  // no token: Stage 2 writes the rows as 0
     if (it.actual <= kLowRows) {
-      if (it.shared) stage1_item<QT, GATHER, kLowRows, false, false>(p, it, smem);
+      if (it.shared || !p.stream) stage1_item<QT, GATHER, kLowRows, false, false>(p, it, smem);
       else stage1_item<QT, GATHER, kLowRows, false, true>(p, it, smem);
     } else if (QT != kQF16 || it.actual <= kWideRows) {
-      if (it.shared) stage1_item<QT, GATHER, kWideRows, false, false>(p, it, smem);
+      if (it.shared || !p.stream) stage1_item<QT, GATHER, kWideRows, false, false>(p, it, smem);
       else stage1_item<QT, GATHER, kWideRows, false, true>(p, it, smem);
     } else if constexpr (QT == kQF16) {
-      if (it.shared) stage1_item<QT, GATHER, kWideRows, true, false>(p, it, smem);
+      if (it.shared || !p.stream) stage1_item<QT, GATHER, kWideRows, true, false>(p, it, smem);
       else stage1_item<QT, GATHER, kWideRows, true, true>(p, it, smem);
     }
   };
@@ -1136,13 +1136,13 @@ __global__ __launch_bounds__(512) void stage2_wide_kernel(Stage2Params p) {
   auto run_bn = [&](const Item& it, auto bn_c) {
     constexpr int BN = decltype(bn_c)::value;
     if (it.actual <= kLowRows) {
-      if (it.shared) stage2_item<QT, FUSED, BN, kLowRows, false, false>(p, it, smem);
+      if (it.shared || !p.stream) stage2_item<QT, FUSED, BN, kLowRows, false, false>(p, it, smem);
       else stage2_item<QT, FUSED, BN, kLowRows, false, true>(p, it, smem);
     } else if (QT != kQF16 || it.actual <= kWideRows) {
-      if (it.shared) stage2_item<QT, FUSED, BN, kWideRows, false, false>(p, it, smem);
+      if (it.shared || !p.stream) stage2_item<QT, FUSED, BN, kWideRows, false, false>(p, it, smem);
       else stage2_item<QT, FUSED, BN, kWideRows, false, true>(p, it, smem);
     } else if constexpr (QT == kQF16) {
-      if (it.shared) stage2_item<QT, FUSED, BN, kWideRows, true, false>(p, it, smem);
+      if (it.shared || !p.stream) stage2_item<QT, FUSED, BN, kWideRows, true, false>(p, it, smem);
       else stage2_item<QT, FUSED, BN, kWideRows, true, true>(p, it, smem);
     }
   };

@@ -78,6 +78,7 @@ struct Stage1Params {
   const int32_t* xb = nullptr;      // wide, gather: [9] first item of each XCD
   int rows_cap = 0;         // wide, gather: rows the buffers hold
   int hmax = 0;             // wide, direct: most rows of an item (moe_common.h Item)
+  bool stream = true;       // wide, and fp8 of 32-row tiles: weights that no other item reads non-temporal
 };
 
 // Stage 2: y = h Wd^T, scaled by the routing weight of each row.
@@ -114,6 +115,7 @@ struct Stage2Params {
   int bn = 0;               // wide, pre-routed: features of an item, 128 or 256
   int rows_cap = 0;
   int hmax = 0;
+  bool stream = true;       // wide: as Stage 1's
   int topk = 0;             // fused, built with MOE_S2_SCATTER: choices per token; `out` is then
                             // fp16 [T, H] (zeroed first) and each pair row is added to its token's
                             // row with packed fp16 atomics
