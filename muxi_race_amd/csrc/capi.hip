@@ -57,7 +57,7 @@ FusedLayout fused_layout(int64_t T, int64_t H, int64_t I, int64_t E, int64_t k, 
   L.gs = o; o += up(E * 4);
   L.go = o; o += up((E + 1) * 4);
   L.gpo = o; o += up((E + 1) * 4);
-  L.plan = o; o += up(moe::ItemPlan::ints(E) * 4);        // the wide items' plan
+  L.plan = o; o += bm == 32 ? 0 : up(moe::ItemPlan::ints(E) * 4);  // the wide items' plan
   L.whist = o; o += up((int64_t)moe::align_groups((int)P) * E * 4);  // align workgroup histograms
   L.h = o; o += up(rows * I * (qt == moe::kQF8 ? 1 : 2));
   L.hq = o; o += i8 ? up(rows * I) : 0;                   // int8: per-row codes of h
@@ -89,21 +89,18 @@ int64_t pick_bm(int64_t T, int64_t E, int64_t k) {
 //   - narrow up to kLowRows rows where one wide item per expert and tile would
 //     leave half of the CUs idle: 8 experts, H 1024, I 512, top-2, 400 tokens
 //     22 / 34 us, but 1000 tokens (250 rows) 41 / 34.
-//   - otherwise pick_bm's padding, at least 64, and 256 from 192 rows on if H is
-//     a multiple of 256.
+//   - otherwise 64: what the rows are padded to matters to no wide item, and
+//     less padding is fewer sentinel rows to write and to skip.
 constexpr int64_t kNarrowRows = 24;
+constexpr int64_t kCus = 256;
 // too many rows for the kernels' 32-bit indices
 bool too_large(int64_t T, int64_t k, int64_t E, int64_t I, int64_t bm) { return cap_rows(T, k, E, bm) * I >= ((int64_t)1 << 32); }
-int64_t align_bm(int64_t T, int64_t E, int64_t k, int64_t H, int64_t I, int64_t block_m) {
+int64_t align_bm(int64_t T, int64_t E, int64_t held, int64_t k, int64_t H, int64_t I, int qt, int64_t block_m) {
   if (block_m) return block_m;
-  const int64_t bm = pick_bm(T, E, k);
   const int64_t avg = E > 0 ? (T * k + E - 1) / E : 0;
   if (avg <= kNarrowRows || (avg <= moe::kLowRows && E * (I / moe::kBN) < 128)) return 32;
-  if (bm == 32) return too_large(T, k, E, I, 64) ? 32 : 64;
-  return bm == 128 && H % 256 == 0 && avg >= 192 ? 256 : bm;
+  return too_large(T, k, E, I, 64) ? 32 : 64;
 }
-
-constexpr int64_t kCus = 256;
 
 // Whether a call streams the weights that no other item reads past the caches.
 // Kernels of one workgroup per CU wait on each step's loads, and a layer whose
@@ -183,6 +180,22 @@ WidePlan wide_plan(int64_t rows, int64_t experts, int64_t H, int64_t I) {
 // run_kernel: average rows of an expert up to which more blocks than experts
 // mean short items.
 constexpr int64_t kSkewRows = 112;
+
+// Workspace of a fused call; block_m = 0: enough for every padding that the call
+// may be given or choose -- also for pick_bm's, with 256 rows per block from 192
+// rows per expert on if H is a multiple of 256, which callers may have sized
+// other calls of the same shape by.
+int64_t fused_bytes(int64_t T, int64_t E, int64_t held, int64_t k, int64_t H, int64_t I, int qt, int64_t block_m) {
+  auto total = [&](int64_t bm) { return fused_layout(T, H, I, held, k, bm, qt).total; };
+  int64_t most = total(align_bm(T, E, held, k, H, I, qt, block_m));
+  if (block_m) return most;
+  const int64_t pick = pick_bm(T, E, k), avg = E > 0 ? (T * k + E - 1) / E : 0;
+  for (int64_t bm = 32; bm <= 256; bm *= 2) {
+    if (bm > pick && !(bm == 256 && pick == 128 && H % 256 == 0 && avg >= 192)) continue;
+    most = total(bm) > most ? total(bm) : most;
+  }
+  return most;
+}
 
 bool aligned16(const void* p) { return ((uintptr_t)p & 15) == 0; }
 
@@ -367,10 +380,10 @@ int64_t moe_pick_block_m(int64_t T, int64_t E, int64_t k) { return pick_bm(T, E,
 int64_t moe_fused_workspace_bytes(int64_t T, int64_t H, int64_t I, int64_t E, int64_t k,
                                   int64_t block_m, int w8a8) {
   if (T < 0 || H <= 0 || I <= 0 || E <= 0 || k <= 0) return 0;
-  // w8a8: 0 fp16, 1 int8, 2 fp8 (one padding rule for all)
+  // w8a8: 0 fp16, 1 int8, 2 fp8
   if (w8a8 < 0 || w8a8 > 2) return 0;
-  block_m = align_bm(T, E, k, H, I, block_m);
-  return fused_layout(T, H, I, E, k, block_m, w8a8 == 2 ? moe::kQF8 : (w8a8 ? moe::kQI8 : moe::kQF16)).total;
+  const int qt = w8a8 == 2 ? moe::kQF8 : (w8a8 ? moe::kQI8 : moe::kQF16);
+  return fused_bytes(T, E, E, k, H, I, qt, block_m);
 }
 
 // The always-on shared expert (wg_s / wu_s / wd_s non-null, fp16 only) runs as
@@ -405,7 +418,7 @@ static int fused_common(int qt, const void* x, const float* logits, const void* 
   if (block_m != 0 && block_m != 32 && block_m != 64 && block_m != 128)
     return fail(MOE_ERR_UNSUPPORTED, "block_m=%lld not in {0,32,64,128}", (long long)block_m);
   const int64_t asked_bm = block_m;
-  block_m = align_bm(T, shard ? E_route : Ee, ke, H, I, block_m);
+  block_m = align_bm(T, shard ? E_route : Ee, Ee, ke, H, I, qt, block_m);
   int rc = check_dims(T, H, I, shard ? E_route : Ee, ke, block_m);
   if (rc) return rc;
   if (T == 0) return MOE_OK;
@@ -427,9 +440,8 @@ static int fused_common(int qt, const void* x, const float* logits, const void* 
       (shared && (!aligned16(wg_s) || !aligned16(wu_s) || !aligned16(wd_s))))
     return fail(MOE_ERR_INVALID_ARG, "x, weights, scales, out and workspace must be 16-byte aligned");
   const int64_t router_ws = w_router ? moe_router_workspace_bytes(T, H, E) : 0;
-  // a workspace sized for pick_bm's padding (128 or 32) keeps it
-  if (!asked_bm && workspace_bytes < fused_layout(T, H, I, Ee, ke, block_m, qt).total + router_ws)
-    block_m = pick_bm(T, shard ? E_route : Ee, ke);
+  // a workspace sized for 32-row blocks gets them
+  if (!asked_bm && workspace_bytes < fused_layout(T, H, I, Ee, ke, block_m, qt).total + router_ws) block_m = 32;
   const FusedLayout L = fused_layout(T, H, I, Ee, ke, block_m, qt);
   const int64_t need = L.total + router_ws;
   if (workspace_bytes < need) return fail(MOE_ERR_WORKSPACE, "workspace %lld < %lld bytes", (long long)workspace_bytes, (long long)need);
@@ -599,8 +611,7 @@ int moe_fused_forward_hidden(const void* x, const void* w_router, const float* b
 int64_t moe_fused_shared_workspace_bytes(int64_t T, int64_t H, int64_t I, int64_t E, int64_t k,
                                          int64_t block_m) {
   if (T < 0 || H <= 0 || I <= 0 || E <= 0 || k <= 0) return 0;
-  block_m = align_bm(T, E + 1, k + 1, H, I, block_m);
-  return fused_layout(T, H, I, E + 1, k + 1, block_m, moe::kQF16).total + moe_router_workspace_bytes(T, H, E);
+  return fused_bytes(T, E + 1, E + 1, k + 1, H, I, moe::kQF16, block_m) + moe_router_workspace_bytes(T, H, E);
 }
 
 int moe_fused_forward_shared(const void* x, const float* logits, const void* w_router, const float* bias,
@@ -620,8 +631,7 @@ int64_t moe_fused_ex_workspace_bytes(int64_t T, int64_t H, int64_t I, int64_t E,
                                      int shared, int with_router) {
   if (T < 0 || H <= 0 || I <= 0 || E <= 0 || k <= 0) return 0;
   const int64_t s = shared ? 1 : 0;
-  block_m = align_bm(T, E + s, k + s, H, I, block_m);
-  return fused_layout(T, H, I, E + s, k + s, block_m, moe::kQF16).total + (with_router ? moe_router_workspace_bytes(T, H, E) : 0);
+  return fused_bytes(T, E + s, E + s, k + s, H, I, moe::kQF16, block_m) + (with_router ? moe_router_workspace_bytes(T, H, E) : 0);
 }
 
 int moe_fused_forward_ex(const void* x, const float* logits, const void* w_router, const float* bias,
@@ -641,8 +651,7 @@ int moe_fused_forward_ex(const void* x, const float* logits, const void* w_route
 int64_t moe_fused_shard_workspace_bytes(int64_t T, int64_t H, int64_t I, int64_t E_total, int64_t k,
                                         int64_t E_local, int64_t block_m) {
   if (T < 0 || H <= 0 || I <= 0 || E_total <= 0 || E_local <= 0 || k <= 0) return 0;
-  block_m = align_bm(T, E_total, k, H, I, block_m);
-  return fused_layout(T, H, I, E_local, k, block_m, moe::kQF16).total;
+  return fused_bytes(T, E_total, E_local, k, H, I, moe::kQF16, block_m);
 }
 
 int moe_fused_forward_shard(const void* x, const float* logits, const float* bias, const void* w_gate,
@@ -720,15 +729,14 @@ int moe_fused_forward_noalloc(const void* x, const float* logits, const float* b
                               float* topk_weights_out, void* stream) {
   if (block_m != 0 && block_m != 32 && block_m != 64 && block_m != 128)
     return fail(MOE_ERR_UNSUPPORTED, "block_m=%lld not in {0,32,64,128}", (long long)block_m);
-  int64_t bm = align_bm(T, E, k, H, I, block_m);
+  int64_t bm = align_bm(T, E, E, k, H, I, moe::kQF16, block_m);
   int rc = check_dims(T, H, I, E, k, bm);
   if (rc) return rc;
   if (T == 0) return MOE_OK;
-  // the padding the call will use: pick_bm's where a larger one does not fit
-  // (as for any workspace sized for that)
+  // the padding the call will use: 32 rows where a larger one does not fit (as
+  // for any workspace sized for that)
   int64_t need = fused_layout(T, H, I, E, k, bm, moe::kQF16).total;
-  if (!block_m && need > kNoAllocScratchBytes)
-    need = fused_layout(T, H, I, E, k, pick_bm(T, E, k), moe::kQF16).total;
+  if (!block_m && need > kNoAllocScratchBytes) need = fused_layout(T, H, I, E, k, 32, moe::kQF16).total;
   if (need > kNoAllocScratchBytes)
     return fail(MOE_ERR_WORKSPACE,
                 "moe_fused_forward_noalloc: T=%lld H=%lld I=%lld E=%lld k=%lld needs %lld bytes of scratch, the "

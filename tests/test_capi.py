@@ -169,3 +169,30 @@ def test_measured_variant_compiles(tmp_path, define, sources):
         cmd = [hipcc, *HIP_FLAGS, f"-D{define}=1", "-c", str(CSRC / src), "-o", str(tmp_path / (src + ".o"))]
         r = subprocess.run(cmd, capture_output=True, text=True)
         assert r.returncode == 0, r.stderr[-2000:]
+
+
+def test_workspace_for_any_block_m_and_batch():
+    """A workspace sized with block_m = 0 holds the call with any block_m that
+    the rows per expert suggest (moe_pick_block_m) or smaller, for every format
+    and entry; and one sized for the largest batch holds the smaller ones."""
+    from muxi_race_amd._lib import lib
+    L = lib()
+    for H, I, E, k in ((7168, 2048, 256, 8), (4096, 14336, 8, 2), (1024, 512, 8, 2), (7168, 1024, 8, 2),
+                       (2048, 768, 128, 8), (384, 128, 1024, 4), (128, 128, 1, 1)):
+        last = {}
+        for T in (1, 7, 32, 100, 128, 129, 200, 256, 400, 512, 513, 800, 1000, 1500, 2048, 4096, 8192):
+            pick = L.moe_pick_block_m(T, E, k)
+            sizes = {f"fmt {f}": lambda bm, f=f: L.moe_fused_workspace_bytes(T, H, I, E, k, bm, f) for f in (0, 1, 2)}
+            sizes["hidden"] = lambda bm: L.moe_fused_hidden_workspace_bytes(T, H, I, E, k, bm)
+            if E > 1:
+                held = max(1, E // 8)
+                sizes["shard"] = lambda bm: L.moe_fused_shard_workspace_bytes(T, H, I, E, k, held, bm)
+            for name, size in sizes.items():
+                for bm in (b for b in (32, 64, 128) if b <= pick):
+                    assert size(0) >= size(bm), (name, T, H, I, E, k, bm)
+                if name != "hidden":  # the router's partial sums shrink where it splits K less
+                    assert size(0) >= last.get(name, 0), (name, T, H, I, E, k)
+                    last[name] = size(0)
+            p = L.moe_pick_block_m(T, E + 1, k + 1)
+            shared = lambda bm: L.moe_fused_shared_workspace_bytes(T, H, I, E, k, bm)
+            assert shared(0) >= shared(p)

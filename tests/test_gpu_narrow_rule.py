@@ -1,0 +1,35 @@
+"""What a fused call with block_m = 0 runs and needs."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _case(T, E, held, k, I):
+    g = torch.Generator(device="cuda").manual_seed(T + E)
+    mk = lambda *sh: torch.randn(sh, generator=g, device="cuda")
+    x, lg = mk(T, 1024).half(), mk(T, E)
+    return x, lg, [(mk(*sh) * 0.05).half() for sh in ((held, I, 1024), (held, I, 1024), (held, 1024, I))]
+
+
+@pytest.mark.parametrize("bm", [32, 64, 128])
+def test_workspace_sized_without_block_m_serves_explicit_blocks(bm):
+    """A C caller's workspace sized with block_m = 0 also holds the call with
+    an explicit block_m up to the one that the rows per expert suggest."""
+    from muxi_race_amd._lib import lib
+    L = lib()
+    T, H, I, E, k = 400, 1024, 512, 8, 2   # 100 rows per expert: moe_pick_block_m says 128
+    assert L.moe_pick_block_m(T, E, k) == 128
+    x, lg, w = _case(T, E, E, k, I)
+    outs = []
+    for b in (bm, 0):
+        ws = torch.empty(L.moe_fused_workspace_bytes(T, H, I, E, k, 0, 0), dtype=torch.uint8, device="cuda")
+        out = torch.full((T, H), float("nan"), dtype=torch.float16, device="cuda")
+        rc = L.moe_fused_forward(x.data_ptr(), lg.data_ptr(), None, *(m.data_ptr() for m in w), out.data_ptr(), T, H, I, E,
+                                 k, b, ws.data_ptr(), ws.numel(), None, None, torch.cuda.current_stream().cuda_stream)
+        assert rc == 0, L.moe_last_error_string()
+        torch.cuda.synchronize()
+        outs.append(out.float())
+    # K sums in another order: one fp16 rounding of h and of the output each
+    assert torch.isfinite(outs[0]).all()
+    assert float((outs[0] - outs[1]).norm() / outs[1].norm()) < 2e-3
