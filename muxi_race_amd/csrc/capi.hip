@@ -86,9 +86,16 @@ int64_t pick_bm(int64_t T, int64_t E, int64_t k) {
 //     3.57, 1024 (32) 4.24 / 3.56; 64 experts top-6, 256 tokens (24) 0.88 /
 //     0.86, 300 (28) 0.97 / 0.89; int8 256 tokens 0.469 / 0.475, 300 0.484 /
 //     0.456.  Above it more and more experts need a second 32-row block.
-//   - narrow up to kLowRows rows where one wide item per expert and tile would
-//     leave half of the CUs idle: 8 experts, H 1024, I 512, top-2, 400 tokens
-//     22 / 34 us, but 1000 tokens (250 rows) 41 / 34.
+//   - narrow where that takes no more than one item per CU (fp8), or about as
+//     much work (fp16 and int8, whose narrow items are smaller but two to a CU):
+//     up to 256 and 200 expected pairs of a 32-row block and a 128-feature tile
+//     over the `held` experts whose weights are here, half a block of padding
+//     each.  Whole calls at 160 / 224 / 288 of them, narrow against wide, us:
+//     8 experts top-2, H 7168, I 1024: fp16 123 / 135, 154 / 143, 180 / 153; int8
+//     84 / 90, 102 / 96, 116 / 103; fp8 83 / 86, 90 / 92, 131 / 98.  16 of H 4096,
+//     I 512: fp16 82 / 86, 99 / 93, 117 / 97; fp8 60 / 63, 66 / 69, 93 / 70.
+//     Over 1248 such calls (13 layers, 8 to 224 rows) the choice is 0.3% slower on
+//     average than the better of the two.
 //   - otherwise 64: what the rows are padded to matters to no wide item, and
 //     less padding is fewer sentinel rows to write and to skip.
 constexpr int64_t kNarrowRows = 24;
@@ -98,7 +105,8 @@ bool too_large(int64_t T, int64_t k, int64_t E, int64_t I, int64_t bm) { return 
 int64_t align_bm(int64_t T, int64_t E, int64_t held, int64_t k, int64_t H, int64_t I, int qt, int64_t block_m) {
   if (block_m) return block_m;
   const int64_t avg = E > 0 ? (T * k + E - 1) / E : 0;
-  if (avg <= kNarrowRows || (avg <= moe::kLowRows && E * (I / moe::kBN) < 128)) return 32;
+  const int64_t narrow_items = qt == moe::kQF8 ? kCus : 200;
+  if (avg <= kNarrowRows || held * (2 * avg + 32) * (I / moe::kBN) <= 64 * narrow_items) return 32;
   return too_large(T, k, E, I, 64) ? 32 : 64;
 }
 

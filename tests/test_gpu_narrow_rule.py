@@ -1,4 +1,8 @@
-"""What a fused call with block_m = 0 runs and needs."""
+"""Which items a fused call with block_m = 0 runs, read off its bits: fp16
+32-row items sum two halves of K, wide ones the whole of it, so the call equals
+either block_m = 32 or block_m = 64 and the other differs.  The line lies where
+the expected 32-row blocks over the experts held here take about one item per
+CU."""
 import pytest
 import torch
 
@@ -10,6 +14,26 @@ def _case(T, E, held, k, I):
     mk = lambda *sh: torch.randn(sh, generator=g, device="cuda")
     x, lg = mk(T, 1024).half(), mk(T, E)
     return x, lg, [(mk(*sh) * 0.05).half() for sh in ((held, I, 1024), (held, I, 1024), (held, 1024, I))]
+
+
+# (tokens, experts routed over, held, k, I, narrow): 200 pairs of a block and a
+# tile are 8 experts of 84 rows at I 1024, of 184 at I 512
+@pytest.mark.parametrize("T,E,held,k,I,narrow", [
+    (336, 8, 8, 2, 1024, True), (400, 8, 8, 2, 1024, False), (512, 8, 8, 2, 1024, False),
+    (736, 8, 8, 2, 512, True), (800, 8, 8, 2, 512, False),
+    (96, 8, 8, 2, 2048, True), (128, 8, 8, 2, 2048, True), (160, 8, 8, 2, 2048, False),
+    # an expert shard counts the experts that it holds: 4 of 64 at 100 rows
+    (3200, 64, 4, 2, 512, True), (3200, 64, 64, 2, 512, False), (8000, 64, 4, 2, 512, True), (16000, 64, 4, 2, 512, False),
+])
+def test_library_picks(T, E, held, k, I, narrow):
+    from muxi_race_amd import fused_moe
+    x, lg, w = _case(T, E, held, k, I)
+    more = {} if held == E else dict(expert_range=(8, held))
+    got, n, wide = (fused_moe(x, lg, *w, k, block_m=bm, **more) for bm in (0, 32, 64))
+    torch.cuda.synchronize()
+    assert not torch.equal(n, wide), "the sums do not tell the items apart"
+    assert torch.equal(got, n if narrow else wide)
+
 
 
 @pytest.mark.parametrize("bm", [32, 64, 128])
