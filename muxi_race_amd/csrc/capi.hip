@@ -169,25 +169,40 @@ moe::ItemPlan fused_plan(int64_t pairs, int64_t rows, int64_t experts, int64_t H
   return p;
 }
 
-// run_kernel: the tallest item and Stage 2's features per item, every expert
-// taken to hold the average of `rows` rows.  Launches that would not give every
-// CU an item take shorter and narrower ones.
+// run_kernel: the tallest item and Stage 2's features per item, for `rows` routed
+// rows over `experts` experts in `blocks` blocks of 128.
+//   - 288 rows; 128 where that would not give every CU an item with every expert
+//     at the average, and where few experts are taller than one block -- no more
+//     than a quarter as many blocks as experts beyond one each, or an average of
+//     at most kSkewRows -- whose tall items would end long after the short ones.
+//     Up to 288 rows, up to 128, us (H 7168, I 2048): 64 experts of 115 rows but 3
+//     of 300 1262 / 1212, of 110 but 10 of 200 1250 / 1239, 32 of 100 but 2 of 380
+//     658 / 628, of 3 but 8 of 336 739 / 667; 16 (H 2048, I 8192) of 110 but one of
+//     300 453 / 386, of 19 but 4 of 350 453 / 416.  On the other side 64 of 90 but
+//     30 of 150 1199 / 1279, of 30 but 41 of 203 1403 / 1497, 32 of 112 but 22 of
+//     155 643 / 783; the line costs 32 of 110 but 4 of 240 2% (629 / 644).
+//   - Stage 2 takes the width whose rounds of 256 CUs cost less, a 128-feature
+//     item costing 0.7 of a 256-feature one (routing.hip kHalfTile).  The pieces
+//     are the blocks for items of up to 128 rows.  16 experts (H 2048, I 8192) of
+//     19 but 4 of 350: 384 items of 128 features 176 us, 192 of 256 153.
+constexpr int64_t kSkewRows = 112;
 struct WidePlan {
   int hmax;
   int bn;
 };
-WidePlan wide_plan(int64_t rows, int64_t experts, int64_t H, int64_t I) {
+WidePlan wide_plan(int64_t rows, int64_t experts, int64_t blocks, int64_t H, int64_t I) {
   const int64_t avg = (rows + experts - 1) / experts;
+  int64_t pieces = experts * moe::items_of((int)avg, moe::kTallRows);
   WidePlan w;
   w.hmax = moe::kTallRows;
-  if (experts * moe::items_of((int)avg, w.hmax) * (I / moe::kBN) < kCus) w.hmax = moe::kLowRows;
-  w.bn = H % 256 == 0 && experts * moe::items_of((int)avg, w.hmax) * (H / 256) >= kCus ? 256 : 128;
+  if (pieces * (I / moe::kBN) < kCus || 4 * (blocks - experts) <= experts || avg <= kSkewRows) {
+    w.hmax = moe::kLowRows;
+    pieces = blocks;
+  }
+  auto rounds = [&](int64_t bn) { return (pieces * (H / bn) + kCus - 1) / kCus; };
+  w.bn = H % 256 == 0 && 10 * rounds(256) <= 7 * rounds(128) ? 256 : 128;
   return w;
 }
-
-// run_kernel: average rows of an expert up to which more blocks than experts
-// mean short items.
-constexpr int64_t kSkewRows = 112;
 
 // Workspace of a fused call; block_m = 0: enough for every padding that the call
 // may be given or choose -- also for pick_bm's, with 256 rows per block from 192
@@ -270,14 +285,7 @@ int moe_run_prerouted_events(const void* x, const void* w_gate, const void* w_up
   p1.H = H;
   p1.I = I;
   const int64_t experts = E < blocks ? E : blocks;
-  WidePlan wide = wide_plan(V > experts ? V : experts, experts, H, I);
-  // A low average beside more blocks than experts: a few tall experts among
-  // short ones.  Items of up to 288 rows then end long after the short ones.
-  // Up to 288 rows, up to 128: 32 experts (H 7168, I 2048) of 3 rows but 8 of 336
-  // 735 -> 653 us, of 11 but 5 of 300 632 -> 604, of 60 but 3 of 380 654 -> 619; 16
-  // (H 2048, I 8192) of 19 but 4 of 350 448 -> 415: averages of 56 to 102.  At
-  // 141 (64 experts of 30 but 41 of 203) 1331 -> 1390, so the line lies between.
-  if (V <= kSkewRows * experts && blocks > experts) wide.hmax = moe::kLowRows;
+  const WidePlan wide = wide_plan(V > experts ? V : experts, experts, blocks, H, I);
   p1.hmax = wide.hmax;
   p1.stream = stream_weights(experts, H, I, moe::kQF16);
   // optional stage markers: ev[0] start, [1] stage 1, [2] stage 2

@@ -468,14 +468,13 @@ __device__ __forceinline__ XcdCut xcd_cut(int x, bool weighted, const int* ist, 
 // third.  slots: workgroups an XCD has in the launch, which a cut has to fit in.
 constexpr int kCusPerXcd = 32;
 struct XcdPick {
-  int item;     // first item of XCD (lane % 18) % 9
-  bool chosen;  // this lane's cut is the better one
-  float slow;   // its slowest XCD's time, in rows of cost; INFINITY: neither fits
+  int item;       // first item of XCD (lane % 18) % 9
+  bool weighted;  // the cut by cost is the better one
+  float slow;     // its slowest XCD's time, in rows of cost; INFINITY: neither fits
 };
-__device__ __forceinline__ XcdPick xcd_pick(const int* ist, const int* gof, int E, int nt, bool active, int slots) {
+// From the cuts themselves, one per lane.
+__device__ __forceinline__ XcdPick xcd_better(XcdCut cut, bool active, int slots) {
   const int l = lane_id(), q = l % 18, base = l - q, x = q % 9;
-  XcdCut cut = {0, 0.0};
-  if (active) cut = xcd_cut(x, q >= 9, ist, gof, E, nt);
   const int items = __shfl_down(cut.item, 1) - cut.item;
   const float cost = __shfl_down((float)cut.cost, 1) - (float)cut.cost;
   float t = 0.0f;
@@ -489,14 +488,15 @@ __device__ __forceinline__ XcdPick xcd_pick(const int* ist, const int* gof, int 
   const uint64_t over = __ballot(active && x < 8 && items > slots) >> base;
   if (over & 0x1ff) equal = INFINITY;
   if (over & 0x3fe00) weighted = INFINITY;
-  const bool take = weighted < equal;
-  return XcdPick{cut.item, active && (q >= 9) == take, take ? weighted : equal};
+  return XcdPick{cut.item, weighted < equal, fminf(weighted, equal)};
 }
-// xb[0..8]: the better cut of one launch.
-__device__ __forceinline__ void xcd_shares(const int* ist, const int* gof, int E, int nt, int32_t* xb, int slots) {
-  const XcdPick p = xcd_pick(ist, gof, E, nt, lane_id() < 18, slots);
-  if (p.chosen) xb[lane_id() % 9] = p.item;
+__device__ __forceinline__ XcdPick xcd_pick(const int* ist, const int* gof, int E, int nt, bool active, int slots) {
+  const int q = lane_id() % 18;
+  XcdCut cut = {0, 0.0};
+  if (active) cut = xcd_cut(q % 9, q >= 9, ist, gof, E, nt);
+  return xcd_better(cut, active, slots);
 }
+
 // An upper bound on an XCD's items with either cut, for `pieces` items per N tile
 // and `rows` routed rows in all.
 inline int64_t xcd_items_bound(int64_t pieces, int64_t rows, int64_t nt) {
@@ -514,160 +514,247 @@ inline int64_t xcd_items_bound(int64_t pieces, int64_t rows, int64_t nt) {
 // tile, which writes its rows as 0.  A gidx value outside [0, E) gives e = -1
 // (rows owned by no expert).
 //
-// The items below a run are counted here, by the workgroup's 512 threads, 512
-// blocks at a time: block j of a run counts the pieces that its rows add,
-// items_of(min(n, 128 (j + 1))) - items_of(min(n, 128 j)), which sums to the
-// run's.  (Numbering by blocks instead, with the surplus items ending at once,
-// left the XCDs unequal work: 22 experts of 155 rows and 10 of 112, H 7168, I
-// 2048, Stage 1 551 us.)
+// The items below a run are counted here, by the workgroup's 512 threads, M
+// neighbouring blocks each (1 up to 512 blocks, else kScanBlocks): block j of a
+// run counts the pieces that its rows add, items_of(min(n, 128 (j + 1))) -
+// items_of(min(n, 128 j)), which sums to the run's.  (Numbering by blocks
+// instead, with the surplus items ending at once, left the XCDs unequal work: 22
+// experts of 155 rows and 10 of 112, H 7168, I 2048, Stage 1 551 us.)  This runs
+// before every item's first load, so it makes two dependent round trips to
+// memory -- block to expert, expert to its rows -- and finds the rest in LDS.
+// A pass covers kThreads * M blocks; only launches of more than 4096 make two.
 //
-// Launches of up to 512 blocks with an expert of more than kCutRows rows cut
-// their items over the XCDs as the fused ones do (xcd_shares, over blocks
-// instead of experts); others into equal numbers, which saves the 2 us that the
-// comparison of the two cuts takes before each item.  So do items of up to
-// kLowRows rows, which differ little (32 experts of 11 rows but 5 of 300: 633 us
-// cut by cost, 604 into equal numbers).
+// Launches of up to 512 blocks with an expert of more than kCutRows rows, in
+// items of more than kLowRows, cut their items over the XCDs as the fused ones
+// do (xcd_better): the thread whose block holds a cut writes it.  Others cut
+// into equal numbers: like items gain nothing by the comparison, 1 us before each
+// item (22 experts of 155 rows and 10 of 112: 602 us without it, 619 with), and
+// short ones differ little (32 experts of 11 rows but 5 of 300: 633 us cut by
+// cost, 604 into equal numbers).
+constexpr int kScanBlocks = 8;
 constexpr int kCutRows = 192;
 struct RunScan {
-  int smem_s[8], smem_p[8], smem_r[8];
-  int xb[9];
-  int ist[513], gof[513];  // items per N tile and rows below each block
+  int last[8], pieces[8], rows[8];     // per wave: its last run's first block, pieces and rows it adds
+  int tall[8];                         // ... whether a run has more than kCutRows rows
+  int run[8], below[8], val[8], left[8];  // per wave: the last run at or before the item
+  int cut_item[2][8];                  // [equal numbers, equal cost][XCD]
+  float cut_cost[2][8];
+  uint32_t firsts[16 * kScanBlocks];   // bit b: block b starts a run
 };
 
-__device__ __forceinline__ bool item_bx(int g, const int32_t* __restrict__ gidx, int nblk, int E, int BN, int nt,
-                                        const int32_t* __restrict__ gs, const int32_t* __restrict__ gpo, int hmax,
-                                        int grid, char* smem, Item& it) {
-  constexpr int BM = 128, kThreads = 512;
+template <int M>
+__device__ __forceinline__ bool item_runs(int g, const int32_t* __restrict__ gidx, int nblk, int E, int BN, int nt,
+                                          const int32_t* __restrict__ gs, const int32_t* __restrict__ gpo, int hmax,
+                                          int grid, char* smem, Item& it) {
+  constexpr int BM = 128, kThreads = 512, kPass = kThreads * M;
   RunScan* sh = reinterpret_cast<RunScan*>(smem);
-  const int l = lane_id(), w = wave_id();
-  // pass over all blocks; f(block, first of its run, items below it, rows below it)
-  int rows_all = 0;
-  bool tall = false;  // a block of this thread belongs to a run of more than kCutRows rows
-  auto sweep = [&](auto&& f) {
-    int carry_s = 0, carry_p = 0, carry_r = 0;
-    for (int base = 0; base < nblk; base += kThreads) {
-      const int b = base + (int)threadIdx.x;
-      const int bc = b < nblk ? b : nblk - 1;
-      const int val = gidx[bc], before = gidx[bc > 0 ? bc - 1 : 0];
-      const bool first = b < nblk && (b == 0 || val != before);
-      const uint64_t m = __ballot(first);
-      if (l == 0) sh->smem_s[w] = m ? base + 64 * w + 63 - __builtin_clzll(m) : -1;
-      const bool owned = val >= 0 && val < E;
-      const int ec = owned ? val : 0;
-      const int gs_e = gs[ec], gpo_e = gpo[ec];
-      __syncthreads();
-      int s = carry_s;
-      for (int v = 0; v < w; ++v) s = sh->smem_s[v] >= 0 ? sh->smem_s[v] : s;
-      const uint64_t upto = m & (l == 63 ? ~0ull : (1ull << (l + 1)) - 1);
-      if (upto) s = base + 64 * w + 63 - __builtin_clzll(upto);
-      const int64_t left = owned ? (int64_t)gs_e - ((int64_t)s * BM - gpo_e) : 0;
+  const int l = lane_id(), w = wave_id(), tid = threadIdx.x;
+  const bool one_pass = nblk <= kPass;
+
+  // this thread's blocks of a pass
+  int below[M], rbelow[M], pcs[M], rws[M], val[M], left[M];
+  uint32_t first = 0;
+  int carry_s = 0, carry_p = 0, carry_r = 0;  // of the passes before
+  auto pass = [&](int base) {
+    const int b0 = base + tid * M;
+    int gs_e[M], gpo_e[M];
+#pragma unroll
+    for (int j = 0; j < M; ++j) val[j] = gidx[b0 + j < nblk ? b0 + j : nblk - 1];
+    int prev = gidx[b0 > 0 ? (b0 <= nblk ? b0 - 1 : nblk - 1) : 0];
+#pragma unroll
+    for (int j = 0; j < M; ++j) {
+      const int ec = val[j] >= 0 && val[j] < E ? val[j] : 0;
+      gs_e[j] = gs[ec];
+      gpo_e[j] = gpo[ec];
+    }
+    first = 0;
+    int last = -1;
+#pragma unroll
+    for (int j = 0; j < M; ++j) {
+      if (b0 + j < nblk && (b0 + j == 0 || val[j] != prev)) {
+        first |= 1u << j;
+        last = b0 + j;
+      }
+      prev = val[j];
+    }
+    const uint64_t m = __ballot(first != 0);
+    const int wave_last = __builtin_amdgcn_readlane(last, m ? 63 - __builtin_clzll(m) : 0);  // -1 if there is none
+    if (l == 0) sh->last[w] = wave_last;
+    if (one_pass) {
+      if constexpr (M == 1) {
+        if (l == 0) reinterpret_cast<uint64_t*>(sh->firsts)[w] = m;
+      } else {
+        reinterpret_cast<uint8_t*>(sh->firsts)[tid] = (uint8_t)first;
+      }
+    }
+    const uint64_t lower = m & ((1ull << l) - 1);
+    const int from_wave = __shfl(last, lower ? 63 - __builtin_clzll(lower) : 0);
+    __syncthreads();
+    int s = carry_s;
+    for (int v = 0; v < w; ++v) s = sh->last[v] >= 0 ? sh->last[v] : s;
+    if (lower) s = from_wave;
+    int c = 0, r = 0;
+#pragma unroll
+    for (int j = 0; j < M; ++j) {
+      const int b = b0 + j;
+      s = first >> j & 1 ? b : s;
+      const bool owned = val[j] >= 0 && val[j] < E;
+      const int64_t lft = owned ? (int64_t)gs_e[j] - ((int64_t)s * BM - gpo_e[j]) : 0;
       const int64_t lo = (int64_t)(b - s) * BM, hi = lo + BM;
-      int c = 0, r = 0;  // pieces and routed rows that this block adds
+      left[j] = (int)(lft < 0 ? 0 : (lft > 0x7fffffff ? 0x7fffffff : lft));
+      pcs[j] = rws[j] = 0;
       if (b < nblk) {
-        const int upto_hi = (int)(left < hi ? left : hi), upto_lo = (int)(left < lo ? left : lo);
-        if (left > 0) {
-          c = items_of(upto_hi, hmax) - items_of(upto_lo, hmax);
-          r = upto_hi - upto_lo;
+        if (lft > 0) {
+          const int upto_hi = (int)(lft < hi ? lft : hi), upto_lo = (int)(lft < lo ? lft : lo);
+          pcs[j] = items_of(upto_hi, hmax) - items_of(upto_lo, hmax);
+          rws[j] = upto_hi - upto_lo;
         } else {
-          c = first;
+          pcs[j] = first >> j & 1;
         }
-        tall = tall || (hmax > kLowRows && left > kCutRows);
       }
-      const int inc = wave_inclusive_scan(c), incr = wave_inclusive_scan(r);
-      if (l == 63) {
-        sh->smem_p[w] = inc;
-        sh->smem_r[w] = incr;
-      }
-      __syncthreads();
-      int below = carry_p, rbelow = carry_r;
-      for (int v = 0; v < 8; ++v) {
-        if (v == w) f(b, first, below + inc - c, rbelow + incr - r);
-        below += sh->smem_p[v];
-        rbelow += sh->smem_r[v];
-        carry_s = sh->smem_s[v] >= 0 ? sh->smem_s[v] : carry_s;
-      }
-      carry_p = below;
-      carry_r = rbelow;
-      __syncthreads();  // the next pass (or caller) writes the same memory
+      c += pcs[j];
+      r += rws[j];
     }
-    rows_all = carry_r;
-    return carry_p;
-  };
-  int p0 = 0;
-  bool first0 = false;
-  const int total = sweep([&](int b, bool first, int below, int rbelow) {
-    if (b < kThreads) {
-      first0 = first;
-      p0 = below;
-      if (b < nblk) {
-        sh->ist[b] = below;
-        sh->gof[b] = rbelow;
-      }
-    }
-  });
-  const bool any = __ballot(tall) != 0;
-  if (l == 0) sh->smem_r[w] = any;
-  __syncthreads();  // orders ist and gof, too
-  bool cut = false;
-  for (int u = 0; u < 8; ++u) cut = cut || sh->smem_r[u];
-  int v;
-  if (nblk <= kThreads && cut) {
-    if (w == 0) {
-      if (l == 0) {
-        sh->ist[nblk] = total;
-        sh->gof[nblk] = rows_all;
-      }
-      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
-      xcd_shares(sh->ist, sh->gof, nblk, nt, sh->xb, grid / kNumXcd);
+    const int inc = wave_inclusive_scan(c), incr = wave_inclusive_scan(r);
+    const int tall = __ballot(left[0] > kCutRows && b0 < nblk) != 0;  // (M == 1 asks)
+    if (l == 63) {
+      sh->pieces[w] = inc;
+      sh->rows[w] = incr;
+      sh->tall[w] = tall;
     }
     __syncthreads();
-    v = sh->xb[g % kNumXcd] + g / kNumXcd;
-    if (v >= sh->xb[g % kNumXcd + 1]) return false;
+    int p = carry_p + inc - c, q = carry_r + incr - r;
+    for (int v = 0; v < 8; ++v) {
+      if (v < w) {
+        p += sh->pieces[v];
+        q += sh->rows[v];
+      }
+      carry_p += sh->pieces[v];
+      carry_r += sh->rows[v];
+      carry_s = sh->last[v] >= 0 ? sh->last[v] : carry_s;
+    }
+#pragma unroll
+    for (int j = 0; j < M; ++j) {
+      below[j] = p;
+      rbelow[j] = q;
+      p += pcs[j];
+      q += rws[j];
+    }
+    if (!one_pass) __syncthreads();  // the next pass writes the same memory
+  };
+  for (int base = 0; base < nblk; base += kPass) pass(base);
+  const int total = carry_p * nt;
+
+  int v;
+  bool cut_by_cost = false;
+  if (M == 1 && one_pass && hmax > kLowRows)
+    for (int u = 0; u < 8; ++u) cut_by_cost = cut_by_cost || sh->tall[u];
+  if (M == 1 && cut_by_cost) {
+    const int64_t all = ((int64_t)kItemCost * carry_p + carry_r) * nt;
+    const int per = (total + kNumXcd - 1) / kNumXcd;
+#pragma unroll
+    for (int j = 0; j < M; ++j) {
+      if (pcs[j] + rws[j] == 0) continue;
+      const int i0 = below[j] * nt, i1 = i0 + pcs[j] * nt;
+      const int64_t k0 = ((int64_t)kItemCost * below[j] + rbelow[j]) * nt, k1 = k0 + ((int64_t)kItemCost * pcs[j] + rws[j]) * nt;
+      for (int x = 1; x < 8; ++x) {
+        const int64_t pos = all * x / 8;
+        if (k0 <= pos && pos < k1) {
+          const int in = (int)((float)(pos - k0) / (float)(k1 - k0) * (float)(i1 - i0));
+          sh->cut_item[1][x] = i0 + (in < i1 - i0 ? in : i1 - i0);
+          sh->cut_cost[1][x] = (float)pos;
+        }
+        if (i0 <= x * per && x * per < i1)
+          sh->cut_cost[0][x] = (float)k0 + (float)(x * per - i0) / (float)(i1 - i0) * (float)(k1 - k0);
+      }
+    }
+    __syncthreads();
+    const int q = l % 18, x = q % 9;
+    XcdCut cut = {0, 0.0};
+    if (x > 0) {
+      const bool weighted = q >= 9, inner = x < 8 && (weighted || x * per < total);
+      cut.item = inner ? (weighted ? sh->cut_item[1][x] : x * per) : total;
+      cut.cost = inner ? sh->cut_cost[weighted][x] : (double)all;
+    }
+    const XcdPick pick = xcd_better(cut, l < 18, grid / kNumXcd);
+    const int at = (pick.weighted ? 9 : 0) + g % kNumXcd;
+    v = __shfl(cut.item, at) + g / kNumXcd;
+    const int end = __shfl(cut.item, at + 1);
+    // (lanes 18.. hold another group's choice)
+    v = __builtin_amdgcn_readfirstlane(v);
+    if (v >= __builtin_amdgcn_readfirstlane(end)) return false;
   } else {
-    v = xcd_item(g, total * nt);
+    v = xcd_item(g, total);
     if (v < 0) return false;
   }
+
   // the last run whose first item is <= v: block s, items below it ps
-  int s = -1, ps = 0;
-  auto find = [&](int b, bool first, int below, int) {
-    const uint64_t m = __ballot(first && below * nt <= v);
-    if (m) {
-      const int lane = 63 - __builtin_clzll(m);
-      s = __shfl(b, lane);
-      ps = __shfl(below, lane);
-    }
+  int s = -1, ps = 0, rval = 0, rleft = 0;
+  auto find = [&](int base) {
+#pragma unroll
+    for (int j = 0; j < M; ++j)
+      if ((first >> j & 1) && below[j] * nt <= v) {
+        s = base + tid * M + j;
+        ps = below[j];
+        rval = val[j];
+        rleft = left[j];
+      }
   };
-  if (nblk <= kThreads) find((int)threadIdx.x, first0, p0, 0);
-  else sweep(find);
-  if (l == 0) {
-    sh->smem_s[w] = s;
-    sh->smem_p[w] = ps;
+  if (one_pass) {
+    find(0);
+  } else {
+    carry_s = carry_p = carry_r = 0;
+    for (int base = 0; base < nblk; base += kPass) {
+      pass(base);
+      find(base);
+    }
+  }
+  int most = s;
+#pragma unroll
+  for (int o = 32; o >= 1; o >>= 1) {
+    const int other = __shfl_xor(most, o);
+    most = other > most ? other : most;
+  }
+  if (l == 0 && most < 0) sh->run[w] = -1;
+  if (most >= 0 && s == most) {
+    sh->run[w] = s;
+    sh->below[w] = ps;
+    sh->val[w] = rval;
+    sh->left[w] = rleft;
   }
   __syncthreads();
-  for (int u = 0; u < 8; ++u)
-    if (sh->smem_s[u] > s) {
-      s = sh->smem_s[u];
-      ps = sh->smem_p[u];
-    }
-  s = __builtin_amdgcn_readfirstlane(s);
-  ps = __builtin_amdgcn_readfirstlane(ps);
-  __syncthreads();  // the caller reuses smem
-  const int val = gidx[s];
-  // run end: the nearest block above s with another value (or nblk)
+  int at = 0;
+  for (int u = 1; u < 8; ++u) at = sh->run[u] > sh->run[at] ? u : at;
+  s = __builtin_amdgcn_readfirstlane(sh->run[at]);
+  ps = __builtin_amdgcn_readfirstlane(sh->below[at]);
+  rval = __builtin_amdgcn_readfirstlane(sh->val[at]);
+  rleft = __builtin_amdgcn_readfirstlane(sh->left[at]);
+  // run end: the next run's first block (or nblk)
   int end = -1;
-  for (int base = s + 1; end < 0; base += 64) {
-    const int b = base + l;
-    const bool diff = b >= nblk || gidx[b] != val;
-    const uint64_t m = __ballot(diff);
-    if (m) end = base + (__ffsll((unsigned long long)m) - 1);
+  if (one_pass) {
+    for (int w0 = (s + 1) / 32; end < 0; w0 += 64) {
+      const int i = w0 + l;
+      uint32_t bits = i * 32 < nblk ? sh->firsts[i] : 0;
+      if (i == (s + 1) / 32) bits &= ~0u << ((s + 1) % 32);
+      const uint64_t m = __ballot(bits != 0);
+      if (m) {
+        const int lane = __ffsll((unsigned long long)m) - 1;
+        end = (w0 + lane) * 32 + __ffs(__builtin_amdgcn_readlane((int)bits, lane)) - 1;
+      } else if ((w0 + 64) * 32 >= nblk) {
+        end = nblk;
+      }
+    }
+  } else {
+    for (int base = s + 1; end < 0; base += 64) {
+      const int b = base + l;
+      const uint64_t m = __ballot(b >= nblk || gidx[b < nblk ? b : nblk - 1] != rval);
+      if (m) end = base + (__ffsll((unsigned long long)m) - 1);
+    }
   }
-  it.e = val >= 0 && val < E ? val : -1;
-  int n = 0;
-  if (it.e >= 0) {
-    const int64_t left = (int64_t)gs[it.e] - ((int64_t)s * BM - gpo[it.e]);
-    const int64_t cap = (int64_t)(end - s) * BM;
-    n = (int)(left < 0 ? 0 : (left > cap ? cap : left));
-  }
+  __syncthreads();  // the caller reuses smem
+  it.e = rval >= 0 && rval < E ? rval : -1;
+  const int64_t cap = (int64_t)(end - s) * BM;
+  const int n = it.e < 0 ? 0 : (int)(rleft > cap ? cap : rleft);
   const int c = n > 0 ? items_of(n, hmax) : 1;
   const int local = v - ps * nt;
   const int t = local / c, i = local % c;
@@ -678,6 +765,12 @@ __device__ __forceinline__ bool item_bx(int g, const int32_t* __restrict__ gidx,
   it.zero_end = i == c - 1 ? end * BM : 0;
   it.shared = c > 1;
   return t < nt;
+}
+__device__ __forceinline__ bool item_bx(int g, const int32_t* __restrict__ gidx, int nblk, int E, int BN, int nt,
+                                        const int32_t* __restrict__ gs, const int32_t* __restrict__ gpo, int hmax,
+                                        int grid, char* smem, Item& it) {
+  return nblk <= 512 ? item_runs<1>(g, gidx, nblk, E, BN, nt, gs, gpo, hmax, grid, smem, it)
+                     : item_runs<kScanBlocks>(g, gidx, nblk, E, BN, nt, gs, gpo, hmax, grid, smem, it);
 }
 
 // Workgroups of a launch of `blocks` blocks (or row pieces) x `ntiles` items.

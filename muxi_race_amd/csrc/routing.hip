@@ -201,7 +201,7 @@ __device__ void item_plan(const int* tot, int E, const ItemPlan& p, int* sm) {
       const int nt = k == 0 ? p.nt1 : (k == 1 ? p.nt2 / 2 : p.nt2);
       pick = xcd_pick(mine, gof, E, nt, k < 3 && may, k == 0 ? p.slots1 : p.slots2);
     }
-    if (pick.chosen) xbs[9 * (3 * w + k) + l % 18 % 9] = pick.item;
+    if (w < nh && k < 3 && may && (l % 18 >= 9) == pick.weighted) xbs[9 * (3 * w + k) + l % 18 % 9] = pick.item;
     if (k < 3 && l % 18 == 0) est[3 * w + k] = may ? pick.slow * (k == 2 ? kHalfTile : 1.0f) : INFINITY;
   }
   __syncthreads();

@@ -4,6 +4,7 @@ an expert's split or its tile changes, over both cuts of the items over the
 XCDs, for every format; run_kernel's item count over more than 512 blocks; and
 the one-launch routing and alignment of small batches against the two
 launches."""
+import numpy as np
 import pytest
 import torch
 
@@ -192,3 +193,64 @@ def test_last_piece_of_one_row(I):
     run_kernel(*args, out)
     torch.cuda.synchronize()
     assert_close(out, prerouted_forward(*args), what=f"prerouted last piece I={I}")
+
+
+def _runs(nblk, seed, E=40):
+    """Metadata of nblk blocks in runs of random lengths, some of them empty, of
+    no expert, or of an expert named before, with any number of rows."""
+    rng = np.random.default_rng(seed)
+    gidx, b = [], 0
+    gs, gpo = np.zeros(E, np.int32), np.zeros(E, np.int32)
+    free = list(rng.permutation(E))
+    while b < nblk:
+        n = int(min(nblk - b, rng.integers(1, 40) if rng.random() < 0.1 else rng.integers(1, 4)))
+        kind = rng.random()
+        if kind < 0.1 or not free:
+            e = int(rng.choice([-1, E, E + 3])) if kind < 0.1 else int(rng.integers(0, E))
+        else:
+            e = int(free.pop())
+            gs[e] = rng.integers(0, 128 * n + 60) if rng.random() < 0.9 else 0
+            gpo[e] = 128 * b
+        gidx += [e] * n
+        b += n
+    return np.array(gidx, np.int32), gs, gpo
+
+
+@pytest.mark.parametrize("nblk", [1, 2, 63, 64, 65, 511, 512, 513, 520, 2047, 4095, 4096, 4097, 5000])
+@pytest.mark.parametrize("I", [128, 2048])
+def test_run_kernel_counts_items_over_any_blocks(nblk, I):
+    """Runs of every kind over one and several passes of the item count (512
+    and 4096 blocks), in short items (I 128) and, from 33 blocks on, in tall
+    ones: every block's rows are its expert's product or 0, from a NaN-poisoned
+    output with NaN in x's rows without a token."""
+    from muxi_race_amd import run_kernel
+    E, H = 40, 128
+    gidx, gs, gpo = _runs(nblk, nblk + I)
+    g = torch.Generator(device="cuda").manual_seed(nblk)
+    mk = lambda *sh: torch.randn(*sh, generator=g, device="cuda")
+    rows = 128 * np.arange(nblk)[:, None] + np.arange(128)
+    e = np.clip(gidx, 0, E - 1)[:, None]
+    valid = ((gidx >= 0) & (gidx < E))[:, None] & (rows >= gpo[e]) & (rows - gpo[e] < gs[e])
+    # (a row before its expert's first one counts as routed, as the blocks' own rule has it)
+    valid |= ((gidx >= 0) & (gidx < E))[:, None] & (rows < gpo[e]) & (rows - gpo[e] < gs[e])
+    valid = torch.from_numpy(valid.reshape(-1)).cuda()
+    x = mk(128 * nblk, H).half()
+    x[~valid] = float("nan")
+    w = [(mk(*sh) * 0.05).half() for sh in ((E, I, H), (E, I, H), (E, H, I))]
+    V = max(int(gs.sum()), 1) if I == 128 else 128 * nblk
+    routed = torch.ones(V, device="cuda")
+    i32 = lambda a: torch.from_numpy(np.ascontiguousarray(a, dtype=np.int32)).cuda()
+    go = np.concatenate([[0], np.cumsum(gs)])
+    out = torch.full((128 * nblk, H), float("nan"), dtype=torch.float16, device="cuda")
+    run_kernel(x, *w, routed, i32(gs), i32(go), i32(np.append(gpo, 128 * nblk)), i32(gidx), out)
+    torch.cuda.synchronize()
+    assert bool(torch.isfinite(out).all())
+    assert (out[~valid] == 0).all()
+    owner = torch.from_numpy(np.repeat(gidx, 128)).cuda()
+    for j in range(E):
+        at = valid & (owner == j)
+        if not bool(at.any()):
+            continue
+        xe = x[at].float()
+        h = (torch.nn.functional.silu(xe @ w[0][j].float().T) * (xe @ w[1][j].float().T)).half().float()
+        assert_close(out[at], h @ w[2][j].float().T, what=f"expert {j} of {nblk} blocks")
