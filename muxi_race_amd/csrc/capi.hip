@@ -134,7 +134,7 @@ bool stream_weights(int64_t experts, int64_t H, int64_t I, int qt) {
 //     the choice won 5-25% on skewed routings (Stage 1 of 60 experts of H 2048, I
 //     1408, 400 tokens top-4, Zipf 112 -> 79 us), at 7 it was level or lost
 //     (Stage 2 of 64 experts of H 7168, I 2048, 200 tokens top-6, Zipf 208 -> 224).
-//   - Stage 2 in 128-feature items as well up to 1.5 items of 256 features per
+//   - Stage 2 in 128-feature items as well below one item of 256 features per
 //     CU; past it none of those cases gained by them.  Its K loop is short
 //     (I / 64 steps), so 256 features are right where they fill the chip: half
 //     the re-reads of the intermediate and twice the work behind each item's fill
@@ -156,7 +156,7 @@ moe::ItemPlan fused_plan(int64_t pairs, int64_t rows, int64_t experts, int64_t H
   const int64_t items = used * moe::items_of((int)avg, p.tall);
   p.any1 = items * p.nt1 <= kPlanRounds * kCus;
   p.any2 = items * ((p.nt2 + 1) / 2) <= kPlanRounds * kCus;
-  p.bn2 = H % 256 ? 128 : (2 * items * (H / 256) <= 3 * kCus ? 0 : 256);
+  p.bn2 = H % 256 ? 128 : (items * (H / 256) < kCus ? 0 : 256);
   auto slots = [&](bool any, int64_t nt, int64_t nt_most) {
     // sum of ceil(n / hmax) over `held` experts: at most pairs / hmax + held
     const int64_t least = moe::xcd_items_bound(pairs / p.tall + held, pairs, nt);
@@ -567,6 +567,7 @@ static int fused_common(int qt, const void* x, const float* logits, const void* 
     p2.istart = plan.out + moe::ItemPlan::istart2(Ee);
     p2.xb = plan.out + moe::ItemPlan::xb2(Ee);
     p2.bn_plan = plan.out + moe::ItemPlan::bn(Ee);
+    p2.bn = plan.bn2;
   }
   p2.rows_cap = (int)rows;
   p2.stream = p1.stream;

@@ -112,7 +112,7 @@ struct Stage2Params {
   const int32_t* istart = nullptr;
   const int32_t* xb = nullptr;
   const int32_t* bn_plan = nullptr;  // wide, fused: features of an item, 128 or 256 (the plan's)
-  int bn = 0;               // wide, pre-routed: features of an item, 128 or 256
+  int bn = 0;               // wide: features of an item, 128 or 256; fused, 0: either, as bn_plan says
   int rows_cap = 0;
   int hmax = 0;
   bool stream = true;       // wide: as Stage 1's
