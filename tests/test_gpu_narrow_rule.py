@@ -35,6 +35,20 @@ def test_library_picks(T, E, held, k, I, narrow):
     assert torch.equal(got, n if narrow else wide)
 
 
+@pytest.mark.parametrize("T,E,held,k,I,narrow", [(800, 64, 4, 2, 512, False), (600, 64, 4, 2, 512, True)])
+def test_library_picks_for_dispatched_tokens(T, E, held, k, I, narrow):
+    """Each token has a choice here, so the experts held here get more rows than
+    the average over all (25 of 800 tokens, above the line; 200 here), and the
+    workspace that the size function asks for holds the wide items."""
+    from muxi_race_amd import fused_moe_routed
+    x, lg, w = _case(T, E, held, k, I)
+    ids = torch.stack([8 + torch.arange(T) % held, torch.full((T,), 40)], 1).int().cuda()
+    wts = torch.softmax(lg[:, :k], 1).contiguous()
+    got, n, wide = (fused_moe_routed(x, ids, wts, *w, expert_begin=8, num_experts=E, block_m=bm) for bm in (0, 32, 64))
+    torch.cuda.synchronize()
+    assert not torch.equal(n, wide), "the sums do not tell the items apart"
+    assert torch.equal(got, n if narrow else wide)
+
 
 @pytest.mark.parametrize("bm", [32, 64, 128])
 def test_workspace_sized_without_block_m_serves_explicit_blocks(bm):
