@@ -128,37 +128,36 @@ def test_capacity_and_workspace_sizes():
 
 
 def test_256_row_padding_policy():
-    """With block_m = 0 the library pads experts to 256 rows only where
-    256-row items run faster: H a multiple of 256 and >= 192 routed rows per
-    expert on average (mixtral, w8a8), never at dsv3's 128."""
+    """The workspace of block_m = 0 still holds experts padded to 256 rows where
+    the library used to pad so -- H a multiple of 256 and >= 192 routed rows per
+    expert on average (mixtral, w8a8), not at dsv3's 128 -- for callers that
+    sized other calls by it."""
     from muxi_race_amd._lib import lib
     L = lib()
     ws = lambda T, H, I, E, k, bm, f: L.moe_fused_workspace_bytes(T, H, I, E, k, bm, f)
     cap = L.moe_align_capacity_rows
-    # mixtral (512 rows per expert): fp16 pads
+    # mixtral (512 rows per expert)
     assert cap(2048, 2, 8, 256) > cap(2048, 2, 8, 128)
     assert ws(2048, 4096, 14336, 8, 2, 0, 0) > ws(2048, 4096, 14336, 8, 2, 128, 0)
-    # w8a8 (192 rows per expert): every format pads; 191 rows per expert does not
+    # w8a8 (192 rows per expert): every format; not 191 rows per expert
     for f in (0, 1, 2):
         assert ws(2048, 7168, 2048, 64, 6, 0, f) > ws(2048, 7168, 2048, 64, 6, 128, f)
         assert ws(2037, 7168, 2048, 64, 6, 0, f) == ws(2037, 7168, 2048, 64, 6, 128, f)
-    # dsv3 (128 rows per expert): nothing pads
+    # dsv3 (128 rows per expert): no format
     for f in (0, 1, 2):
         assert ws(4096, 7168, 2048, 256, 8, 0, f) == ws(4096, 7168, 2048, 256, 8, 128, f)
-    # H not a multiple of 256: no padding
+    # H not a multiple of 256
     assert ws(2048, 4224, 14336, 8, 2, 0, 0) == ws(2048, 4224, 14336, 8, 2, 128, 0)
 
 
 @pytest.mark.parametrize("define,sources", [
     ("MOE_S2_SCATTER", ("grouped_gemm.hip", "capi.hip")),
-    ("MOE_S1_TRIPLE", ("grouped_gemm.hip",)),
 ])
 def test_measured_variant_compiles(tmp_path, define, sources):
     """Variants kept as committed compile-time flags for their A/B must keep
     compiling for gfx950: the Stage 2 scatter-reduce (MOE_S2_SCATTER=1: packed
-    fp16 atomics into the token-ordered output, no combine) and Stage 1's
-    triple items (MOE_S1_TRIPLE=1: an odd multi-block expert's last three
-    blocks as one item per half weight tile)."""
+    fp16 atomics into the token-ordered output, no combine).  Each source must
+    read the flag (or what is compiled is the default)."""
     import subprocess
     from muxi_race_amd.build import CSRC, HIP_FLAGS, _hipcc
     try:
@@ -166,6 +165,7 @@ def test_measured_variant_compiles(tmp_path, define, sources):
     except RuntimeError:
         pytest.skip("hipcc not available")
     for src in sources:
+        assert define in (CSRC / src).read_text(), f"{src} does not read {define}"
         cmd = [hipcc, *HIP_FLAGS, f"-D{define}=1", "-c", str(CSRC / src), "-o", str(tmp_path / (src + ".o"))]
         r = subprocess.run(cmd, capture_output=True, text=True)
         assert r.returncode == 0, r.stderr[-2000:]

@@ -83,10 +83,11 @@ def test_fp8_small(bm):
 
 
 def test_fp8_256_row_padding_ragged():
-    """Both fp8 stages run 256-row items over the 256-row padding.  At T = 800
-    a few e4m3 boundary flips occur, so the oracle gates are those of the large
-    configs; against explicit 128-row blocks (same K order per element) the
-    output must agree to within such flips."""
+    """200 rows per expert in the library's choice (32-row items: two Stage 1
+    tiles over 8 experts).  At T = 800 a few e4m3 boundary flips occur, so the
+    oracle gates are those of the large configs; against the wide items of
+    explicit 128-row blocks (same K order per element) the output must agree to
+    within such flips."""
     from muxi_race_amd import fused_moe, quantize_w8a8_weights
     inp = skewed_8bit_case(76)
     _run(inp)
@@ -95,13 +96,13 @@ def test_fp8_256_row_padding_ragged():
     b = fused_moe(inp["x"], inp["logits"], None, None, None, inp["k"], expert_bias=inp["bias"], w8a8=qw,
                   block_m=128)
     torch.cuda.synchronize()
-    assert_close(a, b, atol=1e-3, rtol=1e-3, what="256-row padding vs 128-row blocks")
+    assert_close(a, b, atol=1e-3, rtol=1e-3, what="32-row items vs wide items")
 
 
 def test_fp8_workspace_sized_for_128_rows_keeps_128_row_padding():
     """A caller that sizes the workspace for block_m = 128 and then passes
-    block_m = 0 still gets a correct result: the call keeps the 128-row
-    padding."""
+    block_m = 0 still gets a correct result, and one that sizes with 0 has room
+    for more."""
     import ctypes
     from muxi_race_amd import fused_moe, quantize_w8a8_weights
     from muxi_race_amd._lib import lib
@@ -121,7 +122,7 @@ def test_fp8_workspace_sized_for_128_rows_keeps_128_row_padding():
                                  ctypes.c_void_p(torch.cuda.current_stream().cuda_stream), P(None))
     assert rc == 0, L.moe_last_error_string()
     torch.cuda.synchronize()
-    assert_close(b, a, atol=1e-3, rtol=1e-3, what="128-row padding vs 256")
+    assert_close(b, a, atol=1e-3, rtol=1e-3, what="workspace of block_m 128")
 
 
 def test_fp8_w8a8_config_full():
@@ -133,7 +134,7 @@ def test_fp8_decode():
 
 
 def test_fp8_dsv3_sampled():
-    """dsv3 on the stratified rows (paired, single and tail items) of its three
+    """dsv3 on the stratified rows (several items each) of its three
     largest multi-block experts plus 8 random tokens.  The oracle expands each
     touched expert's fp8 weights to float64 (exact sums), so the sample is
     bounded; the fp8 schedule is covered in full at the w8a8 config."""

@@ -125,8 +125,7 @@ def _random_case(T, H, I, E, k, seed, bias=True):
     (3, 128, 256, 1024, 32),    # widest routing: E = 1024 experts, k = 32 choices
     (257, 256, 128, 32, 32),    # every token takes every expert (k = E)
     (129, 384, 640, 5, 3),      # odd expert count, H and I not powers of two
-    # more than 256 experts (no absorbed rows): ~109 rows each on paired
-    # 128-row items, and ~218 each on 256-row items (H a multiple of 256)
+    # more than 256 experts (a fifth chunk of the expert scan), ~109 and ~218 rows each
     (4096, 128, 256, 300, 8),
     (8192, 256, 256, 300, 8),
 ])
@@ -135,15 +134,13 @@ def test_extreme_shapes(T, H, I, E, k):
 
 
 def test_256_row_padding_ragged():
-    """fp16 experts with >= 192 routed rows on average and H a multiple of 256:
-    align pads experts to 256 rows, Stage 1 runs 256-row items, Stage 2
-    128-row (paired) items.  Skewed biases give full, partial and empty
-    256-row blocks, 128-row halves with no rows, and two empty experts."""
+    """fp16 experts of 384 routed rows on average, whose skewed biases give
+    several pieces, partial ones and two empty experts."""
     inp = _random_case(1536, 512, 384, 8, 2, 77, bias=False)
     inp["bias"] = torch.tensor([2.5, 2.0, 1.0, 0.5, 0.0, -0.5, -40.0, -40.0], device="cuda")
     from muxi_race_amd import pick_block_m
     assert pick_block_m(1536, 8, 2) == 128
-    _check(inp, what="fp16, 256-row padding")
+    _check(inp, what="fp16, ragged tall experts")
 
 
 def test_empty_batch():

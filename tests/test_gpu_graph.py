@@ -41,7 +41,8 @@ def test_fp16_forward_replays(name):
 
 
 def test_256_row_padding_replays():
-    """fp16 Stage 1 and fp8 Stage 2 on 256-row items (the 256-row padding)."""
+    """fp16 on several wide items per expert (align's item plan is replayed too),
+    and fp8 on several 32-row items per expert."""
     from muxi_race_amd import fused_moe, quantize_w8a8_weights
     g = torch.Generator().manual_seed(104)
     T, H, I, E, k = 1536, 512, 384, 8, 2  # 384 routed rows per expert

@@ -8,10 +8,10 @@ import numpy as np
 import pytest
 import torch
 
+from _plan import HALF_TILE, SHORTER, both_slots, cuts
+
 pytestmark = pytest.mark.gpu
 
-ITEM_COST, HALF_TILE, CUS = 256, 0.7, 32
-SHORTER = [256, 224, 192, 160, 128]
 LAUNCH_ALIGN = "_ZN3moe12launch_alignEPKiiiiPiS2_S2_S2_S2_S2_P12ihipStream_tiRKNS_8ItemPlanE"
 
 
@@ -45,30 +45,9 @@ def _plan(counts, tall, nt1, nt2, any1, any2, bn2, slots, bm=64):
     return o[:E + 1], o[E + 1:2 * E + 2], o[2 * E + 2:2 * E + 11], o[2 * E + 11:2 * E + 20], int(o[2 * E + 20])
 
 
-def _cuts(counts, h, nt):
-    """Both cuts of the items over the XCDs, as (first items [9], time of the slowest XCD in rows of cost)."""
-    cost = np.concatenate([[(ITEM_COST * -(-n // h) + n) / -(-n // h)] * (-(-n // h) * nt) for n in counts if n] or [[]])
-    total, below = len(cost), np.concatenate([[0.0], np.cumsum(cost)])
-    per = -(-total // 8)
-    equal = [min(total, x * per) for x in range(9)]
-    # (a cut that falls between two items may round either way by one item)
-    weighted = [int(np.searchsorted(below, below[-1] * x / 8 * (1 + 1e-12), side="right") - 1) for x in range(8)] + [total]
-    for b in (equal, weighted):
-        n = np.diff(b)
-        s = np.diff(below[b]) if b is equal else below[-1] / 8 * np.ones(8)
-        yield n, max([-(-int(k) // CUS) * c / k for k, c in zip(n, s) if k > 0] or [0.0])
-
-
-def _slots(P, E, tall, short, nt, nt_most):
-    """The host's workgroups per XCD."""
-    bound = lambda h, n: ((P // h + min(P, E)) * 256 + P) * n // (8 * 256) + 2
-    return max(bound(tall, nt), min(bound(short, nt_most), CUS))
-
-
 def _check(counts, tall, nt1, nt2, any1, any2, bn2):
     E, P = len(counts), int(sum(counts))
-    slots = (_slots(P, E, tall, 128 if any1 else tall, nt1, nt1),
-             _slots(P, E, tall, 128 if any2 else tall, nt2 if bn2 == 128 else nt2 // 2, nt2 // 2 if bn2 == 256 else nt2))
+    slots = both_slots(P, E, tall, nt1, nt2, any1, any2, bn2)
     i1, i2, xb1, xb2, bn = _plan(counts, tall, nt1, nt2, any1, any2, bn2, slots)
     chosen = []
     for istart, xb, heights, nts, room in (
@@ -82,9 +61,9 @@ def _check(counts, tall, nt1, nt2, any1, any2, bn2):
         assert xb[0] == 0 and xb[8] == total and (np.diff(xb) >= 0).all()
         assert np.diff(xb).max() <= room
         # what fits, and what a cut that rounds one item further would still let fit
-        est = {(h, v): [t * (HALF_TILE if v == 128 and istart is i2 else 1.0) for k, t in _cuts(counts, h, n) if k.max() < room]
+        est = {(h, v): [t * (HALF_TILE if v == 128 and istart is i2 else 1.0) for k, t in cuts(counts, h, n) if k.max() < room]
                for h in heights for v, n in nts.items()}
-        mine = min([t for h in match for k, t in _cuts(counts, h, nts[w]) if k.max() <= room + 1]) * \
+        mine = min([t for h in match for k, t in cuts(counts, h, nts[w]) if k.max() <= room + 1]) * \
             (HALF_TILE if w == 128 and istart is i2 else 1.0)
         assert mine <= min([t for e in est.values() for t in e] or [np.inf]) * 1.02 + 1, (est, match, w)
         chosen.append((match, w))

@@ -3,8 +3,7 @@
 Token-permutation equivariance.  Each output row depends only on its own
 token: its routing, its gathered rows multiplied in a fixed K order, and a
 fixed choice-order sum.  A permutation of the tokens changes which tokens
-share an expert's blocks, which land in paired, single or absorbed rows, and
-every row's place in the expert-sorted order.  So permuting the rows of x and
+share an expert's items, which land in absorbed rows, and every row's place in the expert-sorted order.  So permuting the rows of x and
 of the logits must permute the output rows, the routing ids and the routing
 weights bit for bit, in every config and format.  A gather, padding,
 absorbed-row or combine mapping mistake breaks this at sizes the CPU oracle
@@ -46,7 +45,7 @@ def test_token_permutation_equivariance(name, fmt):
 def test_identical_tokens_get_identical_rows(name, fmt):
     """A quarter of the tokens repeat other tokens (x row and logits row):
     they are routed alike but sit at other places of the sorted order (other
-    blocks, paired / single / absorbed rows), and each copy's output row must
+    items, absorbed rows among them), and each copy's output row must
     equal the original's bit for bit, in one call."""
     from muxi_race_amd import fused_moe, quantize_w8a8_weights
     inp = moe_inputs(name, 303)

@@ -22,7 +22,7 @@ def _shard(inp, b, n, **kw):
 def test_shards_sum_to_full_and_match_oracle(name, G):
     from muxi_race_amd import fused_moe
     # mixtral at T=1536: 384 routed rows per expert over the whole layer, so every
-    # shard runs on the 256-row padding
+    # shard runs several wide items per expert
     inp = moe_inputs(name, 91, T={"dsv3": 1024, "mixtral": 1536}.get(name))
     E, T = inp["E"], inp["T"]
     full, (fids, fw) = fused_moe(inp["x"], inp["logits"], inp["wg"], inp["wu"], inp["wd"], inp["k"],

@@ -79,9 +79,8 @@ def test_w8a8_small(bm):
 
 @pytest.mark.parametrize("bm", [0, 128])
 def test_w8a8_skewed_ragged(bm):
-    """An empty expert, partial and multi-block experts, over the library's
-    256-row padding (both stages on 256-row items) and over 128-row blocks
-    (Stage 1 pairs the blocks of multi-block experts, Stage 2 too)."""
+    """An empty expert, partial and multi-block experts, in the library's choice
+    (32-row items: two Stage 1 tiles over 8 experts) and in wide items."""
     _run(skewed_8bit_case(22), block_m=bm)
 
 

@@ -9,6 +9,7 @@ import pytest
 import torch
 
 from _cases import prerouted_inputs
+from _plan import chosen
 from conftest import assert_close
 from oracle import fused_moe_forward, prerouted_forward, w8a8_forward
 
@@ -100,6 +101,29 @@ def test_fp8_scale_bytes_reload(bm):
     _close_8bit(out, ref, x, lg, wg, wu, wd, f"fp8 I=2304 bm={bm}")
 
 
+@pytest.mark.parametrize("fmt", ["int8", "fp8"])
+@pytest.mark.parametrize("H,bn", [(2048, 256), (1152, 128)])
+def test_tall_items_8bit(fmt, H, bn):
+    """225 to 256 rows and multiples: the plan takes 256-row items in both stages
+    (asserted against the restated rule), here against 32-row items.  int8 sums
+    exactly: the same bits.  fp8 quantises h from sums of the same K order; a code
+    at a rounding tie may fall the other way (see _close_8bit)."""
+    from muxi_race_amd import fused_moe, quantize_w8a8_weights
+    sizes = [225, 256, 481, 512, 230, 255, 224, 1, 0, 33, 160, 161, 225, 250, 256, 240, 254, 242, 256, 231, 229, 255]
+    assert chosen(sizes, H, 1024, 256) == (256, (256, bn))
+    g = torch.Generator(device="cuda").manual_seed(H)
+    mk = lambda *sh: torch.randn(sh, generator=g, device="cuda").half()
+    E, T, lg = len(sizes), sum(sizes), _logits(sizes, 1).cuda()
+    x = mk(T, H)
+    qw = quantize_w8a8_weights(mk(E, 1024, H) * 0.05, mk(E, 1024, H) * 0.05, mk(E, H, 1024) * 0.05, fmt=fmt)
+    a, b = (fused_moe(x, lg, None, None, None, 1, w8a8=qw, block_m=bm) for bm in (0, 32))
+    torch.cuda.synchronize()
+    assert bool(torch.isfinite(a).all())
+    if fmt == "int8":
+        assert torch.equal(a, b)
+    assert float((a.float() - b.float()).norm() / b.float().norm()) < 5e-3
+
+
 @pytest.mark.parametrize("skew", ["first", "last", "even"])
 def test_xcd_shares_cover_every_item(skew):
     """70 experts, 16 Stage 1 tiles: a few experts of hundreds of rows at one
@@ -123,8 +147,8 @@ def test_xcd_shares_cover_every_item(skew):
 
 
 def test_run_kernel_over_512_blocks():
-    """650 experts (more than 512 blocks: two passes of the item count), with
-    empty, single-block and multi-block experts."""
+    """650 experts (more than 512 blocks: eight blocks to a thread of the item
+    count), with empty, single-block and multi-block experts, in short items."""
     g = torch.Generator().manual_seed(11)
     sizes = [int(v) for v in torch.randint(0, 140, (650,), generator=g)]
     sizes[3], sizes[200], sizes[649] = 600, 0, 290
@@ -164,8 +188,8 @@ def test_small_batches_route_and_align_in_one_launch(E, k, T, bias):
 @pytest.mark.parametrize("tall", [129, 288, 289, 380])
 @pytest.mark.parametrize("low", [1, 100])
 def test_prerouted_few_tall_experts(tall, low):
-    """A few tall experts among short ones: items of up to 128 rows where the
-    average is at most 112 rows and there are more blocks than experts."""
+    """A few tall experts among short ones, in items of up to 128 rows, and (18
+    experts of 100 rows) beside no more than a quarter as many extra blocks."""
     from muxi_race_amd import run_kernel
     sizes = [low] * 18
     sizes[2] = sizes[17] = tall
