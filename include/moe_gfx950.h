@@ -146,9 +146,11 @@ int moe_align(const int32_t* topk_ids, int64_t T, int64_t k, int64_t E, int64_t 
  * Full fused MoE (fp16): route -> align -> Stage1 (gathered gate/up GEMM +
  * SiLU*up) -> Stage2 (down GEMM * routing weight) -> k-way combine into token
  * order.  x fp16 [T, H]; logits fp32 [T, E]; bias fp32 [E] or NULL; weights as
- * for moe_run_prerouted; out fp16 [T, H].  block_m in {32, 64, 128} or 0 for
- * the library's choice (which may pad experts to 256 rows and run one stage
- * on 256-row items).  topk_ids_out / topk_weights_out ([T, k]) may be NULL;
+ * for moe_run_prerouted; out fp16 [T, H].  block_m: 32 runs items of up to 32
+ * rows; 64 or 128 pad experts to that many rows and run wide items, whose
+ * height and width the call picks from the routing; 0 is the library's choice of
+ * the two, from the sizes.  A workspace sized with block_m = 0 also holds the
+ * call with any block_m up to moe_pick_block_m.  topk_ids_out / topk_weights_out ([T, k]) may be NULL;
  * when given they receive the routing result.  moe_fused_workspace_bytes:
  * w8a8 = 0 for fp16, 1 for int8, 2 for fp8.
  * ---------------------------------------------------------------------- */
@@ -330,8 +332,7 @@ int moe_fused_forward_w8a8_events(const void* x, const float* logits, const floa
  * same way inside the call; the SiLU*up intermediate per (row, 128 columns)
  * with power-of-two scales, which the scaled f8 MFMA applies.
  * moe_fused_forward_fp8 takes stage_events as moe_fused_forward_events (or
- * NULL); workspace moe_fused_workspace_bytes(..., w8a8 = 2) (one sized for
- * block_m = 128 also works, without the 256-row padding).  Extends the
+ * NULL); workspace moe_fused_workspace_bytes(..., w8a8 = 2).  Extends the
  * reference's W8A8 variant (submission_v321_int8_fixed.py:421-506) to the fp8
  * MFMA of this part; the reference has no fp8 path.
  * ---------------------------------------------------------------------- */

@@ -460,7 +460,7 @@ def fused_moe(hidden_states, router_logits, w_gate, w_up, w_down, top_k: int, *,
         check(rc, "fused_moe")
         return (out, (ids, wts)) if return_routing else out
     ncol = top_k + (shared_expert is not None)
-    bm = block_m  # 0: the library picks the block rows (and a 256-row padding where that is faster)
+    bm = block_m  # 0: the library picks
     strided = w8a8 is None and not dense
     fmt = None if w8a8 is None else w8a8.fmt
     if strided:
