@@ -185,6 +185,9 @@ moe::ItemPlan fused_plan(int64_t pairs, int64_t rows, int64_t experts, int64_t H
 //     300 453 / 386, of 19 but 4 of 350 453 / 416.  On the other side 64 of 90 but
 //     30 of 150 1199 / 1279, of 30 but 41 of 203 1403 / 1497, 32 of 112 but 22 of
 //     155 643 / 783; the line costs 32 of 110 but 4 of 240 2% (629 / 644).
+//     Against the block-based items before (fef8190): 32 of 3 but 8 of 336 654 ->
+//     650, 16 of 19 but 4 of 350 384 -> 375, 64 of 115 but 3 of 300 1169 -> 1204, of
+//     110 but 10 of 200 1194 -> 1220; other groupings level or up to 18% faster.
 //   - Stage 2 takes the width whose rounds of 256 CUs cost less, a 128-feature
 //     item costing 0.7 of a 256-feature one (routing.hip kHalfTile).  The pieces
 //     are the blocks for items of up to 128 rows.  16 experts (H 2048, I 8192) of
